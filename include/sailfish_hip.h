@@ -296,15 +296,16 @@ int sf_phys_substep(const sf_phys_fields *fields, int32_t precision, double dt, 
                     double cff1, void *stream);
 
 /* The same substep as ONE launch: each workgroup evaluates predictor and corrector
- * on an LDS-staged tile of 64 x tile_j points (tile_j = 4, 8 or 16; 0 = default)
+ * on an LDS-staged tile of 64 x tile_j points (tile_j = 4, 8 or 16; 0 = the tile that
+ * measured fastest on the grid's size, down to 16 x 8 on small grids)
  * with a 3/2-point halo, so no intermediate state goes to memory.  scratch[] is
  * not used.  Results equal sf_phys_substep bit for bit in both precisions.  Same
  * reference lineage as sf_phys_substep. */
 int sf_phys_substep_fused(const sf_phys_fields *fields, int32_t precision, double dt, int32_t first,
                           double cff1, int32_t tile_j, void *stream);
 
-/* Default tile height of sf_phys_substep_fused for a precision and grid size (8, or 4
- * when 64 x 8 tiles would give fewer than 1024 workgroups). */
+/* The 64-wide tile height to name where one has to be named (8, or 4 when 64 x 8 tiles
+ * would give fewer than 1024 workgroups); tile_j = 0 chooses among more shapes. */
 int sf_phys_fused_default_tile(int32_t precision, int32_t szI, int32_t szJ);
 
 /* ---------------- baroclinic terms: state equation, pressure gradient, tracers ------- */
@@ -367,9 +368,8 @@ int sf_phys_substep_coupled(const sf_phys_fields *fields, const sf_couple_fields
                             double dt, int32_t first, double cff1, void *stream);
 
 /* sf_phys_substep_fused coupled with the baroclinic step: the coupling of
- * sf_phys_substep_coupled inside the single-launch tile kernel (the forcing of the
- * ghost-source rows kept in LDS, the DU_avg2 terms from the fluxes the tile already
- * forms).  Tile height 4 or 8 (0: sf_phys_fused_default_tile).  FP64 results equal
+ * sf_phys_substep_coupled inside the single-launch tile kernel (the DU_avg2 terms from
+ * the fluxes the tile already forms).  Tile height 4 or 8 (0: chosen by the grid's size).  FP64 results equal
  * sf_phys_substep_coupled bit for bit; FP32 agrees to rounding (contraction on, as
  * sf_phys_substep_fused). */
 int sf_phys_substep_coupled_fused(const sf_phys_fields *fields, const sf_couple_fields *cpl, int32_t precision,
@@ -524,7 +524,7 @@ int sf_closure_stress(sf_mlp *mlp, const sf_phys_fields *fields, int32_t precisi
  * kernel: the corrector stage's surface stress is sf_closure_stress's sustr_eff /
  * svstr_eff of the substep's t1 state, the predictor keeps sustr / svstr.  f: the
  * Coriolis field in the state precision.  Tile height 4 or 8 (0: 4, the height whose
- * closure instances keep two waves per SIMD). */
+ * closure instances keep two waves per SIMD, or a 32 x 8 form on small grids). */
 int sf_phys_substep_closure_fused(const sf_phys_fields *fields, const sf_mlp *mlp, const void *f,
                                   int32_t precision, double dt, int32_t first, double cff1, int32_t tile_j,
                                   void *stream);

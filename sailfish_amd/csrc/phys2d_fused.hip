@@ -25,7 +25,7 @@ extern "C" int sf_phys_substep_fused(const sf_phys_fields *x, int32_t precision,
     SF_REQUIRE(x->rzeta[0] && x->rzeta[1] && x->rubar[0] && x->rubar[1] && x->rvbar[0] && x->rvbar[1],
                "sf_phys_substep_fused: null rhs slot");
     SF_REQUIRE(x->Zt_avg1 && x->DU_avg1 && x->DV_avg1, "sf_phys_substep_fused: null average");
-    const int tj = tile_j > 0 ? tile_j : sf_phys_fused_default_tile(precision, x->szI, x->szJ);
+    const int tj = tile_j > 0 ? tile_j : 0;
     if (precision == SF_FP64) return dispatch_tj<double>(x, dt, first, cff1, tj, stream);
     if (precision == SF_FP32) return sf_phys_fused_dispatch_f32(x, dt, first, cff1, tj, stream);
     sf::set_error("sf_phys_substep_fused: unknown precision %d", precision);
@@ -48,8 +48,8 @@ extern "C" int sf_phys_substep_coupled_fused(const sf_phys_fields *x, const sf_c
     SF_REQUIRE(!first || (cp->rufrc && cp->rvfrc && cp->Fu1 && cp->Fv1 && cp->Fu2 && cp->Fv2),
                "sf_phys_substep_coupled_fused: the first substep needs rufrc/rvfrc and the forcing history");
     SF_REQUIRE(cp->ab >= 0 && cp->ab <= 2, "sf_phys_substep_coupled_fused: ab=%d", cp->ab);
-    const int tj = tile_j > 0 ? tile_j : sf_phys_fused_default_tile(precision, x->szI, x->szJ);
-    SF_REQUIRE(tj == 4 || tj == 8, "sf_phys_substep_coupled_fused: tile height %d (4 or 8)", tj);
+    const int tj = tile_j > 0 ? tile_j : 0;
+    SF_REQUIRE(tj == 0 || tj == 4 || tj == 8, "sf_phys_substep_coupled_fused: tile height %d (4 or 8)", tj);
     if (precision == SF_FP64) return dispatch_tj<double>(x, dt, first, cff1, tj, stream, cp);
     if (precision == SF_FP32) return sf_phys_fused_dispatch_f32(x, dt, first, cff1, tj, stream, cp);
     sf::set_error("sf_phys_substep_coupled_fused: unknown precision %d", precision);
@@ -69,10 +69,8 @@ extern "C" int sf_phys_substep_closure_fused(const sf_phys_fields *x, const sf_m
     SF_REQUIRE(x->rzeta[0] && x->rzeta[1] && x->rubar[0] && x->rubar[1] && x->rvbar[0] && x->rvbar[1],
                "sf_phys_substep_closure_fused: null rhs slot");
     SF_REQUIRE(x->Zt_avg1 && x->DU_avg1 && x->DV_avg1, "sf_phys_substep_closure_fused: null average");
-    // default 64 x 4: those closure instances keep two waves per SIMD (the 64 x 8 ones need
-    // more registers than that allows, on any grid size)
-    const int tj = tile_j > 0 ? tile_j : 4;
-    SF_REQUIRE(tj == 4 || tj == 8, "sf_phys_substep_closure_fused: tile height %d (4 or 8)", tj);
+    const int tj = tile_j > 0 ? tile_j : 0;
+    SF_REQUIRE(tj == 0 || tj == 4 || tj == 8, "sf_phys_substep_closure_fused: tile height %d (4 or 8)", tj);
     const ClosureIn cl{mlp, f};
     if (precision == SF_FP64) return dispatch_tj<double>(x, dt, first, cff1, tj, stream, nullptr, &cl);
     if (precision == SF_FP32) return sf_phys_fused_dispatch_f32(x, dt, first, cff1, tj, stream, nullptr, &cl);

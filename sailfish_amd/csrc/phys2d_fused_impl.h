@@ -19,20 +19,28 @@
 //   C1     [2, T+3)    corrected zeta z2 (+ averages)   Z1 (reused as Z2)
 //   C2     [3, T+3)    corrected ubar, vbar             -
 //
-// Eleven planes of (TI+5)(TJ+5) values: the seven above plus ubar, vbar (t1), pm and
-// pn over the whole frame, filled in stage L, so that every stencil neighbour of
-// those fields is an LDS read.  The core points come first in every stage with the
-// same thread mapping, so a thread keeps its core points' values (z1, u1, v1, zs,
-// the predictor right-hand sides, metric factors) in registers from stage to stage.
-// The other read-only fields (h, fomn, the stresses, the old time level, the history
-// right-hand sides) are read from global memory where they are used.
+// Ten planes of (TI+5)(TJ+5) values: Z1, DU, DV, ZS, US, VS and ubar, vbar (t1), pm, pn over
+// the whole frame, filled in stage L, so that every stencil neighbour of those fields is an
+// LDS read; some instances add h, fomn and zeta(t0).  RZ stays with its thread (core) or in a
+// row and a column of C1's ring.  The core points come first in every stage with the same
+// thread mapping, so a thread keeps its core points' values (z1, u1, v1, zs, the predictor
+// right-hand sides, metric factors) in registers from stage to stage.  The other read-only
+// fields (fomn, the stresses, the old time level, the history right-hand sides) are read
+// from global memory where they are used.
 //
-// Closed-basin boundary: a ghost rho point takes the value of its clamped interior
-// source, computed by the same thread from the same stencil; u = 0 at i <= 1 and
-// i = L, v = 0 at j <= 1 and j = M; the remaining ghost rows/columns of u and v
-// copy their inward neighbour.  The tile origin is shifted by one point when
-// sz % T == 1 so that the source of every ghost u/v point is a core point of the
-// same tile (its predictor right-hand side was written by the same workgroup).
+// Small grids are bound by the chain of six load, barrier and divide latencies, not by any
+// rate: one wave per SIMD walks it.  There (NR > 0) the ring points get waves of their own,
+// which run beside the core's instead of after them, and every global load of the tile is
+// issued before the first barrier.
+//
+// Closed-basin boundary: a ghost rho point takes the value of its clamped interior source; u
+// = 0 at i <= 1 and i = L, v = 0 at j <= 1 and j = M; the remaining ghost rows/columns of u
+// and v copy their inward neighbour.  The source's thread writes its ghosts along with its own
+// value (to LDS and to global memory), so no thread evaluates a formula at a ghost: against
+// evaluating it there from fresh loads this saves 6 (FP32 64 x 8) to 31 (FP32 64 x 4)
+// registers and up to four dependent load latencies in boundary tiles (128 x 64 FP64: 10.8 ->
+// 9.1 us a substep).  The tile origin is shifted by one point when sz % T == 1 so that the
+// source of every ghost point of a tile's core is a core point of the same tile.
 //
 // Expression order is the one of phys2d_kernels.hip: the FP64 instances (contraction
 // off) equal the oracle and the four-launch form bit for bit; the FP32 instances are
@@ -42,6 +50,7 @@
 #include "mlp_net.h"
 #include "sf_internal.h"
 
+#include <type_traits>
 #include <vector>
 
 // the learned closure of a fused substep: the network and its Coriolis field
@@ -116,16 +125,34 @@ __device__ __forceinline__ void for_region(int tid, F &&fn)
     }
 }
 
-template <int TI, int TJ>
-struct PhysLds {
-    static constexpr int FW = TI + 5, FH = TJ + 5, FN = FW * FH, PLANES = 11;
-};
+// FP64 closure instances of 64-wide tiles keep the network's feature tiles in frame planes
+// 1..5, written only from stage A on, and one more (a barrier ends the closure phase): 27 KB
+// less LDS, so two 64 x 4 workgroups fit a CU.  Smaller planes cannot hold the tiles; they
+// get their own array.
+template <typename T, bool CLO, int TI>
+constexpr bool cl_tiles_in_frame = CLO && sizeof(T) == 8 && TI == 64;
 
-// FP64 closure instances keep the network's feature tiles in frame planes 1..6 (written
-// only from stage A on, after a barrier that ends the closure phase): 27 KB less LDS, so
-// two 64 x 4 workgroups fit a CU.  FP32 planes are too small; the tiles get their own array.
-template <typename T, bool CLO>
-constexpr bool cl_tiles_in_frame = CLO && sizeof(T) == 8;
+// Registers against LDS reads: LEAN instances keep h in a plane too and read the core points'
+// statics and t1 state from LDS where they are used; the others hold them in registers.
+//  - FP64: at 122 VGPRs 64 x 8 tiles on 512 threads fit two workgroups, 16 waves, a CU where
+//    256 threads of 209 VGPRs fit 8 (4096 x 4096: 970 us a substep against 1030; 2048 x 1024:
+//    120 / 128); the coupled split form drops from 142 to 126 (768 x 384: 26 / 34 us).
+//  - FP32 at streaming sizes (4096 x 4096: 547 us against 568); in the last-level cache the
+//    registers are faster (2048 x 1024: 57.3 against 59.1).
+template <typename T, int NT, int NR, bool CPL, bool NTS>
+constexpr bool lean_regs = NR > 0 ? (CPL && sizeof(T) == 8) : (NT == 512 && (sizeof(T) == 8 || NTS));
+
+// LDS planes of a tile's frame: the ten listed above.  NR > 0 (core and ring on different
+// waves): h, fomn and zeta(t0) over the frame as well, so that every stencil neighbour of a
+// static field is an LDS read and all global loads of the tile are issued together at its
+// start.
+template <typename T, int TI, int TJ, int NT, int NR, bool NTS, bool CPL, bool CLO>
+struct PhysLds {
+    static constexpr int FN = (TI + 5) * (TJ + 5);
+    static constexpr int SP = cl_tiles_in_frame<T, CLO, TI> ? 1 : 0;   // spare plane of the feature tiles
+    static constexpr bool HP = NR > 0 || CLO || lean_regs<T, NT, NR, CPL, NTS>;
+    static constexpr int PLANES = 10 + SP + (NR > 0 ? 3 : (HP ? 1 : 0));
+};
 
 // Element (f + d) of p, given the byte offset boff of element f: the address is the
 // array's scalar base plus a 32-bit vector offset (global_load saddr form).  The
@@ -214,39 +241,46 @@ __device__ __forceinline__ auto arg_ptr(const PFA<T> &P)
     else return &P;
 }
 
-template <typename T, int TI, int TJ, int NT, bool FIRST, bool NTS, bool CPL = false, bool CLO = false>
-__device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*sm)[PhysLds<TI, TJ>::FN],
-                                          T *side, double *sideF = nullptr, uint32_t *clX = nullptr,
-                                          float *clN = nullptr, T *clS = nullptr, T *clH = nullptr,
-                                          T *clF = nullptr)
+// Which points a call of phys_tile computes: every thread its core points and then its
+// share of the ring, or (NR > 0) the core points only / the ring only.
+enum TileRole { ROLE_ALL, ROLE_CORE, ROLE_RING };
+
+template <typename T, int TI, int TJ, int NT, int NR, TileRole ROLE, bool FIRST, bool NTS, bool CPL = false,
+          bool CLO = false>
+__device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*sm)[(TI + 5) * (TJ + 5)], T *rzl,
+                                          uint32_t *clX = nullptr, float *clN = nullptr, T *clF = nullptr)
 {
     // the arguments through a pointer that the closure instances re-derive after the closure
     // phase, so that pointers first needed from stage A on are loaded there again instead of
     // being held across the phase
     auto Pp = arg_ptr<T, CLO>(P);
+    constexpr bool XP = NR > 0;              // h, fomn, zeta(t0) planes; all loads issued first
+    constexpr bool CORE = ROLE != ROLE_RING, RINGS = ROLE != ROLE_CORE;
+    static_assert(XP == (ROLE != ROLE_ALL), "core and ring roles go with their own ring threads");
+    constexpr int RT = XP ? NR : NT;         // threads that share the ring
     constexpr int FW = TI + 5;
-    constexpr int KC = TI * TJ / NT;
+    constexpr int KC = CORE ? TI * TJ / NT : 1;
     constexpr uint32_t ES = sizeof(T);
     T *const sZ1 = sm[0], *const sZ2 = sm[0];
     T *const sDU = sm[1], *const sDV = sm[2];
-    T *const sZS = sm[3], *const sRZ = sm[4], *const sUS = sm[5], *const sVS = sm[6];
-    T *const sU1 = sm[7], *const sV1 = sm[8];   // ubar, vbar at t1 over the frame (read-only after L)
-    T *const sPM = sm[9], *const sPN = sm[10];  // pm, pn over the frame (read-only after L)
-    // predictor right-hand sides of the ghost-source row (j = 1, M-1) / column (i = 1, L-1)
-    T *const sRUlo = side, *const sRUhi = side + TI, *const sRVlo = side + 2 * TI, *const sRVhi = side + 2 * TI + TJ;
-    // CPL: the forcing F of the same ghost-source points (formed in P2 on the first substep)
-    double *const sFUlo = sideF, *const sFUhi = sideF + TI, *const sFVlo = sideF + 2 * TI,
-                 *const sFVhi = sideF + 2 * TI + TJ;
+    T *const sZS = sm[3], *const sUS = sm[4], *const sVS = sm[5];
+    // read-only after L: ubar, vbar at t1, pm, pn; HP: h; XP: fomn, zeta at t0
+    using Lds = PhysLds<T, TI, TJ, NT, NR, NTS, CPL, CLO>;
+    constexpr bool HP = Lds::HP, LEAN = lean_regs<T, NT, NR, CPL, NTS>;
+    constexpr int S0 = 6 + Lds::SP;
+    T *const sU1 = sm[S0], *const sV1 = sm[S0 + 1];
+    T *const sPM = sm[S0 + 2], *const sPN = sm[S0 + 3];
+    T *const sH = sm[HP ? S0 + 4 : 0];
+    T *const sFO = sm[XP ? S0 + 5 : 0], *const sZ0 = sm[XP ? S0 + 6 : 0];
 
     const int szI = Pp->szI, szJ = Pp->szJ, L = szI - 1, M = szJ - 1;
     const long long W = szI;
     const int fi0 = ti * TI - Pp->off_i - 3, fj0 = tj * TJ - Pp->off_j - 3;   // frame origin
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, rtid = XP ? tid - NT : tid;
     const T dt = Pp->dt;
     constexpr bool first = FIRST;
 
     auto inside = [&](int i, int j) { return i >= 0 && i <= L && j >= 0 && j <= M; };
-    auto clampi = [](int x, int lo, int hi) { return x < lo ? lo : (x > hi ? hi : x); };
     auto off = [&](int i, int j) { return (uint32_t)(j * szI + i) * ES; };
     auto offd = [&](int i, int j) { return (uint32_t)(j * szI + i) * 8u; };
     auto core_ab = [&](int k, int &a, int &b) {
@@ -254,72 +288,39 @@ __device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*s
         a = 3 + idx % TI;
         b = 3 + idx / TI;
     };
+    auto rho_int = [&](int i, int j) { return i >= 1 && i <= L - 1 && j >= 1 && j <= M - 1; };
+    auto u_int = [&](int i, int j) { return i >= 2 && i <= L - 1 && j >= 1 && j <= M - 1; };
+    auto v_int = [&](int i, int j) { return i >= 1 && i <= L - 1 && j >= 2 && j <= M - 1; };
 
-    // metric factors of a u point / v point at byte offset o
-    auto onu_at = [&](uint32_t o) { return T(2) * sf::recip(ldo(Pp->pn, -1, o) + ldo(Pp->pn, 0, o)); };
-    auto omu_at = [&](uint32_t o) { return T(2) * sf::recip(ldo(Pp->pm, -1, o) + ldo(Pp->pm, 0, o)); };
-    auto omv_at = [&](uint32_t o) { return T(2) * sf::recip(ldo(Pp->pm, -W, o) + ldo(Pp->pm, 0, o)); };
-    auto onv_at = [&](uint32_t o) { return T(2) * sf::recip(ldo(Pp->pn, -W, o) + ldo(Pp->pn, 0, o)); };
-    auto cffu_at = [&](uint32_t o) {
-        return (ldo(Pp->pm, 0, o) + ldo(Pp->pm, -1, o)) * (ldo(Pp->pn, 0, o) + ldo(Pp->pn, -1, o));
+    // Closed-basin ghosts: a ghost point is written by the thread of its interior source,
+    // together with the source's own value.  di (dj): step from a source in the outermost
+    // interior column (row) to its ghost, else 0.
+    auto ghost_di = [&](int i) { return i == 1 ? -1 : (i == L - 1 ? 1 : 0); };
+    auto ghost_dj = [&](int j) { return j == 1 ? -1 : (j == M - 1 ? 1 : 0); };
+    auto put_rho = [&](T *p, int o, int i, int j, T v) {
+        const int di = ghost_di(i), dj = ghost_dj(j) * FW;
+        p[o] = v;
+        if (di) p[o + di] = v;
+        if (dj) {
+            p[o + dj] = v;
+            if (di) p[o + dj + di] = v;
+        }
     };
-    auto cffv_at = [&](uint32_t o) {
-        return (ldo(Pp->pm, 0, o) + ldo(Pp->pm, -W, o)) * (ldo(Pp->pn, 0, o) + ldo(Pp->pn, -W, o));
+    auto put_u = [&](T *p, int o, int j, T v) {   // ghost rows
+        const int dj = ghost_dj(j) * FW;
+        p[o] = v;
+        if (dj) p[o + dj] = v;
     };
+    auto put_v = [&](T *p, int o, int i, T v) {   // ghost columns
+        const int di = ghost_di(i);
+        p[o] = v;
+        if (di) p[o + di] = v;
+    };
+    // u is 0 at i <= 1 and i = L (v likewise), written by the point itself
+    auto u_wall = [&](int i) { return i < 2 || i > L - 1; };
+    auto v_wall = [&](int j) { return j < 2 || j > M - 1; };
 
-    // generic (load-on-demand) inputs of the u / v right-hand side at offset f
-    auto load_u = [&](uint32_t f, int q) {
-        UVIn<T> x;
-        x.pmc = sPM[q];
-        x.pmb = sPM[q - 1];
-        x.pnc = sPN[q];
-        x.pnb = sPN[q - 1];
-        x.hb = ldo(Pp->h, -1, f);
-        x.hc = ldo(Pp->h, 0, f);
-        x.xb = sU1[q - 1];
-        x.xc = sU1[q];
-        x.xf = sU1[q + 1];
-        x.yf = sU1[q + FW];
-        x.yb = sU1[q - FW];
-        x.fc = ldo(Pp->fomn, 0, f);
-        x.fb = ldo(Pp->fomn, -1, f);
-        x.oc = sV1[q];
-        x.of = sV1[q + FW];
-        x.ob = sV1[q - 1];
-        x.obf = sV1[q + FW - 1];
-        x.st = ldo(Pp->sustr, 0, f);
-        x.x0 = first ? x.xc : ldo(Pp->u0, 0, f);
-        x.z0c = first ? T(0) : ldo(Pp->z0, 0, f);
-        x.z0b = first ? T(0) : ldo(Pp->z0, -1, f);
-        return x;
-    };
-    auto load_v = [&](uint32_t f, int q) {
-        UVIn<T> x;
-        x.pmc = sPM[q];
-        x.pmb = sPM[q - FW];
-        x.pnc = sPN[q];
-        x.pnb = sPN[q - FW];
-        x.hb = ldo(Pp->h, -W, f);
-        x.hc = ldo(Pp->h, 0, f);
-        x.xb = sV1[q - FW];
-        x.xc = sV1[q];
-        x.xf = sV1[q + FW];
-        x.yf = sV1[q + 1];
-        x.yb = sV1[q - 1];
-        x.fc = ldo(Pp->fomn, 0, f);
-        x.fb = ldo(Pp->fomn, -W, f);
-        x.oc = sU1[q];
-        x.of = sU1[q + 1];
-        x.ob = sU1[q - FW];
-        x.obf = sU1[q + 1 - FW];
-        x.st = ldo(Pp->svstr, 0, f);
-        x.x0 = first ? x.xc : ldo(Pp->v0, 0, f);
-        x.z0c = first ? T(0) : ldo(Pp->z0, 0, f);
-        x.z0b = first ? T(0) : ldo(Pp->z0, -W, f);
-        return x;
-    };
-
-    // metric factors of generic inputs (same expressions as onu_at / omu_at / cffu_at ...)
+    // metric factors of u / v inputs
     auto metrics_u = [&](UVIn<T> &x) {
         x.m1 = T(2) * sf::recip(x.pnb + x.pnc);
         x.m2 = T(2) * sf::recip(x.pmb + x.pmc);
@@ -330,21 +331,140 @@ __device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*s
         x.m2 = T(2) * sf::recip(x.pnb + x.pnc);
         x.cff = (x.pmc + x.pmb) * (x.pnc + x.pnb);
     };
+    // face fluxes DU, DV of a ring point of state (z, u, v) at LDS index o; h at the point and
+    // its west / south neighbour from the plane or (no plane) rh, rhw, rhs
+    auto flux = [&](const T *z, const T *u, const T *v, int i, int j, int o, T rh, T rhw, T rhs) {
+        T du = T(0), dv = T(0);
+        if (inside(i, j)) {
+            const T hc = HP ? sH[o] : rh;
+            if (i >= 1) {
+                const T onu = T(2) * sf::recip(sPN[o - 1] + sPN[o]);
+                du = ((T(0.5) * (((HP ? sH[o - 1] : rhw) + z[o - 1]) + (hc + z[o]))) * u[o]) * onu;
+            }
+            if (j >= 1) {
+                const T omv = T(2) * sf::recip(sPM[o - FW] + sPM[o]);
+                dv = ((T(0.5) * (((HP ? sH[o - FW] : rhs) + z[o - FW]) + (hc + z[o]))) * v[o]) * omv;
+            }
+        }
+        sDU[o] = du;
+        sDV[o] = dv;
+    };
+    // h of ring point (i, j): loaded ahead of the core's work where no plane holds it
+    auto load_h = [&](int i, int j, T &hc, T &hw, T &hs) {
+        if constexpr (!HP) {
+            if (inside(i, j)) {
+                const uint32_t f = off(i, j);
+                hc = ldo(Pp->h, 0, f);
+                if (i >= 1) hw = ldo(Pp->h, -1, f);
+                if (j >= 1) hs = ldo(Pp->h, -W, f);
+            }
+        }
+    };
+    // inputs of the u / v right-hand side of a ring point: the values that come from global
+    // memory (offset f) and those in the frame's planes (LDS index q)
+    auto load_u_global = [&](UVIn<T> &x, uint32_t f) {
+        if constexpr (!HP) {
+            x.hb = ldo(Pp->h, -1, f);
+            x.hc = ldo(Pp->h, 0, f);
+        }
+        if constexpr (!XP) {
+            x.fc = ldo(Pp->fomn, 0, f);
+            x.fb = ldo(Pp->fomn, -1, f);
+            x.z0c = first ? T(0) : ldo(Pp->z0, 0, f);
+            x.z0b = first ? T(0) : ldo(Pp->z0, -1, f);
+        }
+        x.st = ldo(Pp->sustr, 0, f);
+        if (!first) x.x0 = ldo(Pp->u0, 0, f);
+    };
+    auto load_u_lds = [&](UVIn<T> &x, int q) {
+        x.pmc = sPM[q];
+        x.pmb = sPM[q - 1];
+        x.pnc = sPN[q];
+        x.pnb = sPN[q - 1];
+        if constexpr (HP) {
+            x.hb = sH[q - 1];
+            x.hc = sH[q];
+        }
+        if constexpr (XP) {
+            x.fc = sFO[q];
+            x.fb = sFO[q - 1];
+            x.z0c = first ? T(0) : sZ0[q];
+            x.z0b = first ? T(0) : sZ0[q - 1];
+        }
+        x.xb = sU1[q - 1];
+        x.xc = sU1[q];
+        x.xf = sU1[q + 1];
+        x.yf = sU1[q + FW];
+        x.yb = sU1[q - FW];
+        x.oc = sV1[q];
+        x.of = sV1[q + FW];
+        x.ob = sV1[q - 1];
+        x.obf = sV1[q + FW - 1];
+        if (first) x.x0 = x.xc;
+    };
+    auto load_v_global = [&](UVIn<T> &x, uint32_t f) {
+        if constexpr (!HP) {
+            x.hb = ldo(Pp->h, -W, f);
+            x.hc = ldo(Pp->h, 0, f);
+        }
+        if constexpr (!XP) {
+            x.fc = ldo(Pp->fomn, 0, f);
+            x.fb = ldo(Pp->fomn, -W, f);
+            x.z0c = first ? T(0) : ldo(Pp->z0, 0, f);
+            x.z0b = first ? T(0) : ldo(Pp->z0, -W, f);
+        }
+        x.st = ldo(Pp->svstr, 0, f);
+        if (!first) x.x0 = ldo(Pp->v0, 0, f);
+    };
+    auto load_v_lds = [&](UVIn<T> &x, int q) {
+        x.pmc = sPM[q];
+        x.pmb = sPM[q - FW];
+        x.pnc = sPN[q];
+        x.pnb = sPN[q - FW];
+        if constexpr (HP) {
+            x.hb = sH[q - FW];
+            x.hc = sH[q];
+        }
+        if constexpr (XP) {
+            x.fc = sFO[q];
+            x.fb = sFO[q - FW];
+            x.z0c = first ? T(0) : sZ0[q];
+            x.z0b = first ? T(0) : sZ0[q - FW];
+        }
+        x.xb = sV1[q - FW];
+        x.xc = sV1[q];
+        x.xf = sV1[q + FW];
+        x.yf = sV1[q + 1];
+        x.yb = sV1[q - 1];
+        x.oc = sU1[q];
+        x.of = sU1[q + 1];
+        x.ob = sU1[q - FW];
+        x.obf = sU1[q + 1 - FW];
+        if (first) x.x0 = x.xc;
+    };
 
-    // CPL: forcing of the predictor right-hand side r of a u (v) point at FP64 byte offset
-    // fd: the first substep forms F = rufrc - r and adds its Adams-Bashforth
-    // extrapolation over the baroclinic steps, the others add F (as pred_forcing of the
-    // four-launch form); F is returned in Fk
-    auto pred_forcing = [&](bool vdir, uint32_t fd, T r, double &Fk) {
-        const double *Fo = vdir ? Pp->c.Fv : Pp->c.Fu;
+    // CPL: forcing of the predictor right-hand side r of a u (v) point: the first substep
+    // forms F = rufrc - r and adds its Adams-Bashforth extrapolation over the baroclinic
+    // steps, the others add F (as pred_forcing of the four-launch form); F is returned in Fk
+    struct Forcing { double f0, f1, f2; };
+    auto load_forcing = [&](bool vdir, uint32_t fd) {
+        Forcing q{0.0, 0.0, 0.0};
         if constexpr (FIRST) {
-            const double F = ldo(vdir ? Pp->c.rvfrc : Pp->c.rufrc, 0, fd) - (double)r;
-            Fk = F;
-            const double F1 = Pp->c.ab > 0 ? ldo(vdir ? Pp->c.Fv1 : Pp->c.Fu1, 0, fd) : 0.0;
-            const double F2 = Pp->c.ab > 1 ? ldo(vdir ? Pp->c.Fv2 : Pp->c.Fu2, 0, fd) : 0.0;
-            return r + T(sf::ab_extrapolate(Pp->c.ab, F, F1, F2));
+            q.f0 = ldo(vdir ? Pp->c.rvfrc : Pp->c.rufrc, 0, fd);
+            if (Pp->c.ab > 0) q.f1 = ldo(vdir ? Pp->c.Fv1 : Pp->c.Fu1, 0, fd);
+            if (Pp->c.ab > 1) q.f2 = ldo(vdir ? Pp->c.Fv2 : Pp->c.Fu2, 0, fd);
         } else {
-            Fk = ldo(Fo, 0, fd);
+            q.f0 = ldo(vdir ? Pp->c.Fv : Pp->c.Fu, 0, fd);
+        }
+        return q;
+    };
+    auto pred_forcing = [&](const Forcing &q, T r, double &Fk) {
+        if constexpr (FIRST) {
+            const double F = q.f0 - (double)r;
+            Fk = F;
+            return r + T(sf::ab_extrapolate(Pp->c.ab, F, q.f1, q.f2));
+        } else {
+            Fk = q.f0;
             return r + T(Fk);
         }
     };
@@ -354,7 +474,7 @@ __device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*s
     const T c1dt = first ? T(0.5) * dt : dt;
     auto gzp = [&](int o, T z0) { return first ? T(0.5) * (sZ1[o] + sZS[o]) : cff5 * sZ1[o] + cff4 * (z0 + sZS[o]); };
     auto Dbp = [&](int o, T h, T z0) { return first ? h + sZ1[o] : h + z0; };
-    auto pred_u = [&](int q, const UVIn<T> &x, T &r, uint32_t fd = 0, double *Fk = nullptr) {
+    auto pred_u = [&](int q, const UVIn<T> &x, T &r, const Forcing &fq, double &Fk) {
         const T onu = x.m1, omu = x.m2;
         const T g0 = gzp(q - 1, x.z0b), g1 = gzp(q, x.z0c);
         r = ((T(0.5) * Pp->g) * onu) * ((x.hb + x.hc) * (g0 - g1) + (g0 * g0 - g1 * g1));
@@ -368,15 +488,11 @@ __device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*s
         r = r + T(0.5) * (cr1 + cr0);
         r = r - ((Pp->rdrg * x.xc) * omu) * onu;
         r = r + (x.st * omu) * onu;
-        if constexpr (CPL) {
-            double F;
-            r = pred_forcing(false, fd, r, F);
-            if (Fk) *Fk = F;
-        }
+        if constexpr (CPL) r = pred_forcing(fq, r, Fk);
         const T fac = sf::recip((x.hc + sZS[q]) + (x.hb + sZS[q - 1]));
         return (x.x0 * (Dbp(q, x.hc, x.z0c) + Dbp(q - 1, x.hb, x.z0b)) + (x.cff * c1dt) * r) * fac;
     };
-    auto pred_v = [&](int q, const UVIn<T> &x, T &r, uint32_t fd = 0, double *Fk = nullptr) {
+    auto pred_v = [&](int q, const UVIn<T> &x, T &r, const Forcing &fq, double &Fk) {
         const T omv = x.m1, onv = x.m2;
         const T g0 = gzp(q - FW, x.z0b), g1 = gzp(q, x.z0c);
         r = ((T(0.5) * Pp->g) * omv) * ((x.hb + x.hc) * (g0 - g1) + (g0 * g0 - g1 * g1));
@@ -390,11 +506,7 @@ __device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*s
         r = r - T(0.5) * (cr1 + cr0);
         r = r - ((Pp->rdrg * x.xc) * omv) * onv;
         r = r + (x.st * omv) * onv;
-        if constexpr (CPL) {
-            double F;
-            r = pred_forcing(true, fd, r, F);
-            if (Fk) *Fk = F;
-        }
+        if constexpr (CPL) r = pred_forcing(fq, r, Fk);
         const T fac = sf::recip((x.hc + sZS[q]) + (x.hb + sZS[q - FW]));
         return (x.x0 * (Dbp(q, x.hc, x.z0c) + Dbp(q - FW, x.hb, x.z0b)) + (x.cff * c1dt) * r) * fac;
     };
@@ -407,119 +519,265 @@ __device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*s
     T clsu[CLO ? KC : 1], clsv[CLO ? KC : 1];       // CLO: wind stress at the core point
     T pm_[KC], pn_[KC];
     T onuc[KC], omuc[KC], cffuc[KC], omvc[KC], onvc[KC], cffvc[KC], pmnc[KC];
-    T zsc[KC], ruc[KC], rvc[KC], duc[KC], dvc[KC];
+    T zsc[KC], rzc[KC], ruc[KC], rvc[KC], duc[KC], dvc[KC];
     // G1 (predictor) and G2 (corrector) prefetch
     T z0c_[KC], z0w_[KC], z0s_[KC], u0c_[KC], v0c_[KC], fo_[KC], fow_[KC], fos_[KC], su_[KC], sv_[KC];
     T rz0_[KC], ru0_[KC], rv0_[KC], z1w_[KC], z1s_[KC];
     double zt_[KC], dua_[KC], dva_[KC];
+    // core values at slot k, LDS index o: held in registers, or (LEAN) read where used
+    auto h_c = [&](int k, int o) { if constexpr (LEAN) return sH[o]; else return hc_[k]; };
+    auto h_w = [&](int k, int o) { if constexpr (LEAN) return sH[o - 1]; else return hw_[k]; };
+    auto h_s = [&](int k, int o) { if constexpr (LEAN) return sH[o - FW]; else return hs_[k]; };
+    auto u1_c = [&](int k, int o) { if constexpr (LEAN) return sU1[o]; else return u1c[k]; };
+    auto v1_c = [&](int k, int o) { if constexpr (LEAN) return sV1[o]; else return v1c[k]; };
+    auto cff_u = [&](int o) { return (sPM[o] + sPM[o - 1]) * (sPN[o] + sPN[o - 1]); };
+    auto cff_v = [&](int o) { return (sPM[o] + sPM[o - FW]) * (sPN[o] + sPN[o - FW]); };
     // CPL: stage-A fluxes of the core points, their forcing F and DU_avg2 / DV_avg2
-    double du1c[KC], dv1c[KC], fuc[KC], fvc[KC], du2_[KC], dv2_[KC];
+    T du1c[KC], dv1c[KC], fuc[KC], fvc[KC];
+    double du2_[KC], dv2_[KC];
+    Forcing fqu[KC], fqv[KC];
 
-    // fast-path predicates of a core point (its computations use only its own offset)
-    auto rho_int = [&](int i, int j) { return i >= 1 && i <= L - 1 && j >= 1 && j <= M - 1; };
-    auto u_int = [&](int i, int j) { return i >= 2 && i <= L - 1 && j >= 1 && j <= M - 1; };
-    auto v_int = [&](int i, int j) { return i >= 1 && i <= L - 1 && j >= 2 && j <= M - 1; };
-
-    if constexpr (CLO)   // input normalisation of the closure (read after L's barrier)
-        if (tid < 2 * NIN) clN[tid] = Pp->cl_norm[tid];
-
-    // ---- G0 + L: z1 over the frame; core statics -----------------------------------------
-#pragma unroll
-    for (int k = 0; k < KC; k++) {
+    // core: the predictor's inputs (G1)
+    auto issue_pred = [&](int k) {
         int a, b;
         core_ab(k, a, b);
         const int i = fi0 + a, j = fj0 + b;
-        cin[k] = inside(i, j);
-        cf[k] = cin[k] ? off(i, j) : 0u;
         const uint32_t f = cf[k];
-        // values below are read only under the predicate they are loaded under
-        z1c[k] = T(0);
-        if (cin[k]) {
-            z1c[k] = ldo(Pp->z1, 0, f);
-            u1c[k] = ldo(Pp->u1, 0, f);
-            v1c[k] = ldo(Pp->v1, 0, f);
-            hc_[k] = ldo(Pp->h, 0, f);
-            pm_[k] = ldo(Pp->pm, 0, f);
-            pn_[k] = ldo(Pp->pn, 0, f);
-            if (i >= 1) hw_[k] = ldo(Pp->h, -1, f);
-            if (j >= 1) hs_[k] = ldo(Pp->h, -W, f);
-        }
-        if constexpr (CLO) {   // the closure's f and wind stress, in flight with the frame loads
-            clf0[k] = cin[k] ? ldo(Pp->cl_f, 0, f) : T(0);
-            clsu[k] = u_int(i, j) ? ldo(Pp->sustr, 0, f) : T(0);
-            clsv[k] = v_int(i, j) ? ldo(Pp->svstr, 0, f) : T(0);
-        }
-    }
-    {
-        constexpr int RING = ring_size<TI, TJ, 3, 2>();
-        constexpr int RS = (RING + NT - 1) / NT;
-        T rz[RS], ru[RS], rv[RS], rm[RS], rn[RS];
-        T rh[CLO ? RS : 1], rf[CLO ? RS : 1];   // CLO: h and f of the ring for the closure's stencils
-        int ro[RS];
-#pragma unroll
-        for (int s = 0; s < RS; s++) {
-            const int t = tid + s * NT;
-            rz[s] = ru[s] = rv[s] = rm[s] = rn[s] = T(0);
-            if constexpr (CLO) rh[s] = rf[s] = T(0);
-            ro[s] = -1;
-            if (t < RING) {
-                int a, b;
-                ring_point<TI, TJ, 3, 2>(t, a, b);
-                const int i = fi0 + a, j = fj0 + b;
-                ro[s] = b * FW + a;
-                if (inside(i, j)) {
-                    const uint32_t f = off(i, j);
-                    rz[s] = ldo(Pp->z1, 0, f);
-                    ru[s] = ldo(Pp->u1, 0, f);
-                    rv[s] = ldo(Pp->v1, 0, f);
-                    rm[s] = ldo(Pp->pm, 0, f);
-                    rn[s] = ldo(Pp->pn, 0, f);
-                    if constexpr (CLO) {
-                        rh[s] = ldo(Pp->h, 0, f);
-                        rf[s] = ldo(Pp->cl_f, 0, f);
-                    }
-                }
+        const bool ui = cin[k] && u_int(i, j), vi = cin[k] && v_int(i, j), ri_ = cin[k] && rho_int(i, j);
+        if constexpr (!XP) {
+            if (ri_) {   // holds every u and v point
+                if (!first) z0c_[k] = ldo(Pp->z0, 0, f);
+                fo_[k] = ldo(Pp->fomn, 0, f);
             }
         }
+        if (ui) {
+            if constexpr (!XP) {
+                if (!first) z0w_[k] = ldo(Pp->z0, -1, f);
+                fow_[k] = ldo(Pp->fomn, -1, f);
+            }
+            if (!first) u0c_[k] = ldo(Pp->u0, 0, f);
+            su_[k] = ldo(Pp->sustr, 0, f);
+            if constexpr (CPL && XP) fqu[k] = load_forcing(false, offd(i, j));
+        }
+        if (vi) {
+            if constexpr (!XP) {
+                if (!first) z0s_[k] = ldo(Pp->z0, -W, f);
+                fos_[k] = ldo(Pp->fomn, -W, f);
+            }
+            if (!first) v0c_[k] = ldo(Pp->v0, 0, f);
+            sv_[k] = ldo(Pp->svstr, 0, f);
+            if constexpr (CPL && XP) fqv[k] = load_forcing(true, offd(i, j));
+        }
+    };
+    // core: the averages of an interior point, issued in C0: the ring of P2 needs the registers
+    auto issue_avg = [&](int k, uint32_t fd) {
+        zt_[k] = ldavg<NTS>(Pp->Zt, fd);
+        dua_[k] = ldavg<NTS>(Pp->DUa, fd);
+        dva_[k] = ldavg<NTS>(Pp->DVa, fd);
+        if constexpr (CPL) {
+            du2_[k] = FIRST ? 0.0 : ldavg<NTS>(Pp->c.DU_avg2, fd);
+            dv2_[k] = FIRST ? 0.0 : ldavg<NTS>(Pp->c.DV_avg2, fd);
+        }
+    };
+    // core: the corrector's inputs (G2); LEAN: issued in C0, with the Coriolis factors, the
+    // stress and the forcing read again rather than held across the ring of P2
+    auto issue_corr = [&](int k, bool avg) {
+        int a, b;
+        core_ab(k, a, b);
+        const int i = fi0 + a, j = fj0 + b;
+        const uint32_t f = cf[k], fd = offd(i, j);
+        constexpr bool again = LEAN && !XP;
+        if (rho_int(i, j)) {
+            if (!first) rz0_[k] = ldo(Pp->rz0, 0, f);
+            if (avg) issue_avg(k, fd);
+            if constexpr (again) fo_[k] = ldo(Pp->fomn, 0, f);
+        }
+        if (u_int(i, j)) {
+            if (!first) ru0_[k] = ldo(Pp->ru0, 0, f);
+            if constexpr (again) {
+                fow_[k] = ldo(Pp->fomn, -1, f);
+                su_[k] = ldo(Pp->sustr, 0, f);
+                if constexpr (CPL && !FIRST) fuc[k] = T(ldo(Pp->c.Fu, 0, fd));
+            }
+        }
+        if (v_int(i, j)) {
+            if (!first) rv0_[k] = ldo(Pp->rv0, 0, f);
+            if constexpr (again) {
+                fos_[k] = ldo(Pp->fomn, -W, f);
+                sv_[k] = ldo(Pp->svstr, 0, f);
+                if constexpr (CPL && !FIRST) fvc[k] = T(ldo(Pp->c.Fv, 0, fd));
+            }
+        }
+    };
+
+    // ring slots of each stage
+    constexpr int RSL = (ring_size<TI, TJ, 3, 2>() + RT - 1) / RT;
+    constexpr int RSP2 = (ring_size<TI, TJ, 1, 1>() + RT - 1) / RT;
+    constexpr int RSC1 = (ring_size<TI, TJ, 1, 0>() + RT - 1) / RT;
+    // XP: inputs of the ring's later stages, loaded with the frame
+    UVIn<T> xu[XP ? RSP2 : 1], xv[XP ? RSP2 : 1];
+    Forcing xfu[XP ? RSP2 : 1], xfv[XP ? RSP2 : 1];
+    T xrz0[XP ? RSC1 : 1];
+
+    if constexpr (CLO && CORE)   // input normalisation of the closure (read after L's barrier)
+        if (tid < 2 * NIN) clN[tid] = Pp->cl_norm[tid];
+
+    // ---- G0 + L: z1 over the frame; core statics -----------------------------------------
+    if constexpr (CORE) {
+        T z0f[KC], fof[KC];
 #pragma unroll
         for (int k = 0; k < KC; k++) {
             int a, b;
             core_ab(k, a, b);
-            const int o = b * FW + a;
-            sZ1[o] = z1c[k];
-            sU1[o] = cin[k] ? u1c[k] : T(0);
-            sV1[o] = cin[k] ? v1c[k] : T(0);
-            sPM[o] = cin[k] ? pm_[k] : T(0);
-            sPN[o] = cin[k] ? pn_[k] : T(0);
-            if constexpr (CLO) {
-                clH[o] = cin[k] ? hc_[k] : T(0);
-                clF[o] = clf0[k];
-            }
-        }
-#pragma unroll
-        for (int s = 0; s < RS; s++)
-            if (ro[s] >= 0) {
-                sZ1[ro[s]] = rz[s];
-                sU1[ro[s]] = ru[s];
-                sV1[ro[s]] = rv[s];
-                sPM[ro[s]] = rm[s];
-                sPN[ro[s]] = rn[s];
-                if constexpr (CLO) {
-                    clH[ro[s]] = rh[s];
-                    clF[ro[s]] = rf[s];
+            const int i = fi0 + a, j = fj0 + b;
+            cin[k] = inside(i, j);
+            cf[k] = cin[k] ? off(i, j) : 0u;
+            const uint32_t f = cf[k];
+            // values below are read only under the predicate they are loaded under
+            z1c[k] = u1c[k] = v1c[k] = hc_[k] = pm_[k] = pn_[k] = T(0);
+            if constexpr (XP) z0f[k] = fof[k] = T(0);
+            if (cin[k]) {
+                z1c[k] = ldo(Pp->z1, 0, f);
+                u1c[k] = ldo(Pp->u1, 0, f);
+                v1c[k] = ldo(Pp->v1, 0, f);
+                hc_[k] = ldo(Pp->h, 0, f);
+                pm_[k] = ldo(Pp->pm, 0, f);
+                pn_[k] = ldo(Pp->pn, 0, f);
+                if constexpr (XP) {
+                    fof[k] = ldo(Pp->fomn, 0, f);
+                    if (!first) z0f[k] = ldo(Pp->z0, 0, f);
+                } else if constexpr (!LEAN) {
+                    if (i >= 1) hw_[k] = ldo(Pp->h, -1, f);
+                    if (j >= 1) hs_[k] = ldo(Pp->h, -W, f);
                 }
             }
+            if constexpr (CLO) {   // the closure's f and wind stress, in flight with the frame loads
+                clf0[k] = cin[k] ? ldo(Pp->cl_f, 0, f) : T(0);
+                clsu[k] = u_int(i, j) ? ldo(Pp->sustr, 0, f) : T(0);
+                clsv[k] = v_int(i, j) ? ldo(Pp->svstr, 0, f) : T(0);
+            }
+        }
+        if constexpr (XP) {
+#pragma unroll
+            for (int k = 0; k < KC; k++) issue_pred(k);
+#pragma unroll
+            for (int k = 0; k < KC; k++) issue_corr(k, true);
+#pragma unroll
+            for (int k = 0; k < KC; k++) {
+                int a, b;
+                core_ab(k, a, b);
+                const int o = b * FW + a;
+                sFO[o] = fof[k];
+                if (!first) sZ0[o] = z0f[k];
+            }
+        }
+    }
+    {
+        T rz[RSL], ru[RSL], rv[RSL], rm[RSL], rn[RSL], rfo[XP ? RSL : 1], rz0[XP ? RSL : 1];
+        T rh[HP ? RSL : 1], rf[CLO ? RSL : 1];   // CLO: f of the ring for the closure's stencils
+        int ro[RSL];
+        if constexpr (RINGS) {
+            constexpr int RING = ring_size<TI, TJ, 3, 2>();
+#pragma unroll
+            for (int s = 0; s < RSL; s++) {
+                const int t = rtid + s * RT;
+                rz[s] = ru[s] = rv[s] = rm[s] = rn[s] = T(0);
+                if constexpr (HP) rh[s] = T(0);
+                if constexpr (XP) rfo[s] = rz0[s] = T(0);
+                if constexpr (CLO) rf[s] = T(0);
+                ro[s] = -1;
+                if (t < RING) {
+                    int a, b;
+                    ring_point<TI, TJ, 3, 2>(t, a, b);
+                    const int i = fi0 + a, j = fj0 + b;
+                    ro[s] = b * FW + a;
+                    if (inside(i, j)) {
+                        const uint32_t f = off(i, j);
+                        rz[s] = ldo(Pp->z1, 0, f);
+                        ru[s] = ldo(Pp->u1, 0, f);
+                        rv[s] = ldo(Pp->v1, 0, f);
+                        rm[s] = ldo(Pp->pm, 0, f);
+                        rn[s] = ldo(Pp->pn, 0, f);
+                        if constexpr (HP) rh[s] = ldo(Pp->h, 0, f);
+                        if constexpr (XP) {
+                            rfo[s] = ldo(Pp->fomn, 0, f);
+                            if (!first) rz0[s] = ldo(Pp->z0, 0, f);
+                        }
+                        if constexpr (CLO) rf[s] = ldo(Pp->cl_f, 0, f);
+                    }
+                }
+            }
+            if constexpr (XP) {   // the later stages' global inputs, in flight behind the frame
+#pragma unroll
+                for (int s = 0; s < RSP2; s++) {
+                    const int t = rtid + s * RT;
+                    if (t < ring_size<TI, TJ, 1, 1>()) {
+                        int a, b;
+                        ring_point<TI, TJ, 1, 1>(t, a, b);
+                        const int i = fi0 + a, j = fj0 + b;
+                        if (u_int(i, j)) {
+                            load_u_global(xu[s], off(i, j));
+                            if constexpr (CPL) xfu[s] = load_forcing(false, offd(i, j));
+                        }
+                        if (v_int(i, j)) {
+                            load_v_global(xv[s], off(i, j));
+                            if constexpr (CPL) xfv[s] = load_forcing(true, offd(i, j));
+                        }
+                    }
+                }
+#pragma unroll
+                for (int s = 0; s < RSC1; s++) {
+                    const int t = rtid + s * RT;
+                    if (t < ring_size<TI, TJ, 1, 0>()) {
+                        int a, b;
+                        ring_point<TI, TJ, 1, 0>(t, a, b);
+                        if (!first && rho_int(fi0 + a, fj0 + b)) xrz0[s] = ldo(Pp->rz0, 0, off(fi0 + a, fj0 + b));
+                    }
+                }
+            }
+        }
+        if constexpr (CORE) {
+#pragma unroll
+            for (int k = 0; k < KC; k++) {
+                int a, b;
+                core_ab(k, a, b);
+                const int o = b * FW + a;
+                sZ1[o] = z1c[k];
+                sU1[o] = u1c[k];
+                sV1[o] = v1c[k];
+                sPM[o] = pm_[k];
+                sPN[o] = pn_[k];
+                if constexpr (HP) sH[o] = hc_[k];
+                if constexpr (CLO) clF[o] = clf0[k];
+            }
+        }
+        if constexpr (RINGS) {
+#pragma unroll
+            for (int s = 0; s < RSL; s++)
+                if (ro[s] >= 0) {
+                    sZ1[ro[s]] = rz[s];
+                    sU1[ro[s]] = ru[s];
+                    sV1[ro[s]] = rv[s];
+                    sPM[ro[s]] = rm[s];
+                    sPN[ro[s]] = rn[s];
+                    if constexpr (HP) sH[ro[s]] = rh[s];
+                    if constexpr (XP) {
+                        sFO[ro[s]] = rfo[s];
+                        if (!first) sZ0[ro[s]] = rz0[s];
+                    }
+                    if constexpr (CLO) clF[ro[s]] = rf[s];
+                }
+        }
     }
     lds_barrier();
 
     // ---- CL: the learned closure's corrector-stage stresses at the core points ----------
-    // Each wave evaluates the network on its core row(s) of 64 points (features from the
+    // Each wave evaluates the network on its core points, 64 at a time (features from the
     // t1 frame planes and the h, f planes staged with them) and keeps
-    // sustr + R_u D_u / svstr + R_v D_v of its points for C2; those of the ghost-source
-    // rows / columns (j = 1, M-1 / i = 1, L-1)
-    // also go to clS for the ghost points of C2.  The same arithmetic as sf_closure_stress.
+    // sustr + R_u D_u / svstr + R_v D_v of its points for C2.  The same arithmetic as
+    // sf_closure_stress.
     T csu[KC], csv[KC];
-    if constexpr (CLO) {
+    if constexpr (CLO && CORE) {
 #pragma clang fp contract(off)   // the same roundings as sf_closure_stress in both precisions
         Fwd Wn;
         load_fwd(Wn, Pp->cl_wpk, Pp->cl_w);
@@ -529,165 +787,125 @@ __device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*s
             int a, b;
             core_ab(k, a, b);
             const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
-            const bool in = rho_int(i, j);
-            const uint32_t f = cf[k];
-            float xv[NIN];
+            float xvv[NIN];
 #pragma unroll
             for (int kk = 0; kk < NIN; kk++) {
                 const int fld = kk / 9, dj = (kk % 9) / 3 - 1, di = kk % 3 - 1;
                 const int d = dj * FW + di;
-                const T *pl = fld == 0 ? sU1 : fld == 1 ? sV1 : fld == 2 ? sZ1 : fld == 3 ? clH : clF;
+                const T *pl = fld == 0 ? sU1 : fld == 1 ? sV1 : fld == 2 ? sZ1 : fld == 3 ? sH : clF;
                 const T cv = pl[o], nv = pl[o + d];
-                xv[kk] = (dj == 0 && di == 0) ? (float)cv : (float)(nv - cv);
+                xvv[kk] = (dj == 0 && di == 0) ? (float)cv : (float)(nv - cv);
             }
-            closure_row(X, tid & 63, xv, clN);
+            closure_row(X, tid & 63, xvv, clN);
             float zu, zv;
             closure_eval(Wn, X, zu, zv);
             csu[k] = csv[k] = T(0);   // read in C2 only at u / v interior points
             if (u_int(i, j)) {
-                const T Du = T(0.5) * ((hw_[k] + sZ1[o - 1]) + (hc_[k] + sZ1[o]));
+                const T Du = T(0.5) * ((sH[o - 1] + sZ1[o - 1]) + (sH[o] + sZ1[o]));
                 csu[k] = clsu[k] + T(zu * Pp->cl_ynorm[1] + Pp->cl_ynorm[0]) * Du;
-                if (j == 1) clS[a - 3] = csu[k];
-                if (j == M - 1) clS[TI + a - 3] = csu[k];
             }
             if (v_int(i, j)) {
-                const T Dv = T(0.5) * ((hs_[k] + sZ1[o - FW]) + (hc_[k] + sZ1[o]));
+                const T Dv = T(0.5) * ((sH[o - FW] + sZ1[o - FW]) + (sH[o] + sZ1[o]));
                 csv[k] = clsv[k] + T(zv * Pp->cl_ynorm[3] + Pp->cl_ynorm[2]) * Dv;
-                if (i == 1) clS[2 * TI + b - 3] = csv[k];
-                if (i == L - 1) clS[2 * TI + TJ + b - 3] = csv[k];
             }
         }
     }
 
-    if constexpr (cl_tiles_in_frame<T, CLO>) lds_barrier();   // feature tiles read; planes 1..6 free
-    if constexpr (CLO) asm volatile("" : "+s"(Pp));
+    if constexpr (cl_tiles_in_frame<T, CLO, TI>) lds_barrier();   // feature tiles read; planes 1..6 free
+    if constexpr (CLO && CORE) asm volatile("" : "+s"(Pp));
 
     // ---- A: DU1 at u points, DV1 at v points ---------------------------------------------
     {
         constexpr int RING = ring_size<TI, TJ, 2, 2>();
-        constexpr int RS = (RING + NT - 1) / NT;
+        constexpr int RS = (RING + RT - 1) / RT;
         T rh[RS], rhw[RS], rhs[RS];
-        int ro[RS], ri[RS], rj[RS];
+        if constexpr (RINGS) {
 #pragma unroll
-        for (int s = 0; s < RS; s++) {
-            const int t = tid + s * NT;
-            ro[s] = -1;
-            ri[s] = rj[s] = -1;
-            if (t < RING) {
+            for (int s = 0; s < RS; s++) {
                 int a, b;
-                ring_point<TI, TJ, 2, 2>(t, a, b);
-                const int i = fi0 + a, j = fj0 + b;
-                ro[s] = b * FW + a;
-                if (inside(i, j)) {
-                    ri[s] = i;
-                    rj[s] = j;
-                    const uint32_t f = off(i, j);
-                    rh[s] = ldo(Pp->h, 0, f);
-                    if (i >= 1) rhw[s] = ldo(Pp->h, -1, f);
-                    if (j >= 1) rhs[s] = ldo(Pp->h, -W, f);
-                }
+                ring_point<TI, TJ, 2, 2>(rtid + s * RT, a, b);
+                if (rtid + s * RT < RING) load_h(fi0 + a, fj0 + b, rh[s], rhw[s], rhs[s]);
             }
         }
         // core: metric factors, fluxes
+        if constexpr (CORE) {
 #pragma unroll
-        for (int k = 0; k < KC; k++) {
-            int a, b;
-            core_ab(k, a, b);
-            const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
-            T du = T(0), dv = T(0);
-            if (cin[k]) {
-                pmnc[k] = pm_[k] * pn_[k];
-                if (i >= 1) {
-                    const T pmw = sPM[o - 1], pnw = sPN[o - 1];
-                    onuc[k] = T(2) * sf::recip(pnw + pn_[k]);
-                    omuc[k] = T(2) * sf::recip(pmw + pm_[k]);
-                    cffuc[k] = (pm_[k] + pmw) * (pn_[k] + pnw);
-                    du = ((T(0.5) * ((hw_[k] + sZ1[o - 1]) + (hc_[k] + sZ1[o]))) * u1c[k]) * onuc[k];
+            for (int k = 0; k < KC; k++) {
+                int a, b;
+                core_ab(k, a, b);
+                const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
+                if constexpr (XP && !LEAN) {
+                    hw_[k] = sH[o - 1];
+                    hs_[k] = sH[o - FW];
                 }
-                if constexpr (CPL) du1c[k] = (double)du;
-                if (j >= 1) {
-                    const T pms = sPM[o - FW], pns = sPN[o - FW];
-                    omvc[k] = T(2) * sf::recip(pms + pm_[k]);
-                    onvc[k] = T(2) * sf::recip(pns + pn_[k]);
-                    cffvc[k] = (pm_[k] + pms) * (pn_[k] + pns);
-                    dv = ((T(0.5) * ((hs_[k] + sZ1[o - FW]) + (hc_[k] + sZ1[o]))) * v1c[k]) * omvc[k];
+                T du = T(0), dv = T(0);
+                if (cin[k]) {
+                    const T pmc = LEAN ? sPM[o] : pm_[k], pnc = LEAN ? sPN[o] : pn_[k];
+                    if constexpr (!LEAN) pmnc[k] = pmc * pnc;
+                    if (i >= 1) {
+                        const T pmw = sPM[o - 1], pnw = sPN[o - 1];
+                        onuc[k] = T(2) * sf::recip(pnw + pnc);
+                        omuc[k] = T(2) * sf::recip(pmw + pmc);
+                        if constexpr (!LEAN) cffuc[k] = (pmc + pmw) * (pnc + pnw);
+                        du = ((T(0.5) * ((h_w(k, o) + sZ1[o - 1]) + (h_c(k, o) + sZ1[o]))) * u1_c(k, o)) * onuc[k];
+                    }
+                    if constexpr (CPL) du1c[k] = du;
+                    if (j >= 1) {
+                        const T pms = sPM[o - FW], pns = sPN[o - FW];
+                        omvc[k] = T(2) * sf::recip(pms + pmc);
+                        onvc[k] = T(2) * sf::recip(pns + pnc);
+                        if constexpr (!LEAN) cffvc[k] = (pmc + pms) * (pnc + pns);
+                        dv = ((T(0.5) * ((h_s(k, o) + sZ1[o - FW]) + (h_c(k, o) + sZ1[o]))) * v1_c(k, o)) * omvc[k];
+                    }
+                    if constexpr (CPL) dv1c[k] = dv;
                 }
-                if constexpr (CPL) dv1c[k] = (double)dv;
+                sDU[o] = du;
+                sDV[o] = dv;
             }
-            sDU[o] = du;
-            sDV[o] = dv;
         }
         // ring fluxes
+        if constexpr (RINGS) {
 #pragma unroll
-        for (int s = 0; s < RS; s++) {
-            if (ro[s] < 0) continue;
-            const int o = ro[s];
-            T du = T(0), dv = T(0);
-            if (ri[s] >= 1) {
-                const T onu = T(2) * sf::recip(sPN[o - 1] + sPN[o]);
-                du = ((T(0.5) * ((rhw[s] + sZ1[o - 1]) + (rh[s] + sZ1[o]))) * sU1[o]) * onu;
+            for (int s = 0; s < RS; s++) {
+                if (rtid + s * RT >= RING) continue;
+                int a, b;
+                ring_point<TI, TJ, 2, 2>(rtid + s * RT, a, b);
+                flux(sZ1, sU1, sV1, fi0 + a, fj0 + b, b * FW + a, rh[s], rhw[s], rhs[s]);
             }
-            if (rj[s] >= 1) {
-                const T omv = T(2) * sf::recip(sPM[o - FW] + sPM[o]);
-                dv = ((T(0.5) * ((rhs[s] + sZ1[o - FW]) + (rh[s] + sZ1[o]))) * sV1[o]) * omv;
-            }
-            sDU[o] = du;
-            sDV[o] = dv;
         }
     }
-        // core: issue the predictor inputs (G1)
+    if constexpr (!XP) {
 #pragma unroll
-        for (int k = 0; k < KC; k++) {
-            int a, b;
-            core_ab(k, a, b);
-            const int i = fi0 + a, j = fj0 + b;
-            const uint32_t f = cf[k];
-            const bool ui = cin[k] && u_int(i, j), vi = cin[k] && v_int(i, j), ri_ = cin[k] && rho_int(i, j);
-            if (ri_ || ui || vi) {
-                if (!first) z0c_[k] = ldo(Pp->z0, 0, f);
-                fo_[k] = ldo(Pp->fomn, 0, f);
-            }
-            if (ui) {
-                if (!first) {
-                    z0w_[k] = ldo(Pp->z0, -1, f);
-                    u0c_[k] = ldo(Pp->u0, 0, f);
-                }
-                fow_[k] = ldo(Pp->fomn, -1, f);
-                su_[k] = ldo(Pp->sustr, 0, f);
-            }
-            if (vi) {
-                if (!first) {
-                    z0s_[k] = ldo(Pp->z0, -W, f);
-                    v0c_[k] = ldo(Pp->v0, 0, f);
-                }
-                fos_[k] = ldo(Pp->fomn, -W, f);
-                sv_[k] = ldo(Pp->svstr, 0, f);
-            }
-        }
+        for (int k = 0; k < KC; k++) issue_pred(k);
+    }
     lds_barrier();
 
     // ---- P1: predicted zeta and its right-hand side -----------------------------------
     {
         constexpr int RING = ring_size<TI, TJ, 2, 1>();
-        constexpr int RS = (RING + NT - 1) / NT;
+        constexpr int RS = (RING + RT - 1) / RT;
         T rz0[RS];
-        int ro[RS], rq[RS];
+        int ro[RS], ri[RS], rj[RS];
+        if constexpr (RINGS) {
 #pragma unroll
-        for (int s = 0; s < RS; s++) {
-            const int t = tid + s * NT;
-            ro[s] = -1;
-            rq[s] = 0;
-            if (t < RING) {
-                int a, b;
-                ring_point<TI, TJ, 2, 1>(t, a, b);
-                const int i = fi0 + a, j = fj0 + b;
-                ro[s] = b * FW + a;
-                if (inside(i, j)) {
-                    const int qi = clampi(i, 1, L - 1), qj = clampi(j, 1, M - 1);
-                    rq[s] = ro[s] + (qj - j) * FW + (qi - i);
-                    if (!first) rz0[s] = ldo(Pp->z0, 0, off(qi, qj));
-                } else {
-                    ro[s] = -2 - ro[s];   // outside: store zeros
+            for (int s = 0; s < RS; s++) {
+                const int t = rtid + s * RT;
+                ro[s] = -1;
+                ri[s] = rj[s] = -1;
+                if (t < RING) {
+                    int a, b;
+                    ring_point<TI, TJ, 2, 1>(t, a, b);
+                    const int i = fi0 + a, j = fj0 + b;
+                    ro[s] = b * FW + a;
+                    if (rho_int(i, j)) {
+                        ri[s] = i;
+                        rj[s] = j;
+                        if (!first) rz0[s] = XP ? sZ0[ro[s]] : ldo(Pp->z0, 0, off(i, j));
+                    } else if (inside(i, j)) {
+                        ro[s] = -1;           // a ghost: its source writes it
+                    } else {
+                        ro[s] = -2 - ro[s];   // outside: store zeros
+                    }
                 }
             }
         }
@@ -696,145 +914,138 @@ __device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*s
             if (first) return sZ1[qo] + (pmn * dt) * r;
             return z0 + (pmn * (T(2) * dt)) * r;
         };
+        if constexpr (CORE) {
 #pragma unroll
-        for (int k = 0; k < KC; k++) {
-            int a, b;
-            core_ab(k, a, b);
-            const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
-            T zs = T(0), r = T(0);
-            if (cin[k]) {
-                if (rho_int(i, j)) {
-                    zs = zs_of(o, pmnc[k], z0c_[k], r);
-                    sto<NTS>(Pp->rz1, cf[k], r);
+            for (int k = 0; k < KC; k++) {
+                int a, b;
+                core_ab(k, a, b);
+                const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
+                T zs = T(0), r = T(0);
+                if (cin[k]) {
+                    if (rho_int(i, j)) {
+                        if constexpr (XP) z0c_[k] = first ? T(0) : sZ0[o];
+                        const T pmn = LEAN ? sPM[o] * sPN[o] : pmnc[k];
+                        zs = zs_of(o, pmn, z0c_[k], r);
+                        sto<NTS>(Pp->rz1, cf[k], r);
+                        put_rho(sZS, o, i, j, zs);
+                    }
                 } else {
-                    const int qi = clampi(i, 1, L - 1), qj = clampi(j, 1, M - 1);
-                    const uint32_t fq = off(qi, qj);
-                    const int oq = o + (qj - j) * FW + (qi - i);
-                    const T pmn = sPM[oq] * sPN[oq];
-                    const T z0 = first ? T(0) : ldo(Pp->z0, 0, fq);
-                    zs = zs_of(oq, pmn, z0, r);
+                    sZS[o] = zs;
+                }
+                if constexpr (!LEAN) zsc[k] = zs;
+                rzc[k] = r;
+            }
+        }
+        if constexpr (RINGS) {
+#pragma unroll
+            for (int s = 0; s < RS; s++) {
+                if (ro[s] == -1) continue;
+                if (ro[s] < -1) {
+                    sZS[-2 - ro[s]] = T(0);
+                    continue;
+                }
+                T r;
+                const T zs = zs_of(ro[s], sPM[ro[s]] * sPN[ro[s]], rz0[s], r);
+                put_rho(sZS, ro[s], ri[s], rj[s], zs);
+                const int a = ri[s] - fi0, b = rj[s] - fj0;
+                if (b == 2) {   // the low row and column of C1's ring
+                    if (a >= 2 && a < 3 + TI) rzl[a - 2] = r;
+                } else if (a == 2 && b >= 3 && b < 3 + TJ) {
+                    rzl[TI + 1 + b - 3] = r;
                 }
             }
-            sZS[o] = zs;
-            sRZ[o] = r;
-            zsc[k] = zs;
-        }
-#pragma unroll
-        for (int s = 0; s < RS; s++) {
-            if (ro[s] == -1) continue;
-            if (ro[s] < -1) {
-                sZS[-2 - ro[s]] = T(0);
-                sRZ[-2 - ro[s]] = T(0);
-                continue;
-            }
-            T r;
-            const T zs = zs_of(rq[s], sPM[rq[s]] * sPN[rq[s]], rz0[s], r);
-            sZS[ro[s]] = zs;
-            sRZ[ro[s]] = r;
         }
     }
     lds_barrier();
 
     // ---- P2: predicted ubar / vbar --------------------------------------------------
-    {
+    if constexpr (CORE) {
 #pragma unroll
         for (int k = 0; k < KC; k++) {
             int a, b;
             core_ab(k, a, b);
             const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
-            T us = T(0), vs = T(0);
-            if (cin[k]) {
-                if (u_int(i, j)) {
-                    UVIn<T> x;
-                    x.m1 = onuc[k];
-                    x.m2 = omuc[k];
-                    x.cff = cffuc[k];
-                    x.hb = hw_[k];
-                    x.hc = hc_[k];
-                    x.xb = sU1[o - 1];
-                    x.xc = u1c[k];
-                    x.xf = sU1[o + 1];
-                    x.yf = sU1[o + FW];
-                    x.yb = sU1[o - FW];
-                    x.fc = fo_[k];
-                    x.fb = fow_[k];
-                    x.oc = v1c[k];
-                    x.of = sV1[o + FW];
-                    x.ob = sV1[o - 1];
-                    x.obf = sV1[o + FW - 1];
-                    x.st = su_[k];
-                    x.x0 = first ? u1c[k] : u0c_[k];
-                    x.z0c = z0c_[k];
-                    x.z0b = z0w_[k];
-                    T r;
-                    double F = 0.0;
-                    us = pred_u(o, x, r, offd(i, j), &F);
-                    sto<NTS>(Pp->ru1, cf[k], r);
-                    ruc[k] = r;
-                    if (j == 1) sRUlo[a - 3] = r;
-                    if (j == M - 1) sRUhi[a - 3] = r;
-                    if constexpr (CPL) {
-                        fuc[k] = F;
-                        if constexpr (FIRST) {
-                            sto<NTS>(Pp->c.Fu, offd(i, j), F);
-                            if (j == 1) sFUlo[a - 3] = F;
-                            if (j == M - 1) sFUhi[a - 3] = F;
-                        }
-                    }
-                } else if (i >= 2 && i <= L - 1) {   // ghost row: source (i, 1) or (i, M-1)
-                    const int qj = clampi(j, 1, M - 1);
-                    T r;
-                    UVIn<T> x = load_u(off(i, qj), o + (qj - j) * FW);
-                    metrics_u(x);
-                    us = pred_u(o + (qj - j) * FW, x, r, offd(i, qj));
-                }
-                if (v_int(i, j)) {
-                    UVIn<T> x;
-                    x.m1 = omvc[k];
-                    x.m2 = onvc[k];
-                    x.cff = cffvc[k];
-                    x.hb = hs_[k];
-                    x.hc = hc_[k];
-                    x.xb = sV1[o - FW];
-                    x.xc = v1c[k];
-                    x.xf = sV1[o + FW];
-                    x.yf = sV1[o + 1];
-                    x.yb = sV1[o - 1];
-                    x.fc = fo_[k];
-                    x.fb = fos_[k];
-                    x.oc = u1c[k];
-                    x.of = sU1[o + 1];
-                    x.ob = sU1[o - FW];
-                    x.obf = sU1[o + 1 - FW];
-                    x.st = sv_[k];
-                    x.x0 = first ? v1c[k] : v0c_[k];
-                    x.z0c = z0c_[k];
-                    x.z0b = z0s_[k];
-                    T r;
-                    double F = 0.0;
-                    vs = pred_v(o, x, r, offd(i, j), &F);
-                    sto<NTS>(Pp->rv1, cf[k], r);
-                    rvc[k] = r;
-                    if (i == 1) sRVlo[b - 3] = r;
-                    if (i == L - 1) sRVhi[b - 3] = r;
-                    if constexpr (CPL) {
-                        fvc[k] = F;
-                        if constexpr (FIRST) {
-                            sto<NTS>(Pp->c.Fv, offd(i, j), F);
-                            if (i == 1) sFVlo[b - 3] = F;
-                            if (i == L - 1) sFVhi[b - 3] = F;
-                        }
-                    }
-                } else if (j >= 2 && j <= M - 1) {   // ghost column: source (1, j) or (L-1, j)
-                    const int qi = clampi(i, 1, L - 1);
-                    T r;
-                    UVIn<T> x = load_v(off(qi, j), o + (qi - i));
-                    metrics_v(x);
-                    vs = pred_v(o + (qi - i), x, r, offd(qi, j));
-                }
+            if constexpr (XP) {
+                fo_[k] = sFO[o];
+                fow_[k] = sFO[o - 1];
+                fos_[k] = sFO[o - FW];
+                z0w_[k] = first ? T(0) : sZ0[o - 1];
+                z0s_[k] = first ? T(0) : sZ0[o - FW];
             }
-            sUS[o] = us;
-            sVS[o] = vs;
+            if (u_int(i, j)) {
+                UVIn<T> x;
+                x.m1 = onuc[k];
+                x.m2 = omuc[k];
+                x.cff = LEAN ? cff_u(o) : cffuc[k];
+                x.hb = h_w(k, o);
+                x.hc = h_c(k, o);
+                x.xb = sU1[o - 1];
+                x.xc = u1_c(k, o);
+                x.xf = sU1[o + 1];
+                x.yf = sU1[o + FW];
+                x.yb = sU1[o - FW];
+                x.fc = fo_[k];
+                x.fb = fow_[k];
+                x.oc = v1_c(k, o);
+                x.of = sV1[o + FW];
+                x.ob = sV1[o - 1];
+                x.obf = sV1[o + FW - 1];
+                x.st = su_[k];
+                x.x0 = first ? x.xc : u0c_[k];
+                x.z0c = z0c_[k];
+                x.z0b = z0w_[k];
+                T r;
+                double F = 0.0;
+                Forcing fq{};
+                if constexpr (CPL) fq = XP ? fqu[k] : load_forcing(false, offd(i, j));
+                const T us = pred_u(o, x, r, fq, F);
+                put_u(sUS, o, j, us);
+                sto<NTS>(Pp->ru1, cf[k], r);
+                ruc[k] = r;
+                if constexpr (CPL) {
+                    if constexpr (FIRST || !LEAN || XP) fuc[k] = T(F);
+                    if constexpr (FIRST) sto<NTS>(Pp->c.Fu, offd(i, j), F);
+                }
+            } else if (!cin[k] || u_wall(i)) {
+                sUS[o] = T(0);
+            }
+            if (v_int(i, j)) {
+                UVIn<T> x;
+                x.m1 = omvc[k];
+                x.m2 = onvc[k];
+                x.cff = LEAN ? cff_v(o) : cffvc[k];
+                x.hb = h_s(k, o);
+                x.hc = h_c(k, o);
+                x.xb = sV1[o - FW];
+                x.xc = v1_c(k, o);
+                x.xf = sV1[o + FW];
+                x.yf = sV1[o + 1];
+                x.yb = sV1[o - 1];
+                x.fc = fo_[k];
+                x.fb = fos_[k];
+                x.oc = u1_c(k, o);
+                x.of = sU1[o + 1];
+                x.ob = sU1[o - FW];
+                x.obf = sU1[o + 1 - FW];
+                x.st = sv_[k];
+                x.x0 = first ? x.xc : v0c_[k];
+                x.z0c = z0c_[k];
+                x.z0b = z0s_[k];
+                T r;
+                double F = 0.0;
+                Forcing fq{};
+                if constexpr (CPL) fq = XP ? fqv[k] : load_forcing(true, offd(i, j));
+                const T vs = pred_v(o, x, r, fq, F);
+                put_v(sVS, o, i, vs);
+                sto<NTS>(Pp->rv1, cf[k], r);
+                rvc[k] = r;
+                if constexpr (CPL) {
+                    if constexpr (FIRST || !LEAN || XP) fvc[k] = T(F);
+                    if constexpr (FIRST) sto<NTS>(Pp->c.Fv, offd(i, j), F);
+                }
+            } else if (!cin[k] || v_wall(j)) {
+                sVS[o] = T(0);
+            }
         }
         // core: issue the corrector inputs (G2)
 #pragma unroll
@@ -842,53 +1053,57 @@ __device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*s
             int a, b;
             core_ab(k, a, b);
             const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
-            const uint32_t f = cf[k];
-            if (cin[k] && rho_int(i, j)) {
-                const uint32_t fd = offd(i, j);
-                if (!first) rz0_[k] = ldo(Pp->rz0, 0, f);
-                zt_[k] = ldavg<NTS>(Pp->Zt, fd);
-                dua_[k] = ldavg<NTS>(Pp->DUa, fd);
-                dva_[k] = ldavg<NTS>(Pp->DVa, fd);
-                if constexpr (CPL) {
-                    du2_[k] = FIRST ? 0.0 : ldavg<NTS>(Pp->c.DU_avg2, fd);
-                    dv2_[k] = FIRST ? 0.0 : ldavg<NTS>(Pp->c.DV_avg2, fd);
-                }
-            }
-            if (cin[k] && u_int(i, j)) {
-                if (!first) ru0_[k] = ldo(Pp->ru0, 0, f);
-                z1w_[k] = sZ1[o - 1];   // the Z1 plane holds z1 until C1
-            }
-            if (cin[k] && v_int(i, j)) {
-                if (!first) rv0_[k] = ldo(Pp->rv0, 0, f);
-                z1s_[k] = sZ1[o - FW];
+            if constexpr (!XP && !LEAN) issue_corr(k, false);
+            if constexpr (!LEAN) {   // the Z1 plane holds z1 until C1
+                if (cin[k] && u_int(i, j)) z1w_[k] = sZ1[o - 1];
+                if (cin[k] && v_int(i, j)) z1s_[k] = sZ1[o - FW];
             }
         }
-        // ring: inputs loaded on demand
+    }
+    if constexpr (RINGS) {
         constexpr int RING = ring_size<TI, TJ, 1, 1>();
 #pragma unroll
-        for (int s = 0; s < (RING + NT - 1) / NT; s++) {
-            const int t = tid + s * NT;
+        for (int s = 0; s < RSP2; s++) {
+            const int t = rtid + s * RT;
             if (t >= RING) continue;
             int a, b;
             ring_point<TI, TJ, 1, 1>(t, a, b);
             const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
-            T us = T(0), vs = T(0), r;
-            if (inside(i, j)) {
-                if (i >= 2 && i <= L - 1) {
-                    const int qj = clampi(j, 1, M - 1);
-                    UVIn<T> x = load_u(off(i, qj), o + (qj - j) * FW);
-                    metrics_u(x);
-                    us = pred_u(o + (qj - j) * FW, x, r, offd(i, qj));
+            const bool in = inside(i, j);
+            T r;
+            double F;
+            if (u_int(i, j)) {
+                UVIn<T> x;
+                Forcing fq{};
+                if constexpr (XP) {
+                    x = xu[s];
+                    if constexpr (CPL) fq = xfu[s];
+                } else {
+                    load_u_global(x, off(i, j));
+                    if constexpr (CPL) fq = load_forcing(false, offd(i, j));
                 }
-                if (j >= 2 && j <= M - 1) {
-                    const int qi = clampi(i, 1, L - 1);
-                    UVIn<T> x = load_v(off(qi, j), o + (qi - i));
-                    metrics_v(x);
-                    vs = pred_v(o + (qi - i), x, r, offd(qi, j));
-                }
+                load_u_lds(x, o);
+                metrics_u(x);
+                put_u(sUS, o, j, pred_u(o, x, r, fq, F));
+            } else if (!in || u_wall(i)) {
+                sUS[o] = T(0);
             }
-            sUS[o] = us;
-            sVS[o] = vs;
+            if (v_int(i, j)) {
+                UVIn<T> x;
+                Forcing fq{};
+                if constexpr (XP) {
+                    x = xv[s];
+                    if constexpr (CPL) fq = xfv[s];
+                } else {
+                    load_v_global(x, off(i, j));
+                    if constexpr (CPL) fq = load_forcing(true, offd(i, j));
+                }
+                load_v_lds(x, o);
+                metrics_v(x);
+                put_v(sVS, o, i, pred_v(o, x, r, fq, F));
+            } else if (!in || v_wall(j)) {
+                sVS[o] = T(0);
+            }
         }
     }
     lds_barrier();
@@ -896,59 +1111,54 @@ __device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*s
     // ---- C0: fluxes DUs, DVs of the predicted state ------------------------------------
     {
         constexpr int RING = ring_size<TI, TJ, 1, 1>();
-        constexpr int RS = (RING + NT - 1) / NT;
-        T rh[RS], rhw[RS], rhs[RS];
-        int ro[RS], ri[RS], rj[RS];
+        if constexpr (!XP && !LEAN && CORE) {
 #pragma unroll
-        for (int s = 0; s < RS; s++) {
-            const int t = tid + s * NT;
-            ro[s] = -1;
-            ri[s] = rj[s] = -1;
-            if (t < RING) {
+            for (int k = 0; k < KC; k++) {
                 int a, b;
-                ring_point<TI, TJ, 1, 1>(t, a, b);
-                const int i = fi0 + a, j = fj0 + b;
-                ro[s] = b * FW + a;
-                if (inside(i, j)) {
-                    ri[s] = i;
-                    rj[s] = j;
-                    const uint32_t f = off(i, j);
-                    rh[s] = ldo(Pp->h, 0, f);
-                    if (i >= 1) rhw[s] = ldo(Pp->h, -1, f);
-                    if (j >= 1) rhs[s] = ldo(Pp->h, -W, f);
+                core_ab(k, a, b);
+                if (rho_int(fi0 + a, fj0 + b)) issue_avg(k, offd(fi0 + a, fj0 + b));
+            }
+        }
+        T rh[RSP2], rhw[RSP2], rhs[RSP2];
+        if constexpr (RINGS) {
+#pragma unroll
+            for (int s = 0; s < RSP2; s++) {
+                int a, b;
+                ring_point<TI, TJ, 1, 1>(rtid + s * RT, a, b);
+                if (rtid + s * RT < RING) load_h(fi0 + a, fj0 + b, rh[s], rhw[s], rhs[s]);
+            }
+        }
+        if constexpr (CORE) {
+#pragma unroll
+            for (int k = 0; k < KC; k++) {
+                int a, b;
+                core_ab(k, a, b);
+                const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
+                if constexpr (LEAN) {
+                    if constexpr (!XP) issue_corr(k, true);
+                    z1w_[k] = sZ1[o - 1];   // the Z1 plane holds z1 until C1
+                    z1s_[k] = sZ1[o - FW];
                 }
+                T du = T(0), dv = T(0);
+                if (cin[k]) {
+                    const T hc = h_c(k, o);
+                    if (i >= 1) du = ((T(0.5) * ((h_w(k, o) + sZS[o - 1]) + (hc + sZS[o]))) * sUS[o]) * onuc[k];
+                    if (j >= 1) dv = ((T(0.5) * ((h_s(k, o) + sZS[o - FW]) + (hc + sZS[o]))) * sVS[o]) * omvc[k];
+                }
+                sDU[o] = du;
+                sDV[o] = dv;
+                duc[k] = du;
+                dvc[k] = dv;
             }
         }
+        if constexpr (RINGS) {
 #pragma unroll
-        for (int k = 0; k < KC; k++) {
-            int a, b;
-            core_ab(k, a, b);
-            const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
-            T du = T(0), dv = T(0);
-            if (cin[k]) {
-                if (i >= 1) du = ((T(0.5) * ((hw_[k] + sZS[o - 1]) + (hc_[k] + sZS[o]))) * sUS[o]) * onuc[k];
-                if (j >= 1) dv = ((T(0.5) * ((hs_[k] + sZS[o - FW]) + (hc_[k] + sZS[o]))) * sVS[o]) * omvc[k];
+            for (int s = 0; s < RSP2; s++) {
+                if (rtid + s * RT >= RING) continue;
+                int a, b;
+                ring_point<TI, TJ, 1, 1>(rtid + s * RT, a, b);
+                flux(sZS, sUS, sVS, fi0 + a, fj0 + b, b * FW + a, rh[s], rhw[s], rhs[s]);
             }
-            sDU[o] = du;
-            sDV[o] = dv;
-            duc[k] = du;
-            dvc[k] = dv;
-        }
-#pragma unroll
-        for (int s = 0; s < RS; s++) {
-            if (ro[s] < 0) continue;
-            const int o = ro[s];
-            T du = T(0), dv = T(0);
-            if (ri[s] >= 1) {
-                const T onu = T(2) * sf::recip(sPN[o - 1] + sPN[o]);
-                du = ((T(0.5) * ((rhw[s] + sZS[o - 1]) + (rh[s] + sZS[o]))) * sUS[o]) * onu;
-            }
-            if (rj[s] >= 1) {
-                const T omv = T(2) * sf::recip(sPM[o - FW] + sPM[o]);
-                dv = ((T(0.5) * ((rhs[s] + sZS[o - FW]) + (rh[s] + sZS[o]))) * sVS[o]) * omv;
-            }
-            sDU[o] = du;
-            sDV[o] = dv;
         }
     }
     lds_barrier();
@@ -956,168 +1166,165 @@ __device__ __forceinline__ void phys_tile(const PFA<T> &P, int ti, int tj, T (*s
     // ---- C1: corrected zeta, time averages ------------------------------------------
     const T a1 = dt * T(5.0) / T(12.0), a2 = dt * T(8.0) / T(12.0), a3 = dt * T(1.0) / T(12.0);
     {
-        auto z2_of = [&](int qo, T pmn, T z1q, T rz0) {
+        auto z2_of = [&](int qo, T pmn, T z1q, T rz1, T rz0) {
             const T r = (sDU[qo] - sDU[qo + 1]) + (sDV[qo] - sDV[qo + FW]);
             if (first) return z1q + pmn * (dt * r);
-            return z1q + pmn * ((a1 * r + a2 * sRZ[qo]) - a3 * rz0);
+            return z1q + pmn * ((a1 * r + a2 * rz1) - a3 * rz0);
         };
         constexpr int RING = ring_size<TI, TJ, 1, 0>();
-        constexpr int RS = (RING + NT - 1) / NT;
-        T rz1[RS], rrz0[RS];
-        int ro[RS], rq[RS];
+        T rrz0[RSC1];
+        int ro[RSC1], ri[RSC1], rj[RSC1];
+        if constexpr (RINGS) {
 #pragma unroll
-        for (int s = 0; s < RS; s++) {
-            const int t = tid + s * NT;
-            ro[s] = -1;
-            rq[s] = 0;
-            if (t < RING) {
-                int a, b;
-                ring_point<TI, TJ, 1, 0>(t, a, b);
-                const int i = fi0 + a, j = fj0 + b;
-                ro[s] = b * FW + a;
-                if (inside(i, j)) {
-                    const int qi = clampi(i, 1, L - 1), qj = clampi(j, 1, M - 1);
-                    rq[s] = ro[s] + (qj - j) * FW + (qi - i);
-                    const uint32_t fq = off(qi, qj);
-                    rz1[s] = ldo(Pp->z1, 0, fq);
-                    if (!first) rrz0[s] = ldo(Pp->rz0, 0, fq);
-                } else {
-                    ro[s] = -2 - ro[s];
+            for (int s = 0; s < RSC1; s++) {
+                const int t = rtid + s * RT;
+                ro[s] = -1;
+                ri[s] = rj[s] = -1;
+                if (t < RING) {
+                    int a, b;
+                    ring_point<TI, TJ, 1, 0>(t, a, b);
+                    const int i = fi0 + a, j = fj0 + b;
+                    ro[s] = b * FW + a;
+                    if (rho_int(i, j)) {
+                        ri[s] = i;
+                        rj[s] = j;
+                        if (!first) rrz0[s] = XP ? xrz0[s] : ldo(Pp->rz0, 0, off(i, j));
+                    } else if (inside(i, j)) {
+                        ro[s] = -1;
+                    } else {
+                        ro[s] = -2 - ro[s];
+                    }
                 }
             }
         }
+        // Z2 reuses the Z1 plane: after the last barrier a point's z1 is read by its own
+        // thread only (a ghost's, which its source overwrites, by none)
+        if constexpr (CORE) {
 #pragma unroll
-        for (int k = 0; k < KC; k++) {
-            int a, b;
-            core_ab(k, a, b);
-            const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
-            T z2 = T(0);
-            if (cin[k]) {
+            for (int k = 0; k < KC; k++) {
+                int a, b;
+                core_ab(k, a, b);
+                const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
                 if (rho_int(i, j)) {
-                    z2 = z2_of(o, pmnc[k], z1c[k], rz0_[k]);
+                    const T z2 = z2_of(o, LEAN ? sPM[o] * sPN[o] : pmnc[k], z1c[k], rzc[k], rz0_[k]);
                     const double w = Pp->w1;
                     const uint32_t fd = offd(i, j);
-                    sto<NTS>(Pp->Zt, fd, zt_[k] + w * (double)zsc[k]);
+                    sto<NTS>(Pp->Zt, fd, zt_[k] + w * (double)(LEAN ? sZS[o] : zsc[k]));
                     sto<NTS>(Pp->DUa, fd, dua_[k] + w * (double)duc[k]);
                     sto<NTS>(Pp->DVa, fd, dva_[k] + w * (double)dvc[k]);
                     if constexpr (CPL) {
-                        sto<NTS>(Pp->c.DU_avg2, fd, (du2_[k] + Pp->c.w2p * du1c[k]) + Pp->c.w2c * (double)duc[k]);
-                        sto<NTS>(Pp->c.DV_avg2, fd, (dv2_[k] + Pp->c.w2p * dv1c[k]) + Pp->c.w2c * (double)dvc[k]);
+                        sto<NTS>(Pp->c.DU_avg2, fd, (du2_[k] + Pp->c.w2p * (double)du1c[k]) + Pp->c.w2c * (double)duc[k]);
+                        sto<NTS>(Pp->c.DV_avg2, fd, (dv2_[k] + Pp->c.w2p * (double)dv1c[k]) + Pp->c.w2c * (double)dvc[k]);
                     }
-                } else {
-                    const int qi = clampi(i, 1, L - 1), qj = clampi(j, 1, M - 1);
-                    const uint32_t fq = off(qi, qj);
-                    const int oq = o + (qj - j) * FW + (qi - i);
-                    const T pmn = sPM[oq] * sPN[oq];
-                    const T rz0 = first ? T(0) : ldo(Pp->rz0, 0, fq);
-                    z2 = z2_of(oq, pmn, ldo(Pp->z1, 0, fq), rz0);
+                    const int di = ghost_di(i), dj = ghost_dj(j);
+                    sto<NTS>(Pp->z2, cf[k], z2);
+                    if (di) sto<NTS>(Pp->z2, off(i + di, j), z2);
+                    if (dj) {
+                        sto<NTS>(Pp->z2, off(i, j + dj), z2);
+                        if (di) sto<NTS>(Pp->z2, off(i + di, j + dj), z2);
+                    }
+                    put_rho(sZ2, o, i, j, z2);
+                } else if (!cin[k]) {
+                    sZ2[o] = T(0);
                 }
-                sto<NTS>(Pp->z2, cf[k], z2);
             }
-            // Z2 reuses the Z1 plane: every reader of Z1 finished before the last barrier
-            sZ2[o] = z2;
         }
+        if constexpr (RINGS) {
 #pragma unroll
-        for (int s = 0; s < RS; s++) {
-            if (ro[s] == -1) continue;
-            if (ro[s] < -1) {
-                sZ2[-2 - ro[s]] = T(0);
-                continue;
+            for (int s = 0; s < RSC1; s++) {
+                if (ro[s] == -1) continue;
+                if (ro[s] < -1) {
+                    sZ2[-2 - ro[s]] = T(0);
+                    continue;
+                }
+                const int o = ro[s];
+                const T rz1 = rj[s] - fj0 == 2 ? rzl[ri[s] - fi0 - 2] : rzl[TI + 1 + rj[s] - fj0 - 3];
+                put_rho(sZ2, o, ri[s], rj[s], z2_of(o, sPM[o] * sPN[o], sZ1[o], rz1, rrz0[s]));
             }
-            sZ2[ro[s]] = z2_of(rq[s], sPM[rq[s]] * sPN[rq[s]], rz1[s], rrz0[s]);
         }
     }
     lds_barrier();
 
     // ---- C2: corrected ubar / vbar on the core -----------------------------------------
-    const T cf4 = T(2.0 / 5.0), cf5 = T(1) - cf4;
-    const T b1 = T(0.5) * dt * T(5.0) / T(12.0), b2 = T(0.5) * dt * T(8.0) / T(12.0),
-            b3 = T(0.5) * dt * T(1.0) / T(12.0);
-    auto gzc = [&](int o) { return cf5 * sZ2[o] + cf4 * sZS[o]; };
-    // corrected ubar at LDS index q: metrics m1 = onu, m2 = omu; statics hb/hc, fc/fb, st
-    auto corr_u = [&](int q, T onu, T omu, T cff, T hb, T hc, T fc, T fb, T st, T ru1, T ru0, T z1c_, T z1b,
-                      T u1c_, double F = 0.0) {
-        const T g0 = gzc(q - 1), g1 = gzc(q);
-        T r = ((T(0.5) * Pp->g) * onu) * ((hb + hc) * (g0 - g1) + (g0 * g0 - g1 * g1));
-        const T uc = sUS[q];
-        const T UFx1 = T(0.25) * (sDU[q] + sDU[q + 1]) * (uc + sUS[q + 1]);
-        const T UFx0 = T(0.25) * (sDU[q - 1] + sDU[q]) * (sUS[q - 1] + uc);
-        const T UFe1 = T(0.25) * (sDV[q + FW] + sDV[q + FW - 1]) * (sUS[q + FW] + uc);
-        const T UFe0 = T(0.25) * (sDV[q] + sDV[q - 1]) * (uc + sUS[q - FW]);
-        r = r - ((UFx1 - UFx0) + (UFe1 - UFe0));
-        const T cr1 = ((T(0.5) * (hc + sZS[q])) * fc) * (sVS[q] + sVS[q + FW]);
-        const T cr0 = ((T(0.5) * (hb + sZS[q - 1])) * fb) * (sVS[q - 1] + sVS[q - 1 + FW]);
-        r = r + T(0.5) * (cr1 + cr0);
-        r = r - ((Pp->rdrg * uc) * omu) * onu;
-        r = r + (st * omu) * onu;
-        if constexpr (CPL) r = r + T(F);
-        const T fac = sf::recip((hc + sZ2[q]) + (hb + sZ2[q - 1]));
-        T tend;
-        if (first) tend = (T(0.5) * dt) * r;
-        else tend = (b1 * r + b2 * ru1) - b3 * ru0;
-        return (u1c_ * ((hc + z1c_) + (hb + z1b)) + cff * tend) * fac;
-    };
-    auto corr_v = [&](int q, T omv, T onv, T cff, T hb, T hc, T fc, T fb, T st, T rv1, T rv0, T z1c_, T z1b,
-                      T v1c_, double F = 0.0) {
-        const T g0 = gzc(q - FW), g1 = gzc(q);
-        T r = ((T(0.5) * Pp->g) * omv) * ((hb + hc) * (g0 - g1) + (g0 * g0 - g1 * g1));
-        const T vc = sVS[q];
-        const T VFx1 = T(0.25) * (sDU[q + 1] + sDU[q + 1 - FW]) * (sVS[q + 1] + vc);
-        const T VFx0 = T(0.25) * (sDU[q] + sDU[q - FW]) * (vc + sVS[q - 1]);
-        const T VFe1 = T(0.25) * (sDV[q] + sDV[q + FW]) * (vc + sVS[q + FW]);
-        const T VFe0 = T(0.25) * (sDV[q - FW] + sDV[q]) * (sVS[q - FW] + vc);
-        r = r - ((VFx1 - VFx0) + (VFe1 - VFe0));
-        const T cr1 = ((T(0.5) * (hc + sZS[q])) * fc) * (sUS[q] + sUS[q + 1]);
-        const T cr0 = ((T(0.5) * (hb + sZS[q - FW])) * fb) * (sUS[q - FW] + sUS[q - FW + 1]);
-        r = r - T(0.5) * (cr1 + cr0);
-        r = r - ((Pp->rdrg * vc) * omv) * onv;
-        r = r + (st * omv) * onv;
-        if constexpr (CPL) r = r + T(F);
-        const T fac = sf::recip((hc + sZ2[q]) + (hb + sZ2[q - FW]));
-        T tend;
-        if (first) tend = (T(0.5) * dt) * r;
-        else tend = (b1 * r + b2 * rv1) - b3 * rv0;
-        return (v1c_ * ((hc + z1c_) + (hb + z1b)) + cff * tend) * fac;
-    };
+    if constexpr (CORE) {
+        const T cf4 = T(2.0 / 5.0), cf5 = T(1) - cf4;
+        const T b1 = T(0.5) * dt * T(5.0) / T(12.0), b2 = T(0.5) * dt * T(8.0) / T(12.0),
+                b3 = T(0.5) * dt * T(1.0) / T(12.0);
+        auto gzc = [&](int o) { return cf5 * sZ2[o] + cf4 * sZS[o]; };
+        // corrected ubar at LDS index q: metrics m1 = onu, m2 = omu; statics hb/hc, fc/fb, st
+        auto corr_u = [&](int q, T onu, T omu, T cff, T hb, T hc, T fc, T fb, T st, T ru1, T ru0, T z1c_, T z1b,
+                          T u1c_, T F) {
+            const T g0 = gzc(q - 1), g1 = gzc(q);
+            T r = ((T(0.5) * Pp->g) * onu) * ((hb + hc) * (g0 - g1) + (g0 * g0 - g1 * g1));
+            const T uc = sUS[q];
+            const T UFx1 = T(0.25) * (sDU[q] + sDU[q + 1]) * (uc + sUS[q + 1]);
+            const T UFx0 = T(0.25) * (sDU[q - 1] + sDU[q]) * (sUS[q - 1] + uc);
+            const T UFe1 = T(0.25) * (sDV[q + FW] + sDV[q + FW - 1]) * (sUS[q + FW] + uc);
+            const T UFe0 = T(0.25) * (sDV[q] + sDV[q - 1]) * (uc + sUS[q - FW]);
+            r = r - ((UFx1 - UFx0) + (UFe1 - UFe0));
+            const T cr1 = ((T(0.5) * (hc + sZS[q])) * fc) * (sVS[q] + sVS[q + FW]);
+            const T cr0 = ((T(0.5) * (hb + sZS[q - 1])) * fb) * (sVS[q - 1] + sVS[q - 1 + FW]);
+            r = r + T(0.5) * (cr1 + cr0);
+            r = r - ((Pp->rdrg * uc) * omu) * onu;
+            r = r + (st * omu) * onu;
+            if constexpr (CPL) r = r + F;
+            const T fac = sf::recip((hc + sZ2[q]) + (hb + sZ2[q - 1]));
+            T tend;
+            if (first) tend = (T(0.5) * dt) * r;
+            else tend = (b1 * r + b2 * ru1) - b3 * ru0;
+            return (u1c_ * ((hc + z1c_) + (hb + z1b)) + cff * tend) * fac;
+        };
+        auto corr_v = [&](int q, T omv, T onv, T cff, T hb, T hc, T fc, T fb, T st, T rv1, T rv0, T z1c_, T z1b,
+                          T v1c_, T F) {
+            const T g0 = gzc(q - FW), g1 = gzc(q);
+            T r = ((T(0.5) * Pp->g) * omv) * ((hb + hc) * (g0 - g1) + (g0 * g0 - g1 * g1));
+            const T vc = sVS[q];
+            const T VFx1 = T(0.25) * (sDU[q + 1] + sDU[q + 1 - FW]) * (sVS[q + 1] + vc);
+            const T VFx0 = T(0.25) * (sDU[q] + sDU[q - FW]) * (vc + sVS[q - 1]);
+            const T VFe1 = T(0.25) * (sDV[q] + sDV[q + FW]) * (vc + sVS[q + FW]);
+            const T VFe0 = T(0.25) * (sDV[q - FW] + sDV[q]) * (sVS[q - FW] + vc);
+            r = r - ((VFx1 - VFx0) + (VFe1 - VFe0));
+            const T cr1 = ((T(0.5) * (hc + sZS[q])) * fc) * (sUS[q] + sUS[q + 1]);
+            const T cr0 = ((T(0.5) * (hb + sZS[q - FW])) * fb) * (sUS[q - FW] + sUS[q - FW + 1]);
+            r = r - T(0.5) * (cr1 + cr0);
+            r = r - ((Pp->rdrg * vc) * omv) * onv;
+            r = r + (st * omv) * onv;
+            if constexpr (CPL) r = r + F;
+            const T fac = sf::recip((hc + sZ2[q]) + (hb + sZ2[q - FW]));
+            T tend;
+            if (first) tend = (T(0.5) * dt) * r;
+            else tend = (b1 * r + b2 * rv1) - b3 * rv0;
+            return (v1c_ * ((hc + z1c_) + (hb + z1b)) + cff * tend) * fac;
+        };
 #pragma unroll
-    for (int k = 0; k < KC; k++) {
-        int a, b;
-        core_ab(k, a, b);
-        const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
-        if (!cin[k]) continue;
-        T u2 = T(0), v2 = T(0);
-        if (u_int(i, j)) {
-            u2 = corr_u(o, onuc[k], omuc[k], cffuc[k], hw_[k], hc_[k], fo_[k], fow_[k], CLO ? csu[k] : su_[k], ruc[k],
-                        ru0_[k], z1c[k], z1w_[k], u1c[k], CPL ? fuc[k] : 0.0);
-        } else if (i >= 2 && i <= L - 1) {   // ghost row j = 0 or M: source row 1 or M-1
-            const int qj = clampi(j, 1, M - 1);
-            const uint32_t f = off(i, qj);
-            const T ru1 = qj == 1 ? sRUlo[a - 3] : sRUhi[a - 3];
-            const T ru0 = first ? T(0) : ldo(Pp->ru0, 0, f);
-            double F = 0.0;
-            if constexpr (CPL) F = FIRST ? (qj == 1 ? sFUlo[a - 3] : sFUhi[a - 3]) : ldo(Pp->c.Fu, 0, offd(i, qj));
-            const T st = CLO ? clS[(qj == 1 ? 0 : TI) + a - 3] : ldo(Pp->sustr, 0, f);
-            u2 = corr_u(o + (qj - j) * FW, onu_at(f), omu_at(f), cffu_at(f), ldo(Pp->h, -1, f), ldo(Pp->h, 0, f),
-                        ldo(Pp->fomn, 0, f), ldo(Pp->fomn, -1, f), st, ru1, ru0, ldo(Pp->z1, 0, f), ldo(Pp->z1, -1, f),
-                        sU1[o + (qj - j) * FW], F);
+        for (int k = 0; k < KC; k++) {
+            int a, b;
+            core_ab(k, a, b);
+            const int i = fi0 + a, j = fj0 + b, o = b * FW + a;
+            if (!cin[k]) continue;
+            if (u_int(i, j)) {
+                const T cff = LEAN ? cff_u(o) : cffuc[k];
+                const T u2 = corr_u(o, onuc[k], omuc[k], cff, h_w(k, o), h_c(k, o), fo_[k], fow_[k],
+                                    CLO ? csu[k] : su_[k], ruc[k], ru0_[k], z1c[k], z1w_[k], u1_c(k, o),
+                                    CPL ? fuc[k] : T(0));
+                sto<NTS>(Pp->u2, cf[k], u2);
+                const int dj = ghost_dj(j);
+                if (dj) sto<NTS>(Pp->u2, off(i, j + dj), u2);
+            } else if (u_wall(i)) {
+                sto<NTS>(Pp->u2, cf[k], T(0));
+            }
+            if (v_int(i, j)) {
+                const T cff = LEAN ? cff_v(o) : cffvc[k];
+                const T v2 = corr_v(o, omvc[k], onvc[k], cff, h_s(k, o), h_c(k, o), fo_[k], fos_[k],
+                                    CLO ? csv[k] : sv_[k], rvc[k], rv0_[k], z1c[k], z1s_[k], v1_c(k, o),
+                                    CPL ? fvc[k] : T(0));
+                sto<NTS>(Pp->v2, cf[k], v2);
+                const int di = ghost_di(i);
+                if (di) sto<NTS>(Pp->v2, off(i + di, j), v2);
+            } else if (v_wall(j)) {
+                sto<NTS>(Pp->v2, cf[k], T(0));
+            }
         }
-        sto<NTS>(Pp->u2, cf[k], u2);
-        if (v_int(i, j)) {
-            v2 = corr_v(o, omvc[k], onvc[k], cffvc[k], hs_[k], hc_[k], fo_[k], fos_[k], CLO ? csv[k] : sv_[k], rvc[k],
-                        rv0_[k], z1c[k], z1s_[k], v1c[k], CPL ? fvc[k] : 0.0);
-        } else if (j >= 2 && j <= M - 1) {   // ghost column i = 0 or L: source column 1 or L-1
-            const int qi = clampi(i, 1, L - 1);
-            const uint32_t f = off(qi, j);
-            const T rv1 = qi == 1 ? sRVlo[b - 3] : sRVhi[b - 3];
-            const T rv0 = first ? T(0) : ldo(Pp->rv0, 0, f);
-            double F = 0.0;
-            if constexpr (CPL) F = FIRST ? (qi == 1 ? sFVlo[b - 3] : sFVhi[b - 3]) : ldo(Pp->c.Fv, 0, offd(qi, j));
-            const T st = CLO ? clS[2 * TI + (qi == 1 ? 0 : TJ) + b - 3] : ldo(Pp->svstr, 0, f);
-            v2 = corr_v(o + (qi - i), omv_at(f), onv_at(f), cffv_at(f), ldo(Pp->h, -W, f), ldo(Pp->h, 0, f),
-                        ldo(Pp->fomn, 0, f), ldo(Pp->fomn, -W, f), st, rv1, rv0, ldo(Pp->z1, 0, f), ldo(Pp->z1, -W, f),
-                        sV1[o + (qi - i)], F);
-        }
-        sto<NTS>(Pp->v2, cf[k], v2);
     }
 }
 
@@ -1130,26 +1337,34 @@ __device__ __forceinline__ int xcd_band(int nblk)
     return b;
 }
 
-template <typename T, int TI, int TJ, int NT, bool FIRST, bool NTS, bool CPL = false, bool CLO = false>
-__global__ __launch_bounds__(NT) void k_phys_fused(PFA<T> P)
+template <typename T, int TI, int TJ, int NT, int NR, bool FIRST, bool NTS, bool CPL = false, bool CLO = false>
+__global__ __launch_bounds__(NT + NR) void k_phys_fused(PFA<T> P)
 {
-    __shared__ T sm[PhysLds<TI, TJ>::PLANES][PhysLds<TI, TJ>::FN];
-    __shared__ T side[2 * TI + 2 * TJ];
-    __shared__ double sideF[CPL ? 2 * TI + 2 * TJ : 1];
-    constexpr bool IN_FRAME = cl_tiles_in_frame<T, CLO>;
-    static_assert(!IN_FRAME || 6 * PhysLds<TI, TJ>::FN * sizeof(T) >= (NT / 64) * 64 * XS * sizeof(uint32_t),
+    constexpr bool IN_FRAME = cl_tiles_in_frame<T, CLO, TI>;
+    using Lds = PhysLds<T, TI, TJ, NT, NR, NTS, CPL, CLO>;
+    __shared__ T sm[Lds::PLANES][Lds::FN];
+    __shared__ T rzl[TI + TJ + 1];
+    static_assert(!IN_FRAME || 6 * Lds::FN * sizeof(T) >= (NT / 64) * 64 * XS * sizeof(uint32_t),
                   "frame planes 1..6 hold the feature tiles");
     __shared__ __attribute__((aligned(16))) uint32_t clX[CLO && !IN_FRAME ? (NT / 64) * 64 * XS : 1];
     __shared__ float clN[CLO ? 2 * NIN : 1];
-    __shared__ T clS[CLO ? 2 * TI + 2 * TJ : 1];
-    __shared__ T clH[CLO ? PhysLds<TI, TJ>::FN : 1], clF[CLO ? PhysLds<TI, TJ>::FN : 1];   // h, f over the frame
-    const int b = xcd_band(P.tiles_i * P.tiles_j);
-    phys_tile<T, TI, TJ, NT, FIRST, NTS, CPL, CLO>(P, b % P.tiles_i, b / P.tiles_i, sm, side, sideF,
-                                                   IN_FRAME ? (uint32_t *)sm[1] : clX, clN, clS, clH, clF);
+    __shared__ T clF[CLO ? Lds::FN : 1];   // f over the frame
+    const int b = xcd_band(P.tiles_i * P.tiles_j), ti = b % P.tiles_i, tj = b / P.tiles_i;
+    uint32_t *X = IN_FRAME ? (uint32_t *)sm[1] : clX;
+    if constexpr (NR == 0) {
+        phys_tile<T, TI, TJ, NT, NR, ROLE_ALL, FIRST, NTS, CPL, CLO>(P, ti, tj, sm, rzl, X, clN, clF);
+    } else {
+        // whole waves of one role each: the branch is on a scalar, and both sides meet the
+        // same number of barriers
+        if (__builtin_amdgcn_readfirstlane((int)threadIdx.x) < NT)
+            phys_tile<T, TI, TJ, NT, NR, ROLE_CORE, FIRST, NTS, CPL, CLO>(P, ti, tj, sm, rzl, X, clN, clF);
+        else
+            phys_tile<T, TI, TJ, NT, NR, ROLE_RING, FIRST, NTS, CPL, CLO>(P, ti, tj, sm, rzl, X, clN, clF);
+    }
 }
 
 
-template <typename T, int TI, int TJ, int NT>
+template <typename T, int TI, int TJ, int NT, int NR = 0>
 int launch_fused(const sf_phys_fields *x, double dt, int first, double w1, void *stream,
                  const sf_couple_fields *cp = nullptr, const ClosureIn *cl = nullptr)
 {
@@ -1200,44 +1415,72 @@ int launch_fused(const sf_phys_fields *x, double dt, int first, double w1, void 
                x->szI, x->szJ);
     const long long nb = (long long)a.tiles_i * a.tiles_j;
     SF_REQUIRE(nb < (1LL << 31), "sf_phys_substep_fused: grid too large");
-    const dim3 grid((unsigned)nb), block(NT);
+    const dim3 grid((unsigned)nb), block(NT + NR);
     hipStream_t s = sf::as_stream(stream);
-    if constexpr (TJ <= 8) {
-        if (cl) {
-            SF_REQUIRE(!cp, "sf_phys_substep_closure_fused: coupling and closure together are not supported");
-            if (first && a.nts) hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, true, true, false, true>), grid, block, 0, s, a);
-            else if (first) hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, true, false, false, true>), grid, block, 0, s, a);
-            else if (a.nts) hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, false, true, false, true>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, false, false, false, true>), grid, block, 0, s, a);
-            return sf::check_launch("sf_phys_substep_closure_fused");
-        }
-        if (cp) {
-            if (first && a.nts) hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, true, true, true>), grid, block, 0, s, a);
-            else if (first) hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, true, false, true>), grid, block, 0, s, a);
-            else if (a.nts) hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, false, true, true>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, false, false, true>), grid, block, 0, s, a);
-            return sf::check_launch("sf_phys_substep_coupled_fused");
-        }
+    // one launch of the instance <FIRST, streaming>; split tiles run on small grids only and
+    // never stream
+    auto launch = [&](auto cpl, auto clo, const char *name) {
+        constexpr bool CPL = decltype(cpl)::value, CLO = decltype(clo)::value, S = NR == 0;
+        if (first && S && a.nts) hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, NR, true, S, CPL, CLO>), grid, block, 0, s, a);
+        else if (first) hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, NR, true, false, CPL, CLO>), grid, block, 0, s, a);
+        else if (S && a.nts) hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, NR, false, S, CPL, CLO>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, NR, false, false, CPL, CLO>), grid, block, 0, s, a);
+        return sf::check_launch(name);
+    };
+    using Yes = std::true_type;
+    using No = std::false_type;
+    if (cl) {
+        SF_REQUIRE(!cp, "sf_phys_substep_closure_fused: coupling and closure together are not supported");
+        if constexpr (NT == 256) return launch(No{}, Yes{}, "sf_phys_substep_closure_fused");
+    } else if (cp) {
+        if constexpr (NT <= 256) return launch(Yes{}, No{}, "sf_phys_substep_coupled_fused");
+    } else {
+        if constexpr (NT == 512 || TJ == 4 || NR > 0) return launch(No{}, No{}, "sf_phys_substep_fused");
     }
-    if (cp || cl) {
-        sf::set_error("%s: tile height %d (4 or 8)",
-                      cp ? "sf_phys_substep_coupled_fused" : "sf_phys_substep_closure_fused", TJ);
-        return SF_ERR_ARG;
-    }
-    if (first && a.nts) hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, true, true>), grid, block, 0, s, a);
-    else if (first) hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, true, false>), grid, block, 0, s, a);
-    else if (a.nts) hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, false, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((k_phys_fused<T, TI, TJ, NT, false, false>), grid, block, 0, s, a);
-    return sf::check_launch("sf_phys_substep_fused");
+    sf::set_error("%s: tile height %d (4 or 8)",
+                  cp ? "sf_phys_substep_coupled_fused" : "sf_phys_substep_closure_fused", TJ);
+    return SF_ERR_ARG;
 }
 
+// Tile height tj: 4, 8 or 16 (64-wide tiles), or 0 for the tile that measured fastest on the
+// grid's size (microseconds per substep, graph replays, at the sizes named):
+//  - grids of at most one 16 x 8 tile per CU: core and ring on different waves, all loads at
+//    the start of the tile (128 x 64: FP64 6.4 against 9.1 with 64 x 4 tiles, FP32 5.6 / 7.7);
+//  - up to two 32 x 8 tiles per CU: the same form with 32 x 8 tiles (512 x 256: FP64 11.6
+//    against 12.5, FP32 8.1 / 9.1; 640 x 320 has 800 such tiles and loses, 18.9 / 16.8 and
+//    12.4 / 10.4).  Coupled FP64 instances gain up to 1024 64 x 8 tiles (768 x 384: 26.1
+//    against 28.1; 1024 x 512: 39.6 / 36.4).  The closure needs the registers of a whole CU:
+//    one tile per CU (343 x 129: 11.0 / 12.6; 512 x 256: 18.4 / 14.5);
+//  - FP64 grids whose 64 x 4 tiles all fit at once (three per CU; 513 x 255: 14.3 against 16.5);
+//  - else 64 x 8 tiles; coupled FP32 64 x 4 below four 64 x 8 tiles per CU (768 x 384: 15.5
+//    against 16.8), the closure 64 x 4 (its 64 x 8 instances exceed two waves per SIMD).
 template <typename T>
 int dispatch_tj(const sf_phys_fields *x, double dt, int first, double w1, int tj, void *stream,
                 const sf_couple_fields *cp = nullptr, const ClosureIn *cl = nullptr)
 {
+    constexpr long long CU = 256;
+    constexpr bool F64 = sizeof(T) == 8;
+    if (tj == 0) {
+        auto tiles = [&](int TI, int TJ) {
+            const int oi = x->szI % TI == 1 ? 1 : 0, oj = x->szJ % TJ == 1 ? 1 : 0;
+            return (long long)((x->szI + oi + TI - 1) / TI) * ((x->szJ + oj + TJ - 1) / TJ);
+        };
+        const bool few8 = tiles(64, 8) < 4 * CU;
+        const long long t32 = tiles(32, 8);
+        if (!cl && tiles(16, 8) <= CU) return launch_fused<T, 16, 8, 128, 192>(x, dt, first, w1, stream, cp);
+        if (cl ? t32 <= CU : (cp && F64 ? few8 : t32 <= 2 * CU + 64))
+            return launch_fused<T, 32, 8, 256, 256>(x, dt, first, w1, stream, cp, cl);
+        if (cl) tj = 4;
+        else if (cp) tj = few8 ? 4 : 8;
+        else tj = F64 && tiles(64, 4) <= 3 * CU ? 4 : 8;
+    }
     switch (tj) {
     case 4: return launch_fused<T, 64, 4, 256>(x, dt, first, w1, stream, cp, cl);
-    case 8: return launch_fused<T, 64, 8, 256>(x, dt, first, w1, stream, cp, cl);
+    case 8:
+        // 512 threads: one core point per thread; the coupled and closure instances need too
+        // many registers for that
+        if (cp || cl) return launch_fused<T, 64, 8, 256>(x, dt, first, w1, stream, cp, cl);
+        return launch_fused<T, 64, 8, 512>(x, dt, first, w1, stream);
     case 16: return launch_fused<T, 64, 16, 512>(x, dt, first, w1, stream, cp, cl);
     default: break;
     }
@@ -1262,8 +1505,9 @@ __global__ __launch_bounds__(NT) void k_phys_ensemble(const PFA<T> *__restrict__
                                                       const int2 *__restrict__ list, int ntiles, int order,
                                                       int rot, double w1)
 {
-    __shared__ T sm[PhysLds<TI, TJ>::PLANES][PhysLds<TI, TJ>::FN];
-    __shared__ T side[2 * TI + 2 * TJ];
+    using Lds = PhysLds<T, TI, TJ, NT, 0, NTS, false, false>;
+    __shared__ T sm[Lds::PLANES][Lds::FN];
+    __shared__ T rzl[TI + TJ + 1];
     const int G = gridDim.x;
     int t0, t1, step;
     if (order == 0) {
@@ -1291,7 +1535,7 @@ __global__ __launch_bounds__(NT) void k_phys_ensemble(const PFA<T> *__restrict__
             for (int w = 0; w < (int)(sizeof(PFA<T>) / 4); w++) dst[w] = src[w];
         }
         P.w1 = w1;
-        phys_tile<T, TI, TJ, NT, FIRST, NTS>(P, ey % P.tiles_i, ey / P.tiles_i, sm, side);
+        phys_tile<T, TI, TJ, NT, 0, ROLE_ALL, FIRST, NTS>(P, ey % P.tiles_i, ey / P.tiles_i, sm, rzl);
         lds_barrier();   // the next tile overwrites the LDS planes
     }
 }
@@ -1304,8 +1548,9 @@ __global__ __launch_bounds__(NT) void k_phys_ensemble1(const PFA<T> *__restrict_
                                                        const int2 *__restrict__ list, int order, int rot,
                                                        double w1)
 {
-    __shared__ T sm[PhysLds<TI, TJ>::PLANES][PhysLds<TI, TJ>::FN];
-    __shared__ T side[2 * TI + 2 * TJ];
+    using Lds = PhysLds<T, TI, TJ, NT, 0, NTS, false, false>;
+    __shared__ T sm[Lds::PLANES][Lds::FN];
+    __shared__ T rzl[TI + TJ + 1];
     const int t = order == 0 ? (int)blockIdx.x : xcd_band(gridDim.x);
     const SF_CONST int *clist = (const SF_CONST int *)list;
     const SF_CONST PFA<T> *cmem = (const SF_CONST PFA<T> *)members;
@@ -1318,7 +1563,7 @@ __global__ __launch_bounds__(NT) void k_phys_ensemble1(const PFA<T> *__restrict_
         for (int w = 0; w < (int)(sizeof(PFA<T>) / 4); w++) dst[w] = src[w];
     }
     P.w1 = w1;
-    phys_tile<T, TI, TJ, NT, FIRST, NTS>(P, ey % P.tiles_i, ey / P.tiles_i, sm, side);
+    phys_tile<T, TI, TJ, NT, 0, ROLE_ALL, FIRST, NTS>(P, ey % P.tiles_i, ey / P.tiles_i, sm, rzl);
 }
 }  // namespace
 
@@ -1430,7 +1675,7 @@ int ens_build(sf_ens *e)
 template <typename T, int TJ>
 void ens_launch_tj(sf_ens *e, int first, double w1, int rot, hipStream_t s)
 {
-    constexpr int TI = 64, NT = TJ == 16 ? 512 : 256;
+    constexpr int TI = 64, NT = TJ == 4 ? 256 : 512;
     const int G = e->grid > 0 ? (e->grid < e->ntiles ? e->grid : e->ntiles) : e->ntiles;
     const PFA<T> *m = (const PFA<T> *)e->members;
     if (G == e->ntiles) {   // one workgroup per tile
