@@ -266,6 +266,13 @@ int sf_step2d_substep_parts(sf_ctx *ctx, const sf_step2d_fields *fields, int32_t
                             double dtfast, double cff1, double clamp_val, int32_t flags,
                             int32_t parts, void *stream);
 
+/* nsub substeps in one call: the time slots of a copy of `fields` (the state before the
+ * first) are rotated t0 <- t1 <- t2 <- t0 before each, substep n takes cff1[n] and
+ * clamp_val[n].  *done = substeps issued; an error ends the loop. */
+int sf_step2d_run(sf_ctx *ctx, const sf_step2d_fields *fields, int32_t precision, double dtfast,
+                  const double *cff1, const double *clamp_val, int32_t flags, int32_t nsub, void *stream,
+                  int32_t *done);
+
 /* Tile shape (xi, eta) of the fused substep kernel. */
 int sf_step2d_tile_shape(int32_t *ti, int32_t *tj);
 
@@ -431,6 +438,16 @@ typedef struct sf_open_bc {
  * sf_obc_volcons_work_size doubles; volcons_out: area, flux, ubar_xs of the last). */
 int sf_phys_substep_open(const sf_phys_fields *fields, const sf_open_bc *obc, int32_t precision, double dt,
                          int32_t first, double cff1, double *volcons_work, double *volcons_out, void *stream);
+
+/* nsub physics substeps in one call: the time slots of a copy of `fields` (the state
+ * before the first) are rotated t0 <- t1 <- t2 <- t0 before each; substep n takes w1[n],
+ * the first one `first`.  cpl: the coupled form with the flux weights w2p[n], w2c[n]; obc:
+ * the open form; neither: the closed basin.  fused: one launch per substep (the open form
+ * has none).  *done = substeps issued; an error ends the loop. */
+int sf_phys_run(const sf_phys_fields *fields, const sf_couple_fields *cpl, const double *w2p, const double *w2c,
+                const sf_open_bc *obc, double *volcons_work, double *volcons_out, int32_t precision, double dt,
+                int32_t first, const double *w1, int32_t nsub, int32_t fused, int32_t tile_j, void *stream,
+                int32_t *done);
 
 /* ---------------- ensembles of physics-mode basins ---------------------------------- */
 

@@ -214,3 +214,47 @@ extern "C" int sf_ens_replay(sf_ens *e, void *stream)
     // nsub is a multiple of 3: the rotation is unchanged
     return SF_OK;
 }
+
+// nsub substeps issued by one call: the slots are rotated before each (x: the state before
+// the first), so a host loop in another language pays for one call instead of nsub.
+extern "C" int sf_phys_run(const sf_phys_fields *x, const sf_couple_fields *cp, const double *w2p,
+                           const double *w2c, const sf_open_bc *ob, double *work, double *out, int32_t precision,
+                           double dt, int32_t first, const double *w1, int32_t nsub, int32_t fused,
+                           int32_t tile_j, void *stream, int32_t *done)
+{
+    SF_REQUIRE(x && w1 && done && nsub >= 0, "sf_phys_run: bad arguments");
+    SF_REQUIRE(!(cp && ob), "sf_phys_run: coupling and open edges together are not supported");
+    SF_REQUIRE(!cp || (w2p && w2c), "sf_phys_run: coupling without its flux weights");
+    sf_phys_fields a = *x;
+    sf_couple_fields c = cp ? *cp : sf_couple_fields{};
+    *done = 0;
+    for (int32_t n = 0; n < nsub; n++, (*done)++) {
+        auto rotate = [](auto &s) {
+            auto *t0 = s[0];
+            s[0] = s[1];
+            s[1] = s[2];
+            s[2] = t0;
+        };
+        rotate(a.zeta);
+        rotate(a.ubar);
+        rotate(a.vbar);
+        rotate(a.rzeta);
+        rotate(a.rubar);
+        rotate(a.rvbar);
+        const int32_t f = first && n == 0;
+        int rc;
+        if (cp) {
+            c.w2p = w2p[n];
+            c.w2c = w2c[n];
+            rc = fused ? sf_phys_substep_coupled_fused(&a, &c, precision, dt, f, w1[n], tile_j, stream)
+                       : sf_phys_substep_coupled(&a, &c, precision, dt, f, w1[n], stream);
+        } else if (ob) {
+            rc = sf_phys_substep_open(&a, ob, precision, dt, f, w1[n], work, out, stream);
+        } else {
+            rc = fused ? sf_phys_substep_fused(&a, precision, dt, f, w1[n], tile_j, stream)
+                       : sf_phys_substep(&a, precision, dt, f, w1[n], stream);
+        }
+        if (rc != SF_OK) return rc;
+    }
+    return SF_OK;
+}

@@ -733,6 +733,34 @@ extern "C" int sf_step2d_substep(sf_ctx *c, const sf_step2d_fields *a, int32_t p
     return sf_step2d_substep_parts(c, a, precision, dtfast, cff1, clamp_val, flags, 3, stream);
 }
 
+// nsub substeps issued by one call, the slots rotated before each (a: the state before the
+// first)
+extern "C" int sf_step2d_run(sf_ctx *c, const sf_step2d_fields *x, int32_t precision, double dtfast,
+                             const double *cff1, const double *clamp_val, int32_t flags, int32_t nsub,
+                             void *stream, int32_t *done)
+{
+    SF_REQUIRE(x && cff1 && clamp_val && done && nsub >= 0, "sf_step2d_run: bad arguments");
+    sf_step2d_fields a = *x;
+    *done = 0;
+    for (int32_t n = 0; n < nsub; n++, (*done)++) {
+        auto rotate = [](auto &s) {
+            auto *t0 = s[0];
+            s[0] = s[1];
+            s[1] = s[2];
+            s[2] = t0;
+        };
+        rotate(a.zeta);
+        rotate(a.ubar);
+        rotate(a.vbar);
+        rotate(a.rzeta);
+        rotate(a.rubar);
+        rotate(a.rvbar);
+        const int rc = sf_step2d_substep(c, &a, precision, dtfast, cff1[n], clamp_val[n], flags, stream);
+        if (rc != SF_OK) return rc;
+    }
+    return SF_OK;
+}
+
 extern "C" int sf_step2d_tile_shape(int32_t *ti, int32_t *tj)
 {
     SF_REQUIRE(ti && tj, "sf_step2d_tile_shape: null argument");

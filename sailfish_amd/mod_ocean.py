@@ -16,6 +16,7 @@ import torch
 
 _ROT2D = ("zeta", "ubar", "vbar", "rzeta", "rubar", "rvbar")
 _ROT3D = ("u", "v", "ru", "rv")
+_VIEWS2D = tuple(tuple(f"{n}_t{k}" for k in range(3)) for n in _ROT2D)
 
 
 class T_OCEAN:
@@ -65,8 +66,9 @@ class T_OCEAN:
 
     def cycleTimes2D(self):
         """mod_ocean.py:120-155"""
-        for name in _ROT2D:
-            self._rotate(self, name)
+        d = self.__dict__
+        for t0, t1, t2 in _VIEWS2D:
+            d[t0], d[t1], d[t2] = d[t1], d[t2], d[t0]
 
     def cycleTimes3D(self):
         """mod_ocean.py:157-191"""

@@ -5,12 +5,14 @@ four gfx950 launches (sf_phys_substep) or one fused launch (sf_phys_substep_fuse
 from __future__ import annotations
 
 import ctypes as C
+import struct
 
 import numpy as np
 import torch
 
 from . import _lib
 from .mod_constants import g as G_CONST
+from .mod_ocean import T_OCEAN, _VIEWS2D
 
 P = C.c_void_p
 
@@ -24,6 +26,14 @@ class sf_phys_fields(C.Structure):
         ("scratch", P * 4),
         ("Zt_avg1", P), ("DU_avg1", P), ("DV_avg1", P),
     ]
+
+
+# the same layout in one pack call: building the ctypes arrays field by field takes longer
+# than a small grid's substep
+_FIELDS_PACK = struct.Struct("=iidd31Q")
+assert _FIELDS_PACK.size == C.sizeof(sf_phys_fields)
+_STATIC = ("h", "pm", "pn", "fomn", "sustr", "svstr")
+_VIEWS = tuple(v for views in _VIEWS2D for v in views)
 
 
 class sf_open_bc(C.Structure):
@@ -40,6 +50,9 @@ def _bind():
     lib.sf_phys_substep_fused.argtypes = [C.POINTER(sf_phys_fields), C.c_int32, C.c_double, C.c_int32, C.c_double,
                                           C.c_int32, P]
     lib.sf_phys_substep_fused.restype = C.c_int32
+    lib.sf_phys_run.argtypes = [C.POINTER(sf_phys_fields), P, P, P, P, P, P, C.c_int32, C.c_double, C.c_int32, P,
+                                C.c_int32, C.c_int32, C.c_int32, P, C.POINTER(C.c_int32)]
+    lib.sf_phys_run.restype = C.c_int32
     lib.sf_phys_fused_default_tile.argtypes = [C.c_int32, C.c_int32, C.c_int32]
     lib.sf_phys_fused_default_tile.restype = C.c_int32
     return lib
@@ -97,19 +110,12 @@ class PhysStepper:
             self.vc_out = torch.zeros(3, dtype=torch.float64, device=dev)
 
     def fields(self, OCEAN) -> sf_phys_fields:
-        a = sf_phys_fields()
-        a.szI, a.szJ, a.g, a.rdrg = self.szI, self.szJ, self.g, self.rdrg
         s = self.static
-        a.h, a.pm, a.pn, a.fomn, a.sustr, a.svstr = (s[k].data_ptr() for k in
-                                                     ("h", "pm", "pn", "fomn", "sustr", "svstr"))
-        for name in ("zeta", "ubar", "vbar", "rzeta", "rubar", "rvbar"):
-            arr = getattr(a, name)
-            for k in range(3):
-                arr[k] = getattr(OCEAN, f"{name}_t{k}").data_ptr()
-        for k, buf in enumerate(self.scratch):
-            a.scratch[k] = buf.data_ptr()
-        a.Zt_avg1, a.DU_avg1, a.DV_avg1 = OCEAN.Zt_avg1.data_ptr(), OCEAN.DU_avg1.data_ptr(), OCEAN.DV_avg1.data_ptr()
-        return a
+        scr = [b.data_ptr() for b in self.scratch] or (0, 0, 0, 0)
+        return sf_phys_fields.from_buffer_copy(_FIELDS_PACK.pack(
+            self.szI, self.szJ, self.g, self.rdrg, *[s[k].data_ptr() for k in _STATIC],
+            *[getattr(OCEAN, v).data_ptr() for v in _VIEWS], *scr, OCEAN.Zt_avg1.data_ptr(),
+            OCEAN.DU_avg1.data_ptr(), OCEAN.DV_avg1.data_ptr()))
 
     def step(self, compTimes, OCEAN, first: bool, stream=None):
         a = self.fields(OCEAN)
@@ -131,11 +137,43 @@ class PhysStepper:
         _lib.check(rc, "sf_phys_substep")
 
 
+def issue_substeps(compTimes, OCEAN, nsub: int, what: str, issue, clamp=None):
+    """``nsub`` substeps through one native call: advances the 2D time counter, collects
+    each substep's averaging weight (and ``clamp(time2D)``), calls
+    ``issue(nsub, weights, clamps, done)`` and rotates the host's views as the substeps did.
+    If a substep fails, counter and views stop there, as a loop of single substeps would."""
+    w = (C.c_double * max(nsub, 1))()
+    cl = (C.c_double * max(nsub, 1))() if clamp is not None else None
+    times = []
+    for n in range(nsub):
+        compTimes.next2DTimeStep()
+        w[n] = compTimes.cff1()
+        if cl is not None:
+            cl[n] = clamp(compTimes.time2D)
+        times.append({k: getattr(compTimes, k) for k in ("iif", "time2D") if hasattr(compTimes, k)})
+    done = C.c_int32(0)
+    rc = issue(nsub, w, cl, done)
+    n = nsub if rc == _lib.SF_OK else min(done.value + 1, nsub)
+    if 0 < n < nsub:
+        for k, v in times[n - 1].items():
+            setattr(compTimes, k, v)
+    for _ in range(n % 3):
+        OCEAN.cycleTimes2D()
+    _lib.check(rc, what)
+
+
 def run_phys(compTimes, GRID, OCEAN, nsteps: int, stepper: PhysStepper | None = None, start_first: bool = True):
     """``nsteps`` physics substeps (next2DTimeStep, cycleTimes2D, substep); the
     first substep of the run is forward/backward Euler."""
     st = stepper or PhysStepper(GRID, OCEAN)
-    for n in range(int(nsteps)):
+    if type(st).step is PhysStepper.step and type(OCEAN).cycleTimes2D is T_OCEAN.cycleTimes2D:
+        a = st.fields(OCEAN)
+        ob = (C.addressof(st.open_bc), st.vc_work.data_ptr(), st.vc_out.data_ptr()) if st.open_edges else (None,) * 3
+        issue_substeps(compTimes, OCEAN, int(nsteps), "sf_phys_run", lambda n, w1, _clamp, done: st.lib.sf_phys_run(
+            C.byref(a), None, None, None, *ob, st.precision, float(compTimes.dtfast), int(bool(start_first)), w1, n,
+            int(st.fused), st.tile_j, _lib.stream_handle(), C.byref(done)))
+        return st
+    for n in range(int(nsteps)):     # a caller's own step or state class
         compTimes.next2DTimeStep()
         OCEAN.cycleTimes2D()
         st.step(compTimes, OCEAN, first=(start_first and n == 0))

@@ -44,6 +44,9 @@ def _bind():
     lib.sf_step2d_substep_parts.argtypes = [C.c_void_p, C.POINTER(sf_step2d_fields), C.c_int32, C.c_double,
                                             C.c_double, C.c_double, C.c_int32, C.c_int32, C.c_void_p]
     lib.sf_step2d_substep_parts.restype = C.c_int32
+    lib.sf_step2d_run.argtypes = [C.c_void_p, C.POINTER(sf_step2d_fields), C.c_int32, C.c_double, C.c_void_p,
+                                  C.c_void_p, C.c_int32, C.c_int32, C.c_void_p, _I32P]
+    lib.sf_step2d_run.restype = C.c_int32
     lib.sf_step2d_tile_shape.argtypes = [_I32P, _I32P]
     lib.sf_step2d_tile_shape.restype = C.c_int32
     return lib
@@ -119,6 +122,15 @@ class FusedStepper:
                                               _lib.stream_handle(stream))
         _lib.check(rc, "sf_step2d_substep")
 
+    def run(self, compTimes, OCEAN, nsub: int, zero_vbar: bool = False):
+        """``nsub`` substeps (next2DTimeStep, cycleTimes2D, step) through one native call."""
+        from .phys2d import issue_substeps
+        a = self.fields(OCEAN)
+        flags = SF_SUBSTEP_ZERO_VBAR if zero_vbar else 0
+        issue_substeps(compTimes, OCEAN, nsub, "sf_step2d_run", lambda n, w1, cl, done: self.lib.sf_step2d_run(
+            self.ctx.handle, C.byref(a), self.precision, float(compTimes.dtfast), w1, cl, flags, n,
+            _lib.stream_handle(), C.byref(done)), clamp=clamped_value)
+
     def _cached_fields(self, OCEAN):
         key = (id(OCEAN), OCEAN.zeta_t0.data_ptr(), OCEAN.ubar_t0.data_ptr(), OCEAN.rubar_t0.data_ptr())
         cache = self.__dict__.setdefault("_fcache", {})
@@ -130,10 +142,19 @@ class FusedStepper:
         return a
 
 
-def step2d_substep(compTimes, GRID, OCEAN, BOUNDARY, zero_vbar: bool = False):
-    """One fused barotropic substep (after the caller's next2DTimeStep/cycleTimes2D)."""
+def _stepper(GRID, OCEAN, BOUNDARY) -> FusedStepper:
     st = getattr(GRID, "_sf_fused", None)
     if st is None or st.dtype != OCEAN.dtype:
         st = FusedStepper(GRID, BOUNDARY, OCEAN.dtype)
         GRID._sf_fused = st
-    st.step(compTimes, OCEAN, zero_vbar=zero_vbar)
+    return st
+
+
+def step2d_substep(compTimes, GRID, OCEAN, BOUNDARY, zero_vbar: bool = False):
+    """One fused barotropic substep (after the caller's next2DTimeStep/cycleTimes2D)."""
+    _stepper(GRID, OCEAN, BOUNDARY).step(compTimes, OCEAN, zero_vbar=zero_vbar)
+
+
+def step2d_run(compTimes, GRID, OCEAN, BOUNDARY, nsub: int, zero_vbar: bool = False):
+    """``nsub`` fused substeps, each after next2DTimeStep and cycleTimes2D."""
+    _stepper(GRID, OCEAN, BOUNDARY).run(compTimes, OCEAN, int(nsub), zero_vbar=zero_vbar)
