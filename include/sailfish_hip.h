@@ -196,7 +196,7 @@ int sf_set_lateral_uv_bcs_f32(sf_ctx *ctx, double t, float *u, float *v, const i
  * most SF_STEP3D_REG_LEVELS levels each column's system stays in registers (the scratch
  * is not touched) and tmpU / tmpV may be u / v themselves, so the copies main3d.py:48-52
  * makes before the call are not needed; deeper grids use the scratch and need the copies. */
-#define SF_STEP3D_REG_LEVELS 32
+#define SF_STEP3D_REG_LEVELS 64
 int sf_step3d_uv(sf_ctx *ctx, double *u, double *v, const double *ru, const double *rv,
                  double *ubar_t1, double *vbar_t1, double *ubar_t2, double *vbar_t2,
                  const double *Hz, const double *Akv, const double *z_r, const double *DU_avg1,

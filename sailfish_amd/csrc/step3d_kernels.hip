@@ -12,6 +12,8 @@
 // contraction off: results equal the CPU restatement bit for bit.
 #include "sf_internal.h"
 
+#include <type_traits>
+
 namespace {
 
 // a 3D (or 2D) field in global memory: pointer and element count; value type double
@@ -774,147 +776,186 @@ __global__ __launch_bounds__(256) void k_step3d_uv(G3 g, UVArgs<T> a, double cff
     a.vbar_t1[f] = T(vb);
 }
 
-// step3d_UV with each column's tridiagonal system held in registers (same arithmetic,
-// same order as k_step3d_uv; N <= NMAX).  The matrix of a direction is built and
-// eliminated level by level (build_matrix and the forward sweep of solve_tri fused),
-// the back substitution stores the solution with correct_mean's shift applied, and the
-// depth sums of correct_mean and adjustBarotropicVelocity run in the reference's level
-// order (the barotropic sums re-read the stored velocities).  At u-but-not-v points the
-// v pass solves the u pass's eliminated system a second time, as solve_tri does on the
-// shared scratch.  Each thread reads tmpU / tmpV only before it writes u / v, so they may
-// alias u / v.
+// step3d_UV with each column's tridiagonal system on chip (same arithmetic, same order as
+// k_step3d_uv; N <= NMAX): diagonal and right-hand side in registers, sub-diagonal in LDS.
+// One wave takes one direction (blockIdx.y: u, v) of 64 columns, so the two directions' level
+// chains -- two dependent divisions and a load latency per level, which bound the kernel --
+// run beside each other.  The matrix is built and eliminated level by level (build_matrix and
+// the forward sweep of solve_tri fused), the back substitution stores the solution with
+// correct_mean's shift applied, and the depth sums run in the reference's level order.  At
+// u-but-not-v points the u wave solves its eliminated system a second time for v, as
+// solve_tri does on the shared scratch.  Each thread reads tmpU (tmpV) only before it writes
+// u (v), and no other thread's column of them, so they may alias u / v.
+//
+// Addressing: an array's scalar base, advanced per level and passed through an empty asm
+// statement so that the unrolled levels keep no bases of their own, plus the column's 32-bit
+// byte offset.
+template <class T>
+__device__ __forceinline__ T ldc(const T *p, uint32_t o)
+{
+    return *(const __attribute__((address_space(1))) T *)((const __attribute__((address_space(1))) char *)p + o);
+}
+template <class T>
+__device__ __forceinline__ void stc(T *p, uint32_t o, T v)
+{
+    *(__attribute__((address_space(1))) T *)((__attribute__((address_space(1))) char *)p + o) = v;
+}
+template <class T>
+__device__ __forceinline__ T *step_base(T *p, long long d)
+{
+    p += d;
+    asm("" : "+s"(p));
+    return p;
+}
+
+// K < N, compared again at every unrolled level (kept comparisons of all levels spill)
+__device__ __forceinline__ bool has_level(int K, int N)
+{
+    asm volatile("" : "+s"(N));
+    return K < N;
+}
+
 template <class T, int NMAX>
-__global__ __launch_bounds__(256) void k_step3d_uv_reg(G3 g, UVArgs<T> a, double cff, double lambda, double Dt)
+__global__ __launch_bounds__(64) void k_step3d_uv_col(G3 g, UVArgs<T> a, double cff, double lambda, double Dt)
 {
     COLUMN_INDEX
     const long long S2 = g.S2;
-    const int N = g.N;
+    const int N = g.N, tid = threadIdx.x;
+    const bool vdir = blockIdx.y != 0;
     const bool un = isUNode(g, f), vn = isVNode(g, f);
-    if (!un && !vn) return;
-    T SD[NMAX], D[NMAX], R[NMAX];
+    if (!(vdir ? vn : un)) return;
+    __shared__ T sds[NMAX][64];
+    T D[NMAX], R[NMAX];
+    const uint32_t d = (uint32_t)((vdir ? g.szI : 1) * (long long)sizeof(T));
+    const uint32_t fo = (uint32_t)(f * (long long)sizeof(T)), fd = fo - d;
     const T mldt = T((-lambda) * Dt);
-    // build_matrix + forward elimination of direction vdir; Hs, Hx: correct_mean's sums.
-    // The operands of level K+1 are loaded before level K is computed.
-    auto build_elim = [&](bool vdir, const T *xold, const T *r, double &Hs, double &Hx) {
-        const long long d = vdir ? g.szI : 1;
-        const T pmU = (T(g.pm[f]) + T(g.pm[f - d])) * T(0.5);
-        const T pnU = (T(g.pn[f]) + T(g.pn[f - d])) * T(0.5);
+    const T *xold = vdir ? a.tmpV : a.tmpU, *r = vdir ? a.rv : a.ru;
+    T *x = vdir ? a.v : a.u;
+    double Hs = 0.0, Hx = 0.0;   // correct_mean's sums
+    {
+        const long long nb = vdir ? g.szI : 1;
+        const T pmU = (T(g.pm[f]) + T(g.pm[f - nb])) * T(0.5);
+        const T pnU = (T(g.pn[f]) + T(g.pn[f - nb])) * T(0.5);
         const T cdt_mn = T(cff * Dt) * (pmU * pnU);
-        T zf0 = a.z_r[f], zd0 = a.z_r[f - d];
+        const T *pH = a.Hz, *pX = xold, *pR = r, *pZ = a.z_r, *pK = a.Akv;
+        T zf0 = ldc(pZ, fo), zd0 = ldc(pZ, fd);
+        pZ = step_base(pZ, S2);
         struct Lv {
             T h0, h1, xo, rr, z0, z1, k0, k1;
         };
-        auto load = [&](int K) {
+        // the operands of a level (z_r of the level above); level K+1 is loaded before level
+        // K is computed
+        auto load = [&](bool top) {
             Lv q{};
-            const long long b = K * S2 + f;
-            q.h0 = a.Hz[b];
-            q.h1 = a.Hz[b - d];
-            q.xo = xold[b];
-            q.rr = r[b];
-            if (K < N - 1) {
-                q.z0 = a.z_r[b + S2];
-                q.z1 = a.z_r[b + S2 - d];
-                q.k0 = a.Akv[b];
-                q.k1 = a.Akv[b - d];
+            q.h0 = ldc(pH, fo);
+            q.h1 = ldc(pH, fd);
+            q.xo = ldc(pX, fo);
+            q.rr = ldc(pR, fo);
+            if (!top) {
+                q.z0 = ldc(pZ, fo);
+                q.z1 = ldc(pZ, fd);
+                q.k0 = ldc(pK, fo);
+                q.k1 = ldc(pK, fd);
             }
+            pH = step_base(pH, S2);
+            pX = step_base(pX, S2);
+            pR = step_base(pR, S2);
+            pZ = step_base(pZ, S2);
+            pK = step_base(pK, S2);
             return q;
         };
-        Lv cur = load(0);
-        Hs = 0.0;
-        Hx = 0.0;
+        Lv cur = load(N == 1);
+        T sdp = T(0);   // sub-diagonal of the level below
 #pragma unroll
         for (int K = 0; K < NMAX; K++) {
-            if (K < N) {
+            if (has_level(K, N)) {
                 Lv nxt{};
-                if (K + 1 < N) nxt = load(K + 1);
+                if (has_level(K + 1, N)) nxt = load(K + 1 == N - 1);
                 const T hz = (cur.h0 + cur.h1) * T(0.5);
-                const T xo = cur.xo;
                 Hs += (double)hz;
-                Hx += (double)xo * (double)hz;
+                Hx += (double)cur.xo * (double)hz;
                 T sd = T(0);
-                if (K < N - 1) {
+                if (has_level(K + 1, N)) {
                     const T dz = ((cur.z0 - zf0) + (cur.z1 - zd0)) * T(0.5);
                     sd = (mldt * ((cur.k0 + cur.k1) * T(0.5))) / dz;
                     zf0 = cur.z0;
                     zd0 = cur.z1;
                 }
-                SD[K] = sd;
+                sds[K][tid] = sd;
                 if (K == 0) {
                     D[0] = hz - T(2) * sd;
                     R[0] = T(0);
                 } else {
-                    D[K] = (hz - sd) - SD[K - 1];
-                    R[K] = hz * (xo + cdt_mn * cur.rr);
-                    const T w = SD[K - 1] / D[K - 1];
-                    D[K] -= w * SD[K - 1];
+                    D[K] = (hz - sd) - sdp;
+                    R[K] = hz * (cur.xo + cdt_mn * cur.rr);
+                    const T w = sdp / D[K - 1];
+                    D[K] -= w * sdp;
                     R[K] -= w * R[K - 1];
                 }
+                sdp = sd;
                 cur = nxt;
             }
         }
-    };
-    // the forward sweep of solve_tri on an already eliminated system
-    auto elim_again = [&]() {
-#pragma unroll
-        for (int K = 1; K < NMAX; K++) {
-            if (K < N) {
-                const T w = SD[K - 1] / D[K - 1];
-                D[K] -= w * SD[K - 1];
-                R[K] -= w * R[K - 1];
-            }
-        }
-    };
-    // back substitution; stores x - shift at every level of x
-    auto back_store = [&](T *x, double shift) {
+    }
+    // back substitution; stores x - shift at every level of y, and keeps it in R unless the
+    // system is solved again
+    const bool again = !vdir && !vn;
+    auto back_store = [&](T *y, double shift, bool keep) {
+        y = step_base(y, (long long)(N - 1) * S2);
         T xn = T(0);
 #pragma unroll
         for (int K = NMAX - 1; K >= 0; K--) {
-            if (K < N) {
-                const T xk = K == N - 1 ? R[K] / D[K] : (R[K] - SD[K] * xn) / D[K];
-                x[K * S2 + f] = T((double)xk - shift);
+            if (has_level(K, N)) {
+                const T xk = K == N - 1 ? R[K] / D[K] : (R[K] - sds[K][tid] * xn) / D[K];
+                const T xs = T((double)xk - shift);
+                stc(y, fo, xs);
+                y = step_base(y, -S2);
+                if (keep) R[K] = xs;
                 xn = xk;
             }
         }
     };
-    double HU = 0.0, HuU = 0.0;
-    if (un) {
-        double Hs, Hx;
-        build_elim(false, a.tmpU, a.ru, Hs, Hx);
-        const double diff = (Hx - a.DU_avg1[f] / g.on_u[f]) / Hs;
-        back_store(a.u, diff);   // leaves SD, D, R as they are (reused below where !vn)
-    }
-    if (vn) {
-        double Hs, Hx;
-        build_elim(true, a.tmpV, a.rv, Hs, Hx);
-        const double diff = (Hx - a.DV_avg1[f] / g.om_v[f]) / Hs;
-        if (un) {
-            back_store(a.v, diff);
-        } else {
-            for (int K = 0; K < N; K++) a.v[K * S2 + f] = T((double)a.v[K * S2 + f] - diff);
+    // adjustBarotropicVelocity of one direction: yk(K) the stored velocity, hd the byte
+    // offset of the neighbour the thickness averages with
+    auto barotropic = [&](bool kept, const T *y, uint32_t hd, const double *Davg, const double *met, T *t1, T *t2) {
+        double Hsum = 0.0, Hy = 0.0;
+        const T *pH = a.Hz;
+#pragma unroll
+        for (int K = 0; K < NMAX; K++) {
+            if (has_level(K, N)) {
+                const T hz = (ldc(pH, fo) + ldc(pH, hd)) * T(0.5);
+                pH = step_base(pH, S2);
+                const T yk = kept ? R[K] : y[K * S2 + f];
+                Hsum += (double)hz;
+                Hy += (double)hz * (double)yk;
+            }
         }
-    } else {
-        elim_again();
-        back_store(a.v, 0.0);
+        const double up = (Hy - Davg[f] / met[f]) / Hsum;
+        const T yb = T((Davg[f] / met[f]) / Hsum + up);
+        t2[f] = yb;
+        t1[f] = yb;
+    };
+    const double *Davg = vdir ? a.DV_avg1 : a.DU_avg1, *met = vdir ? g.om_v : g.on_u;
+    const double diff = (Hx - Davg[f] / met[f]) / Hs;
+    if (!un) {   // a v point that solve_tri skips: the shift alone
+        for (int K = 0; K < N; K++) x[K * S2 + f] = T((double)x[K * S2 + f] - diff);
+        return;
     }
-    if (!un) return;
-    double HV = 0.0, HvV = 0.0;
-    for (int K = 0; K < N; K++) {
-        const long long b = K * S2 + f;
-        const T hzu = (a.Hz[b] + a.Hz[b - 1]) * T(0.5);
-        const T hzv = (a.Hz[b] + a.Hz[b - g.szI]) * T(0.5);
-        HU += (double)hzu;
-        HV += (double)hzv;
-        HuU += (double)hzu * (double)a.u[b];
-        HvV += (double)hzv * (double)a.v[b];
+    back_store(x, diff, !again);
+    barotropic(!again, x, fd, Davg, met, vdir ? a.vbar_t1 : a.ubar_t1, vdir ? a.vbar_t2 : a.ubar_t2);
+    if (again) {
+        // the forward sweep of solve_tri on the already eliminated system, solved into v
+#pragma unroll
+        for (int K = 1; K < NMAX; K++) {
+            if (has_level(K, N)) {
+                const T w = sds[K - 1][tid] / D[K - 1];
+                D[K] -= w * sds[K - 1][tid];
+                R[K] -= w * R[K - 1];
+            }
+        }
+        back_store(a.v, 0.0, true);
+        barotropic(true, a.v, fo - (uint32_t)(g.szI * (long long)sizeof(T)), a.DV_avg1, g.om_v, a.vbar_t1, a.vbar_t2);
     }
-    const double uUp = (HuU - a.DU_avg1[f] / g.on_u[f]) / HU;
-    const double vUp = (HvV - a.DV_avg1[f] / g.om_v[f]) / HV;
-    const double ub = (a.DU_avg1[f] / g.on_u[f]) / HU + uUp;
-    const double vb = (a.DV_avg1[f] / g.om_v[f]) / HV + vUp;
-    a.ubar_t2[f] = T(ub);
-    a.vbar_t2[f] = T(vb);
-    a.ubar_t1[f] = T(ub);
-    a.vbar_t1[f] = T(vb);
 }
 
 // ---- coupling of the 2D and 3D momentum equations (ROMS split-explicit form) ----------
@@ -1100,17 +1141,19 @@ __device__ __forceinline__ uint32_t next_level(uint32_t o, uint32_t stride)
 }
 
 template <class T, int NMAX>
-__global__ __launch_bounds__(256) void k_step3d_uv_coupled_reg(G3 g, UVC<T> a, double lambda, double Dt)
+__global__ __launch_bounds__(64) void k_step3d_uv_coupled_col(G3 g, UVC<T> a, double lambda, double Dt)
 {
     COLUMN_INDEX
     const int N = g.N;
+    const bool vdir = blockIdx.y != 0;
+    if (!coupled_point(g, vdir, f)) return;
     const uint32_t SB = (uint32_t)(g.S2 * (long long)sizeof(T));   // level stride in bytes
     const uint32_t o0 = (uint32_t)(f * (long long)sizeof(T));      // level 0 of the column
-    __shared__ T sds[NMAX][256];   // the sub-diagonal of each column (thread)
+    __shared__ T sds[NMAX][64];   // the sub-diagonal of each column (thread)
     T D[NMAX], R[NMAX];
     const int tid = threadIdx.x;
     const T mldt = T((-lambda) * Dt);
-    auto column = [&](bool vdir) {
+    {
         const long long d = vdir ? g.szI : 1;
         const uint32_t dB = (uint32_t)(d * (long long)sizeof(T));
         T *x = vdir ? a.v : a.u, *keep = vdir ? a.rv_keep : a.ru_keep, *Hf = vdir ? a.Hvom : a.Huon;
@@ -1149,12 +1192,12 @@ __global__ __launch_bounds__(256) void k_step3d_uv_coupled_reg(G3 g, UVC<T> a, d
         Lv cur = load(ob, N - 1 == 0);
 #pragma unroll
         for (int K = 0; K < NMAX; K++) {
-            if (K < N) {
+            if (has_level(K, N)) {
                 const uint32_t on = next_level(ob, SB);
                 Lv nxt{};
-                if (K + 1 < N) nxt = load(on, K + 1 >= N - 1);
+                if (has_level(K + 1, N)) nxt = load(on, K + 1 >= N - 1);
                 T sd = T(0);
-                if (K < N - 1) {
+                if (has_level(K + 1, N)) {
                     const T dz = ((cur.z0 - zf0) + (cur.z1 - zd0)) * T(0.5);
                     sd = (mldt * ((cur.k0 + cur.k1) * T(0.5))) / dz;
                     zf0 = cur.z0;
@@ -1187,7 +1230,7 @@ __global__ __launch_bounds__(256) void k_step3d_uv_coupled_reg(G3 g, UVC<T> a, d
         // back substitution: R(K) := x(K)
 #pragma unroll
         for (int K = NMAX - 1; K >= 0; K--) {
-            if (K < N) R[K] = K == N - 1 ? R[K] / D[K] : (R[K] - sds[K][tid] * R[K + 1]) / D[K];
+            if (has_level(K, N)) R[K] = K == N - 1 ? R[K] / D[K] : (R[K] - sds[K][tid] * R[K + 1]) / D[K];
         }
         // couple_column: replace the column mean, correct the mass flux
         const double met = vdir ? 2.0 / (g.pm[f - g.szI] + g.pm[f]) : 2.0 / (g.pn[f - 1] + g.pn[f]);
@@ -1195,7 +1238,7 @@ __global__ __launch_bounds__(256) void k_step3d_uv_coupled_reg(G3 g, UVC<T> a, d
         ob = o0;
 #pragma unroll
         for (int K = 0; K < NMAX; K++) {
-            if (K < N) {
+            if (has_level(K, N)) {
                 const T hn = (ldb(a.Hz, ob) + ldb(a.Hz, ob - dB)) * T(0.5);
                 D[K] = hn;
                 const double dc = met * (double)hn;
@@ -1214,7 +1257,7 @@ __global__ __launch_bounds__(256) void k_step3d_uv_coupled_reg(G3 g, UVC<T> a, d
         ob = o0;
 #pragma unroll
         for (int K = 0; K < NMAX; K++) {
-            if (K < N) {
+            if (has_level(K, N)) {
                 const T xk = T((double)R[K] - CF);
                 stb(x, ob, xk);
                 const T hf = T(0.5 * ((double)ldb((const T *)Hf, ob) + (double)xk * (met * (double)D[K])));
@@ -1227,14 +1270,24 @@ __global__ __launch_bounds__(256) void k_step3d_uv_coupled_reg(G3 g, UVC<T> a, d
         ob = o0;
 #pragma unroll
         for (int K = 0; K < NMAX; K++) {
-            if (K < N) {
+            if (has_level(K, N)) {
                 stb(Hf, ob, T((double)R[K] - (met * (double)D[K]) * FC));
                 ob = next_level(ob, SB);
             }
         }
-    };
-    if (coupled_point(g, false, f)) column(false);
-    if (coupled_point(g, true, f)) column(true);
+    }
+}
+
+// fn with the fewest levels (a compile-time count) that hold N <= SF_STEP3D_REG_LEVELS
+template <class F>
+int by_levels(int N, F &&fn)
+{
+    if (N <= 16) return fn(std::integral_constant<int, 16>{});
+    if (N <= 24) return fn(std::integral_constant<int, 24>{});
+    if (N <= 32) return fn(std::integral_constant<int, 32>{});
+    if (N <= 40) return fn(std::integral_constant<int, 40>{});
+    if (N <= 48) return fn(std::integral_constant<int, 48>{});
+    return fn(std::integral_constant<int, SF_STEP3D_REG_LEVELS>{});
 }
 
 G3 grid3(const sf_ctx *c)
@@ -1449,18 +1502,22 @@ extern "C" int sf_set_lateral_uv_bcs_f32(sf_ctx *c, double t, float *u, float *v
     LAUNCH_COLUMNS(k_lateral_uv<float>, c, stream, grid3(c), t, u, v, uType, vType);
 }
 
-// step3d_UV: columns of up to 32 levels in registers (k_step3d_uv_reg), deeper ones
-// through the SD/D/RHS scratch (k_step3d_uv)
+// step3d_UV: columns of up to 64 levels on chip (k_step3d_uv_col), deeper ones through the
+// SD/D/RHS scratch (k_step3d_uv)
 template <class T>
 static int step3d_uv_launch(sf_ctx *c, const UVArgs<T> &a, double cff, double lambda, double Dt, void *stream)
 {
-    if (c->szK <= 16) {
-        LAUNCH_COLUMNS((k_step3d_uv_reg<T, 16>), c, stream, grid3(c), a, cff, lambda, Dt);
+    if (c->szK > SF_STEP3D_REG_LEVELS) {
+        LAUNCH_COLUMNS(k_step3d_uv<T>, c, stream, grid3(c), a, cff, lambda, Dt);
     }
-    if (c->szK <= 32) {
-        LAUNCH_COLUMNS((k_step3d_uv_reg<T, 32>), c, stream, grid3(c), a, cff, lambda, Dt);
-    }
-    LAUNCH_COLUMNS(k_step3d_uv<T>, c, stream, grid3(c), a, cff, lambda, Dt);
+    SF_REQUIRE(c->S2 * sizeof(T) < (1ull << 32), "sf_step3d_uv: a level of %lld points exceeds 4 GiB", c->S2);
+    // by_levels: the fewest levels an instance holds; registers and LDS of the unused ones
+    // would cost waves (FP64: 3 waves per SIMD up to 24 levels, 2 up to 48, 1 to 64)
+    return by_levels(c->szK, [&](auto nmax) {
+        hipLaunchKernelGGL((k_step3d_uv_col<T, decltype(nmax)::value>), dim3(sf::grid1d(c->S2, 64), 2), dim3(64), 0,
+                           sf::as_stream(stream), grid3(c), a, cff, lambda, Dt);
+        return sf::check_launch("sf_step3d_uv");
+    });
 }
 
 extern "C" int sf_step3d_uv(sf_ctx *c, double *u, double *v, const double *ru, const double *rv, double *ubar_t1,
@@ -1521,12 +1578,12 @@ int step3d_uv_coupled_launch(sf_ctx *c, const sf_uv_coupled *p, double lambda, d
              (T *)p->Hvom, p->sustr, p->svstr, p->rdrg, p->ab, (T *)p->SD, (T *)p->D, (T *)p->RHS};
     // register columns address every level with 32-bit byte offsets
     const bool fits = (unsigned long long)(c->szK + 1) * (unsigned long long)c->S2 * sizeof(T) < (1ull << 32);
-    if (fits && c->szK <= 16) {
-        LAUNCH_COLUMNS((k_step3d_uv_coupled_reg<T, 16>), c, stream, grid3(c), a, lambda, Dt);
-    }
-    if (fits && c->szK <= 32) {
-        LAUNCH_COLUMNS((k_step3d_uv_coupled_reg<T, 32>), c, stream, grid3(c), a, lambda, Dt);
-    }
+    if (fits && c->szK <= SF_STEP3D_REG_LEVELS)
+        return by_levels(c->szK, [&](auto nmax) {
+            hipLaunchKernelGGL((k_step3d_uv_coupled_col<T, decltype(nmax)::value>), dim3(sf::grid1d(c->S2, 64), 2),
+                               dim3(64), 0, sf::as_stream(stream), grid3(c), a, lambda, Dt);
+            return sf::check_launch("sf_step3d_uv_coupled");
+        });
     LAUNCH_COLUMNS(k_step3d_uv_coupled<T>, c, stream, grid3(c), a, lambda, Dt);
 }
 

@@ -3,7 +3,7 @@
 Per baroclinic step: set_maxflux, omega, set_zeta, rhs3d, the nfast+1 barotropic
 substeps (main3d.py:166-189), the NetCDF history record when one is due
 (main3d.py:202-216; ``history`` is an ``io_netcdf.HistoryWriter``), set_depth,
-step3d_UV (on copies tmpU/tmpV above 32 levels), setLateralUVBCs, omega, nextTimeStep.  ``fused=True``
+step3d_UV (on copies tmpU/tmpV above 64 levels), setLateralUVBCs, omega, nextTimeStep.  ``fused=True``
 runs each barotropic substep as one fused kernel (same state).
 """
 from __future__ import annotations
@@ -17,7 +17,7 @@ from .rhs import rhs3d
 
 # columns of at most this many levels are solved in registers by step3d_UV, which then
 # reads the old velocities before it writes the new ones (SF_STEP3D_REG_LEVELS)
-STEP3D_REG_LEVELS = 32
+STEP3D_REG_LEVELS = 64
 
 
 class Main3dState:
