@@ -14,9 +14,15 @@ struct Col {
     int szI, szJ, N;
     long long S2;
     const double *pm, *pn;
+    bool band;   // columns in XCD bands (sf::column_block)
 };
 
-inline Col col_of(const sf_ctx *c) { return Col{c->szI, c->szJ, c->szK, c->S2, c->pm, c->pn}; }
+// elem: bytes of a 3D field's element
+inline Col col_of(const sf_ctx *c, size_t elem)
+{
+    const bool band = (c->szK + 1.0) * (double)c->S2 * (double)elem <= sf::kBandBytes;
+    return Col{c->szI, c->szJ, c->szK, c->S2, c->pm, c->pn, band};
+}
 
 // ---- linear equation of state: rho = ((R0 - 1000) - R0 Tcoef (T - T0)) + R0 Scoef (S - S0)
 template <class T>
@@ -76,7 +82,7 @@ template <class T>
 __global__ __launch_bounds__(256) void k_prsgrd(Col g, const T *rho, const T *z_r, const T *z_w, const T *Hz,
                                                 double grav, double rho0, T *ru, T *rv)
 {
-    const long long f = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long f = (long long)sf::column_block(g.band) * blockDim.x + threadIdx.x;
     if (f >= g.S2) return;
     pgf_column(g, false, f, rho, z_r, z_w, Hz, grav, rho0, ru);
     pgf_column(g, true, f, rho, z_r, z_w, Hz, grav, rho0, rv);
@@ -90,7 +96,7 @@ template <class T>
 __global__ __launch_bounds__(256) void k_step3d_t(Col g, const T *t, T *tn, const T *Huon, const T *Hvom,
                                                   const T *Hz_old, const T *Hz_new, double dt)
 {
-    const long long f = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long f = (long long)sf::column_block(g.band) * blockDim.x + threadIdx.x;
     if (f >= g.S2) return;
     const long long S2 = g.S2, W = g.szI;
     const int N = g.N, i = (int)(f % W), j = (int)(f / W), L = g.szI - 1, M = g.szJ - 1;
@@ -156,7 +162,7 @@ template <class T>
 int prsgrd_launch(sf_ctx *c, const void *rho, const void *z_r, const void *z_w, const void *Hz, double g,
                   double rho0, void *ru, void *rv, void *stream)
 {
-    hipLaunchKernelGGL(k_prsgrd<T>, dim3(sf::grid1d(c->S2)), dim3(256), 0, sf::as_stream(stream), col_of(c),
+    hipLaunchKernelGGL(k_prsgrd<T>, dim3(sf::column_grid(c->S2)), dim3(256), 0, sf::as_stream(stream), col_of(c, sizeof(T)),
                        (const T *)rho, (const T *)z_r, (const T *)z_w, (const T *)Hz, g, rho0, (T *)ru, (T *)rv);
     return sf::check_launch("sf_prsgrd");
 }
@@ -166,8 +172,8 @@ int tracer_launch(sf_ctx *c, const void *t, void *tn, const void *Huon, const vo
                   const void *Hz_new, double dt, void *stream)
 {
     hipStream_t s = sf::as_stream(stream);
-    const Col g = col_of(c);
-    hipLaunchKernelGGL(k_step3d_t<T>, dim3(sf::grid1d(c->S2)), dim3(256), 0, s, g, (const T *)t, (T *)tn,
+    const Col g = col_of(c, sizeof(T));
+    hipLaunchKernelGGL(k_step3d_t<T>, dim3(sf::column_grid(c->S2)), dim3(256), 0, s, g, (const T *)t, (T *)tn,
                        (const T *)Huon, (const T *)Hvom, (const T *)Hz_old, (const T *)Hz_new, dt);
     hipLaunchKernelGGL(k_tracer_ghost_rows<T>, dim3(sf::grid1d(c->szI), c->szK), dim3(256), 0, s, g, (T *)tn);
     hipLaunchKernelGGL(k_tracer_ghost_cols<T>, dim3(sf::grid1d(c->szJ), c->szK), dim3(256), 0, s, g, (T *)tn);

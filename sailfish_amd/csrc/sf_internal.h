@@ -80,6 +80,29 @@ inline unsigned grid1d(long long n, int block = kBlock1D)
     return (unsigned)((n + block - 1) / block);
 }
 
+// Blocks of water columns in XCD bands.  Block b runs on XCD b % 8, each with its own L2;
+// with blocks of columns dealt out in turn, the rows j-1 and j+1 that a stencil reads belong
+// to other XCDs and are fetched once per XCD.  In bands XCD x takes the x-th eighth of the
+// columns, so a row fetched for its own columns serves its neighbours from L2.  Measured
+// (FP32, 67 MB a field, 1024 x 512 x 32): set_maxflux 66 us -> 57; FP64 700 x 400 x 32 (72 MB):
+// 71 -> 60.  Where a field passes about half the last-level cache the kernels stream from
+// HBM, and eight far-apart streams lose there: FP64 1024 x 512 x 32 (138 MB) 140 us -> 157,
+// tracer step 503 -> 520.  So bands up to 100 MB a field.
+constexpr double kBandBytes = 100e6;
+inline unsigned column_grid(long long n, int block = kBlock1D) { return (grid1d(n, block) + 7) / 8 * 8; }
+__device__ __forceinline__ unsigned column_block(bool band)
+{
+    return band ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+}
+// the same with two blocks per block of columns (grid 2 * column_grid), one after the other
+// on the same XCD
+__device__ __forceinline__ bool column_pair_second() { return (blockIdx.x >> 3) & 1; }
+__device__ __forceinline__ unsigned column_pair_block(bool band)
+{
+    const unsigned x = blockIdx.x & 7, k = blockIdx.x >> 4;
+    return band ? x * (gridDim.x >> 4) + k : k * 8 + x;
+}
+
 }  // namespace sf
 
 #define SF_REQUIRE(cond, ...)                 \

@@ -47,6 +47,7 @@ struct G3 {
     int szI, szJ, N;
     long long S2;
     const double *on_u, *om_v, *pn, *pm;
+    bool band;   // columns in XCD bands (sf::column_block)
 };
 
 __device__ __forceinline__ bool isRNode(const G3 &g, long long f) { return (f % g.szI) > 0 && (f / g.szI) > 0; }
@@ -62,8 +63,8 @@ __device__ __forceinline__ bool isInnerCell(const G3 &g, long long f)
     return i > 1 && i < g.szI - 2 && j > 1 && j < g.szJ - 2;
 }
 
-#define COLUMN_INDEX                                                      \
-    const long long f = (long long)blockIdx.x * blockDim.x + threadIdx.x; \
+#define COLUMN_INDEX                                                                 \
+    const long long f = (long long)sf::column_block(g.band) * blockDim.x + threadIdx.x; \
     if (f >= g.S2) return;
 
 // ---- addCoriolis (rhs_kernels.cpp:6-35) -------------------------------------------
@@ -343,7 +344,7 @@ __global__ __launch_bounds__(256) void k_verticalAdvection(G3 g, A U, A V, A Wa,
 // stencils are read from global memory, u/v along the column through a sliding window.
 //
 // The levels are split into nchunk chunks of kchunk levels (the last one takes the
-// remainder and has at least 3 levels), one workgroup per tile and chunk.  A chunk seeds
+// remainder), one workgroup per tile and chunk.  A chunk seeds
 // the vertical-flux window at its first interior level with the same expression the
 // sliding window evaluates there, so the split changes no result.  The first chunk
 // (levels 0, 1) does the bottom special levels, the last chunk (levels N-3 .. N) the
@@ -356,7 +357,7 @@ __global__ __launch_bounds__(256) void k_verticalAdvection(G3 g, A U, A V, A Wa,
 template <int TJ, class T, int WPE>
 __global__ __launch_bounds__(HTI * TJ) __attribute__((amdgpu_waves_per_eu(WPE)))
 void k_rhs3d_fused(G3 g, HG<T> h, A fomn, AG<T> Hz, AG<T> Wa, const int32_t *BC, T *ru, T *rv, long long tail_end,
-                   int cor, int adv, int tiles_i, int ntiles, int kchunk, int nchunk)
+                   int cor, int adv, int tiles_i, int ntiles, int ntiles8, int kchunk, int nchunk)
 {
     constexpr int NT = HTI * TJ, LN = HLW * (TJ + 5);
     // The face fluxes of the level are each evaluated once, into LDS -- x-faces
@@ -370,7 +371,10 @@ void k_rhs3d_fused(G3 g, HG<T> h, A fomn, AG<T> Hz, AG<T> Wa, const int32_t *BC,
     constexpr bool SB = sizeof(T) == 8;   // single tile buffer
     __shared__ T sl[SB ? 1 : 2][4][LN];
     __shared__ T fxu[TJ][HTI + 1], fxv[TJ][HTI + 1], feu[TJ + 1][HTI], fev[TJ + 1][HTI];
-    const int tile = blockIdx.x % ntiles, kc = blockIdx.x / ntiles;
+    // XCD-banded tile order, as the columns of the other kernels
+    const int b8 = blockIdx.x % (unsigned)ntiles8, kc = blockIdx.x / (unsigned)ntiles8;
+    const int tile = g.band ? (b8 & 7) * (ntiles8 >> 3) + (b8 >> 3) : b8;
+    if (tile >= ntiles) return;
     const int ti = tile % tiles_i, tj = tile / tiles_i;
     const int i0 = ti * HTI, j0 = tj * TJ;
     const int c = threadIdx.x % HTI, r = threadIdx.x / HTI;
@@ -778,7 +782,7 @@ __global__ __launch_bounds__(256) void k_step3d_uv(G3 g, UVArgs<T> a, double cff
 
 // step3d_UV with each column's tridiagonal system on chip (same arithmetic, same order as
 // k_step3d_uv; N <= NMAX): diagonal and right-hand side in registers, sub-diagonal in LDS.
-// One wave takes one direction (blockIdx.y: u, v) of 64 columns, so the two directions' level
+// One wave takes one direction (u or v) of 64 columns, so the two directions' level
 // chains -- two dependent divisions and a load latency per level, which bound the kernel --
 // run beside each other.  The matrix is built and eliminated level by level (build_matrix and
 // the forward sweep of solve_tri fused), the back substitution stores the solution with
@@ -818,10 +822,11 @@ __device__ __forceinline__ bool has_level(int K, int N)
 template <class T, int NMAX>
 __global__ __launch_bounds__(64) void k_step3d_uv_col(G3 g, UVArgs<T> a, double cff, double lambda, double Dt)
 {
-    COLUMN_INDEX
+    const bool vdir = sf::column_pair_second();
+    const long long f = (long long)sf::column_pair_block(true) * blockDim.x + threadIdx.x;
+    if (f >= g.S2) return;
     const long long S2 = g.S2;
     const int N = g.N, tid = threadIdx.x;
-    const bool vdir = blockIdx.y != 0;
     const bool un = isUNode(g, f), vn = isVNode(g, f);
     if (!(vdir ? vn : un)) return;
     __shared__ T sds[NMAX][64];
@@ -1143,9 +1148,10 @@ __device__ __forceinline__ uint32_t next_level(uint32_t o, uint32_t stride)
 template <class T, int NMAX>
 __global__ __launch_bounds__(64) void k_step3d_uv_coupled_col(G3 g, UVC<T> a, double lambda, double Dt)
 {
-    COLUMN_INDEX
+    const bool vdir = sf::column_pair_second();
+    const long long f = (long long)sf::column_pair_block(g.band) * blockDim.x + threadIdx.x;
+    if (f >= g.S2) return;
     const int N = g.N;
-    const bool vdir = blockIdx.y != 0;
     if (!coupled_point(g, vdir, f)) return;
     const uint32_t SB = (uint32_t)(g.S2 * (long long)sizeof(T));   // level stride in bytes
     const uint32_t o0 = (uint32_t)(f * (long long)sizeof(T));      // level 0 of the column
@@ -1290,9 +1296,11 @@ int by_levels(int N, F &&fn)
     return fn(std::integral_constant<int, SF_STEP3D_REG_LEVELS>{});
 }
 
-G3 grid3(const sf_ctx *c)
+// elem: bytes of a 3D field's element
+G3 grid3(const sf_ctx *c, size_t elem)
 {
-    return G3{c->szI, c->szJ, c->szK, c->S2, c->on_u, c->om_v, c->pn, c->pm};
+    const bool band = (c->szK + 1.0) * (double)c->S2 * (double)elem <= sf::kBandBytes;
+    return G3{c->szI, c->szJ, c->szK, c->S2, c->on_u, c->om_v, c->pn, c->pm, band};
 }
 
 }  // namespace
@@ -1302,7 +1310,7 @@ G3 grid3(const sf_ctx *c)
     SF_REQUIRE((c)->szK >= 4, "%s: needs at least 4 levels (N=%d)", __func__, (c)->szK)
 
 #define LAUNCH_COLUMNS(kern, c, stream, ...)                                                                  \
-    hipLaunchKernelGGL(kern, dim3(sf::grid1d((c)->S2)), dim3(sf::kBlock1D), 0, sf::as_stream(stream), __VA_ARGS__); \
+    hipLaunchKernelGGL(kern, dim3(sf::column_grid((c)->S2)), dim3(sf::kBlock1D), 0, sf::as_stream(stream), __VA_ARGS__); \
     return sf::check_launch(__func__)
 
 extern "C" int sf_add_coriolis(sf_ctx *c, const double *fomn, const double *u, const double *v, double *ru,
@@ -1311,7 +1319,7 @@ extern "C" int sf_add_coriolis(sf_ctx *c, const double *fomn, const double *u, c
     CTX3(c);
     SF_REQUIRE(fomn && u && v && ru && rv && Hz, "sf_add_coriolis: null field");
     const long long n3 = (c->szK + 1LL) * c->S2;
-    LAUNCH_COLUMNS(k_addCoriolis, c, stream, grid3(c), A{fomn, c->S2}, A{u, n3}, A{v, n3}, ru, rv,
+    LAUNCH_COLUMNS(k_addCoriolis, c, stream, grid3(c, sizeof(double)), A{fomn, c->S2}, A{u, n3}, A{v, n3}, ru, rv,
                    A{Hz, (long long)c->szK * c->S2});
 }
 
@@ -1325,7 +1333,7 @@ extern "C" int sf_horizontal_advection(sf_ctx *c, const double *u, const double 
     H h{A{u, n3}, A{v, n3}, A{Huon, n3}, A{Hvom, n3}, c->szI};
     const int tiles_i = (c->szI + HTI - 1) / HTI, tiles_j = (c->szJ + HTJ - 1) / HTJ;
     hipLaunchKernelGGL(k_horizontalAdvection_tiled, dim3((unsigned)(tiles_i * tiles_j)), dim3(HNT), 0,
-                       sf::as_stream(stream), grid3(c), h, ru, rv, tiles_i);
+                       sf::as_stream(stream), grid3(c, sizeof(double)), h, ru, rv, tiles_i);
     int rc = sf::check_launch("sf_horizontal_advection");
     if (rc != SF_OK) return rc;
     const long long end = launch_threads < n3 ? (long long)launch_threads : n3;
@@ -1343,7 +1351,7 @@ extern "C" int sf_vertical_advection(sf_ctx *c, const double *u, const double *v
     CTX3(c);
     SF_REQUIRE(u && v && W && ru && rv && BC, "sf_vertical_advection: null field");
     const long long n3 = (c->szK + 1LL) * c->S2;
-    LAUNCH_COLUMNS(k_verticalAdvection, c, stream, grid3(c), A{u, n3}, A{v, n3}, A{W, n3}, ru, rv, BC);
+    LAUNCH_COLUMNS(k_verticalAdvection, c, stream, grid3(c, sizeof(double)), A{u, n3}, A{v, n3}, A{W, n3}, ru, rv, BC);
 }
 
 template <class T>
@@ -1363,25 +1371,37 @@ static int rhs3d_launch(sf_ctx *c, const double *fomn, const T *u, const T *v, c
     // only its register limit); smaller grids run the 4-wave instance with level chunks
     // (512 x 256 x 32: 65 us in three chunks, 73 us in four).
     const bool wide32 = sizeof(T) == 4 && ntiles >= 4 * cus;
-    // level chunks: the fewest that give every resident workgroup slot (three per CU) a
-    // workgroup, with at least 3 levels per chunk (the bottom and top special levels each
-    // stay within one chunk); the last chunk takes the remainder.  1024 x 512 x 32 runs
-    // unsplit.
-    const long long slots = 3 * cus;
+    // Level chunks (at least 3 levels each, so that the bottom and top special levels stay
+    // within one; the last takes the remainder): the count that minimises rounds of resident
+    // workgroups times levels of the longest chunk, two levels' worth of start-up added per
+    // round.  Resident: four workgroups a CU for the 8-wave FP32 instance, three for the
+    // others.  Unsplit, a few tiles more than fit cost a whole second round: 1024 x 512 x 32
+    // FP64 468 us -> 420 in two chunks, 700 x 400 x 32 279 -> 230 in four, FP32 1000 x 520 x 32
+    // 361 -> 262 in four.
+    const long long slots = (wide32 ? 4 : 3) * cus;
     int nchunk = 1;
-    while (!wide32 && (long long)ntiles * nchunk < slots && c->szK / (nchunk + 1) >= 3) nchunk++;
+    long long best = 0;
+    for (int n = 1; n == 1 || c->szK / n >= 3; n++) {
+        const long long rounds = ((long long)ntiles * n + slots - 1) / slots;
+        const long long cost = rounds * (c->szK - (n - 1) * (c->szK / n) + 2);
+        if (n == 1 || cost < best) {
+            best = cost;
+            nchunk = n;
+        }
+    }
     const int kchunk = c->szK / nchunk;
-    const dim3 grid((unsigned)ntiles * (unsigned)nchunk), block(HTI * TJ);
+    const int ntiles8 = (ntiles + 7) / 8 * 8;
+    const dim3 grid((unsigned)ntiles8 * (unsigned)nchunk), block(HTI * TJ);
     const AG<T> hz{Hz, (long long)c->szK * c->S2}, wa{W, n3};
     if (wide32) {
-        hipLaunchKernelGGL((k_rhs3d_fused<TJ, T, 8>), grid, block, 0, sf::as_stream(stream), grid3(c), h,
+        hipLaunchKernelGGL((k_rhs3d_fused<TJ, T, 8>), grid, block, 0, sf::as_stream(stream), grid3(c, sizeof(T)), h,
                            A{fomn, c->S2}, hz, wa, BC, ru, rv, end, cor ? 1 : 0, adv ? 1 : 0, tiles_i, ntiles,
-                           kchunk, nchunk);
+                           ntiles8, kchunk, nchunk);
     } else {
         constexpr int WPE = sizeof(T) == 8 ? 6 : 4;   // FP64: at most 80 VGPRs, three workgroups per CU
-        hipLaunchKernelGGL((k_rhs3d_fused<TJ, T, WPE>), grid, block, 0, sf::as_stream(stream), grid3(c), h,
+        hipLaunchKernelGGL((k_rhs3d_fused<TJ, T, WPE>), grid, block, 0, sf::as_stream(stream), grid3(c, sizeof(T)), h,
                            A{fomn, c->S2}, hz, wa, BC, ru, rv, end, cor ? 1 : 0, adv ? 1 : 0, tiles_i, ntiles,
-                           kchunk, nchunk);
+                           ntiles8, kchunk, nchunk);
     }
     return sf::check_launch("sf_rhs3d");
 }
@@ -1409,7 +1429,7 @@ extern "C" int sf_set_maxflux(sf_ctx *c, const double *u, const double *v, doubl
 {
     CTX3(c);
     SF_REQUIRE(u && v && Huon && Hvom && Hz, "sf_set_maxflux: null field");
-    LAUNCH_COLUMNS(k_set_maxflux<double>, c, stream, grid3(c), u, v, Huon, Hvom, Hz);
+    LAUNCH_COLUMNS(k_set_maxflux<double>, c, stream, grid3(c, sizeof(double)), u, v, Huon, Hvom, Hz);
 }
 
 extern "C" int sf_set_maxflux_f32(sf_ctx *c, const float *u, const float *v, float *Huon, float *Hvom,
@@ -1417,7 +1437,7 @@ extern "C" int sf_set_maxflux_f32(sf_ctx *c, const float *u, const float *v, flo
 {
     CTX3(c);
     SF_REQUIRE(u && v && Huon && Hvom && Hz, "sf_set_maxflux_f32: null field");
-    LAUNCH_COLUMNS(k_set_maxflux<float>, c, stream, grid3(c), u, v, Huon, Hvom, Hz);
+    LAUNCH_COLUMNS(k_set_maxflux<float>, c, stream, grid3(c, sizeof(float)), u, v, Huon, Hvom, Hz);
 }
 
 template <class T>
@@ -1427,12 +1447,12 @@ static int omega_launch(sf_ctx *c, T *W, const T *Huon, const T *Hvom, const T *
     const long long n3 = (c->szK + 1LL) * c->S2;
     const AG<T> hu{Huon, n3}, hv{Hvom, n3};
     if (c->szK <= 16) {
-        LAUNCH_COLUMNS((k_omega_reg<16, T>), c, stream, grid3(c), W, hu, hv, z_w, BC);
+        LAUNCH_COLUMNS((k_omega_reg<16, T>), c, stream, grid3(c, sizeof(T)), W, hu, hv, z_w, BC);
     }
     if (c->szK <= 32) {
-        LAUNCH_COLUMNS((k_omega_reg<32, T>), c, stream, grid3(c), W, hu, hv, z_w, BC);
+        LAUNCH_COLUMNS((k_omega_reg<32, T>), c, stream, grid3(c, sizeof(T)), W, hu, hv, z_w, BC);
     }
-    LAUNCH_COLUMNS((k_omega_reg<64, T>), c, stream, grid3(c), W, hu, hv, z_w, BC);
+    LAUNCH_COLUMNS((k_omega_reg<64, T>), c, stream, grid3(c, sizeof(T)), W, hu, hv, z_w, BC);
 }
 
 extern "C" int sf_omega(sf_ctx *c, double *W, const double *Huon, const double *Hvom, const double *z_w,
@@ -1442,7 +1462,7 @@ extern "C" int sf_omega(sf_ctx *c, double *W, const double *Huon, const double *
     SF_REQUIRE(W && Huon && Hvom && z_w && BC, "sf_omega: null field");
     if (c->szK <= 64) return omega_launch<double>(c, W, Huon, Hvom, z_w, BC, stream);
     const long long n3 = (c->szK + 1LL) * c->S2;
-    LAUNCH_COLUMNS(k_omega, c, stream, grid3(c), W, A{Huon, n3}, A{Hvom, n3}, z_w, BC);
+    LAUNCH_COLUMNS(k_omega, c, stream, grid3(c, sizeof(double)), W, A{Huon, n3}, A{Hvom, n3}, z_w, BC);
 }
 
 extern "C" int sf_omega_f32(sf_ctx *c, float *W, const float *Huon, const float *Hvom, const float *z_w,
@@ -1461,7 +1481,7 @@ extern "C" int sf_set_depth(sf_ctx *c, int32_t Vtransform, const double *Zt_avg1
     CTX3(c);
     SF_REQUIRE(Zt_avg1 && z_w && z_r && h && Hz && sc_r && sc_w && Cs_r && Cs_w, "sf_set_depth: null field");
     SF_REQUIRE(Vtransform == 1 || Vtransform == 2, "sf_set_depth: Vtransform=%d", Vtransform);
-    LAUNCH_COLUMNS(k_set_depth<double>, c, stream, grid3(c), Vtransform, Zt_avg1, z_w, z_r, h, hc, Hz, sc_r, sc_w,
+    LAUNCH_COLUMNS(k_set_depth<double>, c, stream, grid3(c, sizeof(double)), Vtransform, Zt_avg1, z_w, z_r, h, hc, Hz, sc_r, sc_w,
                    Cs_r, Cs_w);
 }
 
@@ -1472,34 +1492,34 @@ extern "C" int sf_set_depth_f32(sf_ctx *c, int32_t Vtransform, const double *Zt_
     CTX3(c);
     SF_REQUIRE(Zt_avg1 && z_w && z_r && h && Hz && sc_r && sc_w && Cs_r && Cs_w, "sf_set_depth_f32: null field");
     SF_REQUIRE(Vtransform == 1 || Vtransform == 2, "sf_set_depth_f32: Vtransform=%d", Vtransform);
-    LAUNCH_COLUMNS(k_set_depth<float>, c, stream, grid3(c), Vtransform, Zt_avg1, z_w, z_r, h, hc, Hz, sc_r, sc_w,
+    LAUNCH_COLUMNS(k_set_depth<float>, c, stream, grid3(c, sizeof(float)), Vtransform, Zt_avg1, z_w, z_r, h, hc, Hz, sc_r, sc_w,
                    Cs_r, Cs_w);
 }
 
 extern "C" int sf_set_zeta(sf_ctx *c, double *zeta_t1, double *zeta_t2, const double *Zt_avg1, void *stream)
 {
     SF_REQUIRE(c && zeta_t1 && zeta_t2 && Zt_avg1, "sf_set_zeta: null argument");
-    LAUNCH_COLUMNS(k_set_zeta<double>, c, stream, grid3(c), zeta_t1, zeta_t2, Zt_avg1);
+    LAUNCH_COLUMNS(k_set_zeta<double>, c, stream, grid3(c, sizeof(double)), zeta_t1, zeta_t2, Zt_avg1);
 }
 
 extern "C" int sf_set_zeta_f32(sf_ctx *c, float *zeta_t1, float *zeta_t2, const double *Zt_avg1, void *stream)
 {
     SF_REQUIRE(c && zeta_t1 && zeta_t2 && Zt_avg1, "sf_set_zeta_f32: null argument");
-    LAUNCH_COLUMNS(k_set_zeta<float>, c, stream, grid3(c), zeta_t1, zeta_t2, Zt_avg1);
+    LAUNCH_COLUMNS(k_set_zeta<float>, c, stream, grid3(c, sizeof(float)), zeta_t1, zeta_t2, Zt_avg1);
 }
 
 extern "C" int sf_set_lateral_uv_bcs(sf_ctx *c, double t, double *u, double *v, const int32_t *uType,
                                      const int32_t *vType, void *stream)
 {
     SF_REQUIRE(c && u && v && uType && vType, "sf_set_lateral_uv_bcs: null argument");
-    LAUNCH_COLUMNS(k_lateral_uv<double>, c, stream, grid3(c), t, u, v, uType, vType);
+    LAUNCH_COLUMNS(k_lateral_uv<double>, c, stream, grid3(c, sizeof(double)), t, u, v, uType, vType);
 }
 
 extern "C" int sf_set_lateral_uv_bcs_f32(sf_ctx *c, double t, float *u, float *v, const int32_t *uType,
                                          const int32_t *vType, void *stream)
 {
     SF_REQUIRE(c && u && v && uType && vType, "sf_set_lateral_uv_bcs_f32: null argument");
-    LAUNCH_COLUMNS(k_lateral_uv<float>, c, stream, grid3(c), t, u, v, uType, vType);
+    LAUNCH_COLUMNS(k_lateral_uv<float>, c, stream, grid3(c, sizeof(float)), t, u, v, uType, vType);
 }
 
 // step3d_UV: columns of up to 64 levels on chip (k_step3d_uv_col), deeper ones through the
@@ -1508,14 +1528,14 @@ template <class T>
 static int step3d_uv_launch(sf_ctx *c, const UVArgs<T> &a, double cff, double lambda, double Dt, void *stream)
 {
     if (c->szK > SF_STEP3D_REG_LEVELS) {
-        LAUNCH_COLUMNS(k_step3d_uv<T>, c, stream, grid3(c), a, cff, lambda, Dt);
+        LAUNCH_COLUMNS(k_step3d_uv<T>, c, stream, grid3(c, sizeof(T)), a, cff, lambda, Dt);
     }
     SF_REQUIRE(c->S2 * sizeof(T) < (1ull << 32), "sf_step3d_uv: a level of %lld points exceeds 4 GiB", c->S2);
     // by_levels: the fewest levels an instance holds; registers and LDS of the unused ones
     // would cost waves (FP64: 3 waves per SIMD up to 24 levels, 2 up to 48, 1 to 64)
     return by_levels(c->szK, [&](auto nmax) {
-        hipLaunchKernelGGL((k_step3d_uv_col<T, decltype(nmax)::value>), dim3(sf::grid1d(c->S2, 64), 2), dim3(64), 0,
-                           sf::as_stream(stream), grid3(c), a, cff, lambda, Dt);
+        hipLaunchKernelGGL((k_step3d_uv_col<T, decltype(nmax)::value>), dim3(2 * sf::column_grid(c->S2, 64)), dim3(64), 0,
+                           sf::as_stream(stream), grid3(c, sizeof(T)), a, cff, lambda, Dt);
         return sf::check_launch("sf_step3d_uv");
     });
 }
@@ -1564,7 +1584,7 @@ template <class T>
 int couple_rufrc_launch(sf_ctx *c, const void *ru, const void *rv, const void *u, const void *v, const double *sustr,
                         const double *svstr, double rdrg, double *rufrc, double *rvfrc, void *stream)
 {
-    LAUNCH_COLUMNS(k_couple_rufrc<T>, c, stream, grid3(c), (const T *)ru, (const T *)rv, (const T *)u, (const T *)v,
+    LAUNCH_COLUMNS(k_couple_rufrc<T>, c, stream, grid3(c, sizeof(T)), (const T *)ru, (const T *)rv, (const T *)u, (const T *)v,
                    sustr, svstr, rdrg, rufrc, rvfrc);
 }
 
@@ -1580,11 +1600,11 @@ int step3d_uv_coupled_launch(sf_ctx *c, const sf_uv_coupled *p, double lambda, d
     const bool fits = (unsigned long long)(c->szK + 1) * (unsigned long long)c->S2 * sizeof(T) < (1ull << 32);
     if (fits && c->szK <= SF_STEP3D_REG_LEVELS)
         return by_levels(c->szK, [&](auto nmax) {
-            hipLaunchKernelGGL((k_step3d_uv_coupled_col<T, decltype(nmax)::value>), dim3(sf::grid1d(c->S2, 64), 2),
-                               dim3(64), 0, sf::as_stream(stream), grid3(c), a, lambda, Dt);
+            hipLaunchKernelGGL((k_step3d_uv_coupled_col<T, decltype(nmax)::value>), dim3(2 * sf::column_grid(c->S2, 64)),
+                               dim3(64), 0, sf::as_stream(stream), grid3(c, sizeof(T)), a, lambda, Dt);
             return sf::check_launch("sf_step3d_uv_coupled");
         });
-    LAUNCH_COLUMNS(k_step3d_uv_coupled<T>, c, stream, grid3(c), a, lambda, Dt);
+    LAUNCH_COLUMNS(k_step3d_uv_coupled<T>, c, stream, grid3(c, sizeof(T)), a, lambda, Dt);
 }
 
 }  // namespace
