@@ -2,15 +2,23 @@
 // passes of nonlinear/step2d.py:23-127) in one tiled kernel plus one small kernel
 // over the points that computeMomentumPred masks.
 //
-// Layout and tiling.  A workgroup of 256 threads owns a TI x TJ tile T of rho points
-// (TI along xi, the contiguous axis) and stages what it needs in LDS on the tile
-// plus a 2-point halo (R2); predictor quantities are recomputed on the 1-point halo
-// (R1) instead of being exchanged between workgroups.  Each HBM field is read or
-// written once per substep (halo re-reads hit L2), so the kernel is bound by HBM
-// bandwidth.  Workgroup ids are remapped so that each XCD walks a contiguous band
-// of tiles (its L2 then serves the halo re-reads).
+// Layout and tiling.  A workgroup owns a TI x TJ tile T of rho points (TI along xi, the
+// contiguous axis) and stages what it needs in LDS on the tile plus a 2-point halo (R2);
+// predictor quantities are recomputed on the 1-point halo (R1) instead of being exchanged
+// between workgroups.  Each HBM field is read or written once per substep (halo re-reads
+// hit L2).  Workgroup ids are remapped so that each XCD walks a contiguous band of tiles
+// (its L2 then serves the halo re-reads).
 //
-// Stages (each followed by a barrier), with the reference code they restate:
+// What bounds it: HBM traffic on large grids, the chain of stages on small ones.  The
+// threads first take the tile's points, a row per wave, then the halo ring, so that ring
+// points carry no registers for what only the tile needs; the boundary maps and the values
+// that only boundary points read come with the first loads; tiles away from the boundary
+// skip the map stages and their barriers.  Per substep, against 256 threads walking the
+// frame row by row with the boundary's loads where they were used: FP64 129 x 97 15.0 ->
+// 7.2 us, 388 x 260 16.1 -> 7.9, 1023 x 511 32.7 -> 23.7 (92 MB, 3.9 TB/s), 4096 x 2048
+// 377 -> 298 (1.5 GB, 5.0 TB/s); FP32 388 x 260 14.6 -> 6.4, 1023 x 511 21.1 -> 17.1.
+//
+// Stages (a barrier between them), with the reference code they restate:
 //   A  D1 = zeta_t1 + h, h, zeta_t0 on R2
 //   B  FX = (ubar_t1*RtoU(D1))*on_u, FY = (vbar_t1*RtoV(D1))*om_v  (mod_cppkernels.cpp:80-128)
 //   C  predicted zeta before BC on R1: zeta_t0 + Dt*rzeta          (cpp:133-150)
@@ -40,16 +48,18 @@
 #include "step2d_fused.h"
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 namespace {
 
 constexpr int TI = SF_FUSED_TI;
 constexpr int TJ = SF_FUSED_TJ;
-constexpr int NT = 256;
 constexpr int W2 = TI + 4;           // R2 frame width
 constexpr int H2 = TJ + 4;
 constexpr int N2 = W2 * H2;
+constexpr int NCORE = TI * TJ;
+constexpr int kCUs = 256;
 
 // dense boundary-code values
 constexpr int kKeep = -1;
@@ -94,9 +104,12 @@ __device__ __forceinline__ T am3(T x, T Dt, T r2, T r1, T r0)
     return x + Dt * (AM3_2 * r2 + AM3_1 * r1 + AM3_0 * r0);
 }
 
-__device__ __forceinline__ bool is_masked(long long f, int stride)
+// The points computeMomentumPred skips: f % stride == 0 or f < stride.  sf_step2d_check_maps
+// takes only strides that divide szI, so f % stride is i % stride.
+__device__ __forceinline__ bool is_masked(int i, int j, const Params &P)
 {
-    return (f % stride == 0) || (f / stride == 0);
+    if (P.fold_masked) return i == 0 || j == 0;
+    return (j == 0 && i < P.q5_stride) || i % P.q5_stride == 0;
 }
 
 // NTS: outputs written with streaming (non-temporal) stores and the FP64 averages read
@@ -114,10 +127,33 @@ __device__ __forceinline__ double ldavg(const double *p)
     return *p;
 }
 
+// Point p of a tile's frame: the TI*TJ tile points first (one row of the tile per wave,
+// so the bulk loads and all stores are whole lines), then the two-point ring around them.
+__device__ __forceinline__ void frame_point(int p, int *li, int *lj)
+{
+    if (p < NCORE) {
+        *li = 2 + p % TI;
+        *lj = 2 + p / TI;
+        return;
+    }
+    p -= NCORE;
+    if (p < 4 * W2) {                      // two rows below, two rows above
+        const int row = p / W2;
+        *li = p % W2;
+        *lj = row < 2 ? row : TJ + row;
+    } else {                               // two columns left, two right
+        p -= 4 * W2;
+        const int col = p & 3;
+        *li = col < 2 ? col : TI + col;
+        *lj = 2 + (p >> 2);
+    }
+}
+
 // VC: a velocity boundary map copies from neighbours (gradient boundaries).  Stage E
 // then keeps the predicted velocities before the map in two more LDS planes, and a
 // destination takes its source's value from them after a barrier.
-template <typename T, bool NTS, bool VC>
+// NT: threads of a workgroup; each holds the frame points tid, tid + NT, ...
+template <typename T, int NT, bool NTS, bool VC>
 __global__ __launch_bounds__(NT) void k_step2d_fused(Fields<T> F, Params P)
 {
     // six LDS planes on the R2 frame, reused as their contents die:
@@ -135,35 +171,51 @@ __global__ __launch_bounds__(NT) void k_step2d_fused(Fields<T> F, Params P)
 
     const int szI = P.szI, szJ = P.szJ;
     const int nblk = P.tiles_i * P.tiles_j;
-    int b = blockIdx.x;
-    if ((nblk & 7) == 0) b = (blockIdx.x & 7) * (nblk >> 3) + (blockIdx.x >> 3);
+    // workgroup x runs on XCD x % 8: each takes a run of nblk / 8 tiles, the first
+    // nblk % 8 of them one more
+    const int xcd = blockIdx.x & 7, nx = nblk & 7;
+    const int b = xcd * (nblk >> 3) + (xcd < nx ? xcd : nx) + (blockIdx.x >> 3);
     const int ti = b % P.tiles_i, tj = b / P.tiles_i;
     const int i0 = ti * TI - P.off_i, j0 = tj * TJ - P.off_j;
     const int gi0 = i0 - 2, gj0 = j0 - 2;   // global coords of the R2 frame origin
     const int tid = threadIdx.x;
     const T Dt = T(P.Dt);
+    // no point of R1 lies on the boundary band: nothing is mapped in this tile
+    const bool calm = gi0 + 1 >= 2 && gi0 + TI + 2 < szI - 2 && gj0 + 1 >= 2 && gj0 + TJ + 2 < szJ - 2;
 
     auto inside = [&](int i, int j) { return i >= 0 && i < szI && j >= 0 && j < szJ; };
     auto interior = [&](int i, int j) { return i > 0 && i < szI - 1 && j > 0 && j < szJ - 1; };
     auto band = [&](int i, int j) { return i <= 1 || i >= szI - 2 || j <= 1 || j >= szJ - 2; };
 
-    // Every thread owns the same R2-frame points r = tid + k*NT in all stages, so
-    // per-point inputs stay in registers; only neighbour accesses go through LDS.
+    // Every thread owns the same frame points p = tid + k*NT in all stages, so per-point
+    // inputs stay in registers; only neighbour accesses go through LDS.
     constexpr int KP = (N2 + NT - 1) / NT;
+    int lis[KP], ljs[KP];
     T ub1[KP], vb1[KP], onu[KP], omv[KP], pmr[KP], pnr[KP];
     T rz0[KP], rz2[KP], up[KP], vp[KP], z0r[KP], hr[KP], zp[KP], dU1[KP], dV1[KP];
     double zt[KP], du[KP], dv[KP];
+    // what only boundary points read: loaded with the rest, or a tile on the boundary
+    // would wait for memory once more in each stage
+    T rz1[KP], ru1[KP], rv1[KP], ru0[KP];
+    int cz[KP], cu[KP], cv[KP];
+    auto used = [&](int k) { return (k + 1) * NT <= N2 || tid + k * NT < N2; };
+    auto on_r1 = [&](int k) { return lis[k] >= 1 && lis[k] <= TI + 2 && ljs[k] >= 1 && ljs[k] <= TJ + 2; };
+    auto on_e = [&](int k) { return lis[k] >= 2 && lis[k] <= TI + 2 && ljs[k] >= 2 && ljs[k] <= TJ + 2; };
+    auto core = [&](int k) { return (k + 1) * NT <= NCORE || tid + k * NT < NCORE; };
 
-    // ---- prologue: every bulk load of the tile, issued back to back ----------------
+    // ---- prologue: every load of the tile, issued back to back ---------------------
 #pragma unroll
     for (int k = 0; k < KP; k++) {
-        const int r = tid + k * NT;
-        const int li = r % W2, lj = r / W2;
-        const int i = gi0 + li, j = gj0 + lj;
+        if (!used(k)) continue;
+        frame_point(tid + k * NT, &lis[k], &ljs[k]);
+        const int r = lidx(lis[k], ljs[k]);
+        const int i = gi0 + lis[k], j = gj0 + ljs[k];
         T z1 = T(0), hh = T(0), z0 = T(0);
         ub1[k] = vb1[k] = onu[k] = omv[k] = pmr[k] = pnr[k] = rz0[k] = rz2[k] = T(0);
+        up[k] = vp[k] = zp[k] = rz1[k] = ru1[k] = rv1[k] = ru0[k] = T(0);
+        cz[k] = cu[k] = cv[k] = kKeep;
         zt[k] = du[k] = dv[k] = 0.0;
-        if (r < N2 && inside(i, j)) {
+        if (inside(i, j)) {
             const long long f = (long long)j * szI + i;
             z1 = F.zeta_t1[f];
             hh = F.h[f];
@@ -172,11 +224,11 @@ __global__ __launch_bounds__(NT) void k_step2d_fused(Fields<T> F, Params P)
             vb1[k] = F.vbar_t1[f];
             onu[k] = F.on_u[f];
             omv[k] = F.om_v[f];
-            if (li >= 1 && li <= TI + 2 && lj >= 1 && lj <= TJ + 2) {
+            if (on_r1(k)) {
                 pmr[k] = F.pm[f];
                 pnr[k] = F.pn[f];
             }
-            if (li >= 2 && li <= TI + 1 && lj >= 2 && lj <= TJ + 1) {
+            if (core(k)) {
                 rz0[k] = F.rzeta_t0[f];
                 rz2[k] = F.rzeta_t2[f];
                 if (interior(i, j)) {
@@ -185,26 +237,47 @@ __global__ __launch_bounds__(NT) void k_step2d_fused(Fields<T> F, Params P)
                     dv[k] = ldavg<NTS>(F.DV_avg1 + f);
                 }
             }
+            if (on_r1(k) && band(i, j)) {
+                cz[k] = F.bc_zeta[f];
+                // computeZetaRHS never writes non-interior points
+                if (!interior(i, j)) rz1[k] = F.rzeta_t1[f];
+                // computeZetaPred leaves column 0 and row 0 alone (the buffer keeps its
+                // value).  Outside the own tile such points are boundary-map
+                // destinations whose halo copies are never consumed: not read.
+                if ((i == 0 || j == 0) && core(k)) zp[k] = F.zeta_t2[f];
+            }
+            if (on_e(k)) {
+                if (band(i, j)) {
+                    cu[k] = F.bc_ubar[f];
+                    cv[k] = F.bc_vbar[f];
+                    if (!interior(i, j)) {   // never written there either
+                        ru1[k] = F.rubar_t1[f];
+                        rv1[k] = F.rvbar_t1[f];
+                    }
+                }
+                if (is_masked(i, j, P)) {    // the t2 buffers keep their values
+                    up[k] = F.ubar_t2[f];
+                    vp[k] = F.vbar_t2[f];
+                    if (P.fold_masked && core(k)) ru0[k] = F.rubar_t0[f];
+                }
+            }
         }
         z0r[k] = z0;
         hr[k] = hh;
-        if (r < N2) {
-            sD1[r] = z1 + hh;
-            sH[r] = hh;
-        }
+        sD1[r] = z1 + hh;
+        sH[r] = hh;
     }
     __syncthreads();
 
     // ---- B: face fluxes of the t1 state (computeZetaRHS, cpp:80-128) ---------------
 #pragma unroll
     for (int k = 0; k < KP; k++) {
-        const int r = tid + k * NT;
-        if (r >= N2) continue;
-        const int li = r % W2, lj = r / W2;
-        const int i = gi0 + li, j = gj0 + lj;
+        if (!used(k)) continue;
+        const int r = lidx(lis[k], ljs[k]);
+        const int i = gi0 + lis[k], j = gj0 + ljs[k];
         T fx = T(0), fy = T(0);
         dU1[k] = dV1[k] = T(0);
-        if (li >= 1 && lj >= 1 && inside(i, j)) {
+        if (lis[k] >= 1 && ljs[k] >= 1 && inside(i, j)) {
             const T D = sD1[r];
             // ubar_t1*RtoU(D1) is also the first term of computeMomentumPred's
             // numerator (cpp:183): kept for stage E.  Row 0 reads row -1 as zero
@@ -222,84 +295,54 @@ __global__ __launch_bounds__(NT) void k_step2d_fused(Fields<T> F, Params P)
     __syncthreads();
 
     // ---- C: predicted zeta before BC on R1 (computeZetaPred, cpp:133-150) ----------
+    const T w = T(2.0 / 5.0);
+    const T a = T(1) - w;
+    auto put_pred = [&](int k, int r) {
+        sD2[r] = zp[k] + hr[k];
+        sGZ[r] = a * zp[k] + w * z0r[k];
+    };
 #pragma unroll
     for (int k = 0; k < KP; k++) {
-        const int r = tid + k * NT;
-        if (r >= N2) continue;
-        const int li = r % W2, lj = r / W2;
-        if (li < 1 || li > TI + 2 || lj < 1 || lj > TJ + 2) continue;
-        const int i = gi0 + li, j = gj0 + lj;
-        T zq = T(0);
-        if (inside(i, j)) {
-            const long long f = (long long)j * szI + i;
-            if (i == 0 || j == 0) {
-                // computeZetaPred leaves column 0 and row 0 alone (the buffer keeps its
-                // value).  Outside the own tile such points are boundary-map
-                // destinations whose halo copies are never consumed: not read.
-                if (li >= 2 && li <= TI + 1 && lj >= 2 && lj <= TJ + 1) zq = F.zeta_t2[f];
-            } else {
-                T rz;
-                if (interior(i, j))
-                    rz = (((sFX[r + 1] - sFX[r]) + (sFY[r + W2] - sFY[r])) * pmr[k]) * pnr[k];
-                else
-                    rz = F.rzeta_t1[f];   // computeZetaRHS never writes non-interior points
-                zq = z0r[k] + Dt * rz;
-            }
+        if (!used(k) || !on_r1(k)) continue;
+        const int r = lidx(lis[k], ljs[k]);
+        const int i = gi0 + lis[k], j = gj0 + ljs[k];
+        if (inside(i, j) && i != 0 && j != 0) {
+            T rz = rz1[k];
+            if (interior(i, j))
+                rz = (((sFX[r + 1] - sFX[r]) + (sFY[r + W2] - sFY[r])) * pmr[k]) * pnr[k];
+            zp[k] = z0r[k] + Dt * rz;
         }
-        sZq[r] = zq;
+        if (calm) put_pred(k, r);
+        else sZq[r] = zp[k];
     }
     __syncthreads();
 
-    // ---- D: zeta boundary map on R1 (zetabc.py:5-12) --------------------------------
-#pragma unroll
-    for (int k = 0; k < KP; k++) {
-        const int r = tid + k * NT;
-        if (r >= N2) continue;
-        const int li = r % W2, lj = r / W2;
-        if (li < 1 || li > TI + 2 || lj < 1 || lj > TJ + 2) continue;
-        const int i = gi0 + li, j = gj0 + lj;
-        T z = sZq[r];
-        if (inside(i, j) && band(i, j)) {
-            const int s = F.bc_zeta[(long long)j * szI + i];
-            if (s >= 0) z = sZq[lidx(s % szI - gi0, s / szI - gj0)];
-        }
-        zp[k] = z;
-    }
-    __syncthreads();   // P1's D1 and P5's pre-map values are read above: write after
-    {
-        const T w = T(2.0 / 5.0);
-        const T a = T(1) - w;
+    // ---- D: zeta boundary map on R1 (zetabc.py:5-12); P1's D1 was last read in B ----
+    if (!calm) {
 #pragma unroll
         for (int k = 0; k < KP; k++) {
-            const int r = tid + k * NT;
-            if (r >= N2) continue;
-            const int li = r % W2, lj = r / W2;
-            if (li < 1 || li > TI + 2 || lj < 1 || lj > TJ + 2) continue;
-            sD2[r] = zp[k] + hr[k];
-            sGZ[r] = a * zp[k] + w * z0r[k];
+            if (!used(k) || !on_r1(k)) continue;
+            if (cz[k] >= 0) zp[k] = sZq[lidx(cz[k] % szI - gi0, cz[k] / szI - gj0)];
+            put_pred(k, lidx(lis[k], ljs[k]));
         }
+        __syncthreads();
     }
-    __syncthreads();
 
     // ---- E: momentum RHS and predicted velocities on T + right column + top row
     //      (cpp:12-42, cpp:155-186, barotropicVelocityBC.py:7-31); then the corrector's
     //      face fluxes PX/PY and time averages (cpp:80-128) ---------------------------
-    const T w = T(2.0 / 5.0);
-    const T a = T(1) - w;
     const T gc = T(10.0);
     const double cff1 = P.cff1;
     // the boundary map at (i, j), the corrector's face fluxes of the predicted state and
     // the time averages; VC copies read the pre-map values of E in P7 / P8
-    auto e_tail = [&](int k, int r, int i, int j, long long f, bool inT, T u2, T v2) {
-        if (band(i, j)) {
-            const int cu = F.bc_ubar[f], cv = F.bc_vbar[f];
-            if (cu == kZero) u2 = T(0);
-            else if (cu == kClamp) u2 = T(P.clamp);
-            else if (VC && cu >= 0) u2 = P7[lidx(cu % szI - gi0, cu / szI - gj0)];
-            if (cv == kZero) v2 = T(0);
-            else if (cv == kClamp) v2 = T(P.clamp);
-            else if (VC && cv >= 0) v2 = P8[lidx(cv % szI - gi0, cv / szI - gj0)];
-        }
+    auto e_tail = [&](int k, int r, int i, int j, long long f) {
+        T u2 = up[k], v2 = vp[k];
+        if (cu[k] == kZero) u2 = T(0);
+        else if (cu[k] == kClamp) u2 = T(P.clamp);
+        else if (VC && cu[k] >= 0) u2 = P7[lidx(cu[k] % szI - gi0, cu[k] / szI - gj0)];
+        if (cv[k] == kZero) v2 = T(0);
+        else if (cv[k] == kClamp) v2 = T(P.clamp);
+        else if (VC && cv[k] >= 0) v2 = P8[lidx(cv[k] % szI - gi0, cv[k] / szI - gj0)];
         up[k] = u2;
         vp[k] = v2;
         // corrector fluxes of the predicted state: DU = ubar*RtoU(D), DV = vbar*RtoV(D)
@@ -308,7 +351,7 @@ __global__ __launch_bounds__(NT) void k_step2d_fused(Fields<T> F, Params P)
         const T Dd = sD2[r - W2];
         const T DU = u2 * ((D + Dl) * T(0.5));
         const T DV = v2 * ((D + Dd) * T(0.5));
-        if (inT && interior(i, j)) {
+        if (core(k) && interior(i, j)) {
             stv<NTS>(F.Zt_avg1 + f, zt[k] + cff1 * (double)zp[k]);
             stv<NTS>(F.DU_avg1 + f, du[k] + (cff1 * (double)DU) * (double)onu[k]);
             stv<NTS>(F.DV_avg1 + f, dv[k] + (cff1 * (double)DV) * (double)omv[k]);
@@ -318,52 +361,33 @@ __global__ __launch_bounds__(NT) void k_step2d_fused(Fields<T> F, Params P)
     };
 #pragma unroll
     for (int k = 0; k < KP; k++) {
-        const int r = tid + k * NT;
-        if (r >= N2) continue;
-        const int li = r % W2, lj = r / W2;
-        up[k] = vp[k] = T(0);
-        if (li < 2 || li > TI + 2 || lj < 2 || lj > TJ + 2) continue;
-        const int i = gi0 + li, j = gj0 + lj;
+        if (!used(k) || !on_e(k)) continue;
+        const int r = lidx(lis[k], ljs[k]);
+        const int i = gi0 + lis[k], j = gj0 + ljs[k];
         if (inside(i, j)) {
             const long long f = (long long)j * szI + i;
-            const bool inT = li <= TI + 1 && lj <= TJ + 1;
-            T u2, v2;
-            if (!is_masked(f, P.q5_stride)) {
-                T ru, rv;
-                if (interior(i, j)) {
-                    const T gz = sGZ[r];
-                    const T gzl = sGZ[r - 1];
-                    const T gzd = sGZ[r - W2];
-                    const T hu = (sH[r] + sH[r - 1]) * T(0.5);
-                    const T hv = (sH[r] + sH[r - W2]) * T(0.5);
-                    ru = (gc * onu[k]) * (hu * (gz - gzl) + T(0.5) * (gz * gz - gzl * gzl));
-                    rv = (gc * omv[k]) * (hv * (gz - gzd) + T(0.5) * (gz * gz - gzd * gzd));
-                    if (inT) stv<NTS>(F.rubar_t1 + f, ru);
-                } else {
-                    ru = F.rubar_t1[f];   // never written at non-interior points
-                    rv = F.rvbar_t1[f];
-                }
+            const bool masked = is_masked(i, j, P);
+            T ru = ru1[k], rv = rv1[k];
+            if (interior(i, j)) {
+                const T gz = sGZ[r];
+                const T gzl = sGZ[r - 1];
+                const T gzd = sGZ[r - W2];
+                const T hu = (sH[r] + sH[r - 1]) * T(0.5);
+                const T hv = (sH[r] + sH[r - W2]) * T(0.5);
+                ru = (gc * onu[k]) * (hu * (gz - gzl) + T(0.5) * (gz * gz - gzl * gzl));
+                rv = (gc * omv[k]) * (hv * (gz - gzd) + T(0.5) * (gz * gz - gzd * gzd));
+                if (core(k)) stv<NTS>(F.rubar_t1 + f, ru);
+            }
+            if (!masked) {
                 const T D2 = sD2[r], D2l = sD2[r - 1], D2d = sD2[r - W2];
-                u2 = (dU1[k] + ((Dt * ru) * pmr[k]) * pnr[k]) / ((D2 + D2l) * T(0.5));
-                v2 = (dV1[k] + ((Dt * rv) * pmr[k]) * pnr[k]) / ((D2 + D2d) * T(0.5));
-            } else {
-                // masked: the t2 buffer keeps its value
-                u2 = F.ubar_t2[f];
-                v2 = F.vbar_t2[f];
-                if (interior(i, j) && inT) {
-                    const T gz = sGZ[r];
-                    const T gzl = sGZ[r - 1];
-                    const T hu = (sH[r] + sH[r - 1]) * T(0.5);
-                    stv<NTS>(F.rubar_t1 + f, (gc * onu[k]) * (hu * (gz - gzl) + T(0.5) * (gz * gz - gzl * gzl)));
-                }
+                up[k] = (dU1[k] + ((Dt * ru) * pmr[k]) * pnr[k]) / ((D2 + D2l) * T(0.5));
+                vp[k] = (dV1[k] + ((Dt * rv) * pmr[k]) * pnr[k]) / ((D2 + D2d) * T(0.5));
             }
             if constexpr (VC) {
-                up[k] = u2;   // the map is applied after the barrier below
-                vp[k] = v2;
-                P7[r] = u2;
-                P8[r] = v2;
+                P7[r] = up[k];   // the map is applied after the barrier below
+                P8[r] = vp[k];
             } else {
-                e_tail(k, r, i, j, f, inT, u2, v2);
+                e_tail(k, r, i, j, f);
             }
         } else {
             sPX[r] = T(0);
@@ -374,13 +398,10 @@ __global__ __launch_bounds__(NT) void k_step2d_fused(Fields<T> F, Params P)
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < KP; k++) {
-            const int r = tid + k * NT;
-            if (r >= N2) continue;
-            const int li = r % W2, lj = r / W2;
-            if (li < 2 || li > TI + 2 || lj < 2 || lj > TJ + 2) continue;
-            const int i = gi0 + li, j = gj0 + lj;
+            if (!used(k) || !on_e(k)) continue;
+            const int i = gi0 + lis[k], j = gj0 + ljs[k];
             if (!inside(i, j)) continue;
-            e_tail(k, r, i, j, (long long)j * szI + i, li <= TI + 1 && lj <= TJ + 1, up[k], vp[k]);
+            e_tail(k, lidx(lis[k], ljs[k]), i, j, (long long)j * szI + i);
         }
     }
     __syncthreads();
@@ -388,53 +409,42 @@ __global__ __launch_bounds__(NT) void k_step2d_fused(Fields<T> F, Params P)
     // ---- F: corrector on T: rzeta (cpp:80-128), zeta AM3 (cpp:190-209) -----------------
 #pragma unroll
     for (int k = 0; k < KP; k++) {
-        const int r = tid + k * NT;
-        if (r >= N2) continue;
-        const int li = r % W2, lj = r / W2;
-        if (li < 2 || li > TI + 1 || lj < 2 || lj > TJ + 1) continue;
-        const int i = gi0 + li, j = gj0 + lj;
+        if (!used(k) || !core(k)) continue;
+        const int r = lidx(lis[k], ljs[k]);
+        const int i = gi0 + lis[k], j = gj0 + ljs[k];
         if (!inside(i, j)) continue;
         const long long f = (long long)j * szI + i;
-        T rz;
+        T rz = rz1[k];
         if (interior(i, j)) {
             rz = (((sPX[r + 1] - sPX[r]) + (sPY[r + W2] - sPY[r])) * pmr[k]) * pnr[k];
             stv<NTS>(F.rzeta_t1 + f, rz);
-        } else {
-            rz = F.rzeta_t1[f];
         }
-        sZc[r] = am3(zp[k], Dt, rz2[k], rz, rz0[k]);
+        zp[k] = am3(zp[k], Dt, rz2[k], rz, rz0[k]);
+        if (!calm) sZc[r] = zp[k];
     }
-    __syncthreads();
+    if (!calm) __syncthreads();
 
     // ---- G: zeta boundary map on T (zetabc.py:5-12), stores ------------------------
 #pragma unroll
     for (int k = 0; k < KP; k++) {
-        const int r = tid + k * NT;
-        if (r >= N2) continue;
-        const int li = r % W2, lj = r / W2;
-        if (li < 2 || li > TI + 1 || lj < 2 || lj > TJ + 1) continue;
-        const int i = gi0 + li, j = gj0 + lj;
+        if (!used(k) || !core(k)) continue;
+        const int i = gi0 + lis[k], j = gj0 + ljs[k];
         if (!inside(i, j)) continue;
         const long long f = (long long)j * szI + i;
-        T z = sZc[r];
-        if (band(i, j)) {
-            const int s = F.bc_zeta[f];
-            if (s >= 0) z = sZc[lidx(s % szI - gi0, s / szI - gj0)];
-        }
+        T z = zp[k];
+        if (cz[k] >= 0) z = sZc[lidx(cz[k] % szI - gi0, cz[k] / szI - gj0)];
         stv<NTS>(F.zeta_t2 + f, z);
-        if (!is_masked(f, P.q5_stride)) {
+        const bool masked = is_masked(i, j, P);
+        if (!masked || P.fold_masked) {
             stv<NTS>(F.ubar_t2 + f, up[k]);
             stv<NTS>(F.vbar_t2 + f, P.zero_vbar ? T(0) : vp[k]);
-        } else if (P.fold_masked) {
-            // stride == szI: the masked points are column 0 and row 0, which no
-            // other workgroup reads, so they are finished here (as k_step2d_masked)
-            stv<NTS>(F.ubar_t2 + f, up[k]);
-            stv<NTS>(F.vbar_t2 + f, P.zero_vbar ? T(0) : vp[k]);
-            stv<NTS>(F.ubar_t1 + f, am3(ub1[k], Dt, F.rubar_t1[f], F.rubar_t0[f], vb1[k]));
         }
+        // stride == szI: the masked points are column 0 and row 0, which no other
+        // workgroup reads, so they are finished here (as k_step2d_masked)
+        if (masked && P.fold_masked)
+            stv<NTS>(F.ubar_t1 + f, am3(ub1[k], Dt, ru1[k], ru0[k], vb1[k]));
     }
 }
-
 
 // Masked points (f%stride == 0 or f < stride): velocity boundary constants,
 // main3d's vbar_t2 := 0, and the AM3 update of ubar_t1 from step2d.py:120-123.
@@ -523,13 +533,19 @@ int launch(sf_ctx *c, const sf_step2d_fields *a, double dtfast, double cff1, dou
         // 11 bulk fields read and 5 written, 3 FP64 averages read and written
         const bool nts = (double)c->S2 * (16.0 * sizeof(T) + 6.0 * 8) > sf::kStreamingBytes;
         const dim3 grid(P.tiles_i * P.tiles_j);
-        if (c->bc_vel_copy) {
-            if (nts) hipLaunchKernelGGL((k_step2d_fused<T, true, true>), grid, dim3(NT), 0, s, F, P);
-            else hipLaunchKernelGGL((k_step2d_fused<T, false, true>), grid, dim3(NT), 0, s, F, P);
-        } else {
-            if (nts) hipLaunchKernelGGL((k_step2d_fused<T, true, false>), grid, dim3(NT), 0, s, F, P);
-            else hipLaunchKernelGGL((k_step2d_fused<T, false, false>), grid, dim3(NT), 0, s, F, P);
-        }
+        auto go = [&](auto kernel, int nt) { hipLaunchKernelGGL(kernel, grid, dim3(nt), 0, s, F, P); };
+        auto shape = [&](auto nt) {
+            constexpr int NT = decltype(nt)::value;
+            if (c->bc_vel_copy) nts ? go(k_step2d_fused<T, NT, true, true>, NT) : go(k_step2d_fused<T, NT, false, true>, NT);
+            else nts ? go(k_step2d_fused<T, NT, true, false>, NT) : go(k_step2d_fused<T, NT, false, false>, NT);
+        };
+        // At most one workgroup a CU: a thread per frame point, the shortest chain from
+        // loads to stores.  More tiles than CUs: two points a thread, so that two (FP64) or
+        // four (FP32) workgroups share a CU.  Per substep, 832 / 512 threads: FP64
+        // 388 x 260 (231 tiles) 7.9 / 9.1 us, 513 x 255 (288) 11.9 / 10.6, 1023 x 511
+        // (1024) 25.0 / 23.7; FP32 6.4 / 8.2, 9.3 / 8.4, 18.7 / 17.1
+        if (P.tiles_i * P.tiles_j <= kCUs) shape(std::integral_constant<int, 832>{});
+        else shape(std::integral_constant<int, 512>{});
         int rc = sf::check_launch("sf_step2d_substep (tiles)");
         if (rc != SF_OK) return rc;
     }
