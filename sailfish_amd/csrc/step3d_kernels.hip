@@ -67,6 +67,23 @@ __device__ __forceinline__ bool isInnerCell(const G3 &g, long long f)
     const long long f = (long long)sf::column_block(g.band) * blockDim.x + threadIdx.x; \
     if (f >= g.S2) return;
 
+// Kernels whose levels are independent, or meet only in a sum: a block is kColumns columns
+// by kLevelWaves waves, a wave one run of levels lo .. hi-1 out of FIRST .. LAST-1.
+// BATCH_LEVEL: level K + q of a batch, the last one again past the run's end, so that a
+// batch's loads have no branch between them and are all in flight together.
+constexpr int kColumns = 64, kLevelWaves = 4, kBatch = 4;
+#define LEVEL_WAVE_INDEX(FIRST, LAST)                                                               \
+    const long long f = (long long)sf::column_block(g.band) * kColumns + threadIdx.x % kColumns;     \
+    const int wave_ = __builtin_amdgcn_readfirstlane(threadIdx.x / kColumns);                        \
+    const int run_ = ((LAST) - (FIRST) + kLevelWaves - 1) / kLevelWaves;                             \
+    const int lo = (FIRST) + wave_ * run_ < (LAST) ? (FIRST) + wave_ * run_ : (LAST);                \
+    const int hi = lo + run_ < (LAST) ? lo + run_ : (LAST);
+#define BATCH_LEVEL(q) (long long)(K + (q) < hi ? K + (q) : hi - 1)
+#define LAUNCH_LEVEL_WAVES(kern, lds, c, stream, ...)                                               \
+    hipLaunchKernelGGL(kern, dim3(sf::column_grid((c)->S2, kColumns)), dim3(kColumns * kLevelWaves), \
+                       lds, sf::as_stream(stream), __VA_ARGS__);                                     \
+    return sf::check_launch(__func__)
+
 // ---- addCoriolis (rhs_kernels.cpp:6-35) -------------------------------------------
 template <bool CHK>
 __device__ __forceinline__ double cor_UF(const G3 &g, A fomn, A v, A Hz, long long K, long long f)
@@ -533,18 +550,35 @@ void k_rhs3d_fused(G3 g, HG<T> h, A fomn, AG<T> Hz, AG<T> Wa, const int32_t *BC,
 // ---- set_maxflux (step3D_uv.kernels.cpp:372-405) ----------------------------------
 // the fluxes are stored with streaming (non-temporal) stores: no thread of the launch
 // reads them back.  Both fluxes of a level are formed together, so Hz is read once.
+// HBM-bound; against a thread per column: FP64 700 x 400 x 32 67 -> 56 us, 386 x 258 x 40
+// 37 -> 30, 1024 x 512 x 32 (five fields, 671 MB) 135 -> 140; FP32 63 -> 54 there.
 template <class T>
-__global__ __launch_bounds__(256) void k_set_maxflux(G3 g, const T *u, const T *v, T *Huon, T *Hvom, const T *Hz)
+__global__ __launch_bounds__(kColumns * kLevelWaves) void k_set_maxflux(G3 g, const T *u, const T *v, T *Huon,
+                                                                        T *Hvom, const T *Hz)
 {
-    COLUMN_INDEX
+    LEVEL_WAVE_INDEX(0, g.N)
+    if (f >= g.S2) return;
     const bool un = isUNode(g, f), vn = isVNode(g, f);
-    if (!un && !vn) return;
+    if (!un && !vn) return;   // the others have i, j >= 1: b - 1 and b - szI exist
     const T onu = un ? T(g.on_u[f]) : T(0), omv = vn ? T(g.om_v[f]) : T(0);
-    for (long long K = 0; K < g.N; K++) {
-        const long long b = K * g.S2 + f;
-        const T hz = Hz[b];
-        if (un) __builtin_nontemporal_store((((hz + Hz[b - 1]) * T(0.5)) * u[b]) * onu, Huon + b);
-        if (vn) __builtin_nontemporal_store((((hz + Hz[b - g.szI]) * T(0.5)) * v[b]) * omv, Hvom + b);
+    for (int K = lo; K < hi; K += kBatch) {
+        T hz[kBatch], hw[kBatch], hs[kBatch], uu[kBatch], vv[kBatch];
+#pragma unroll
+        for (int q = 0; q < kBatch; q++) {
+            const long long b = BATCH_LEVEL(q) * g.S2 + f;
+            hz[q] = Hz[b];
+            hw[q] = Hz[b - 1];
+            hs[q] = Hz[b - g.szI];
+            uu[q] = u[b];
+            vv[q] = v[b];
+        }
+#pragma unroll
+        for (int q = 0; q < kBatch; q++) {
+            if (K + q >= hi) break;
+            const long long b = (K + q) * g.S2 + f;
+            if (un) __builtin_nontemporal_store((((hz[q] + hw[q]) * T(0.5)) * uu[q]) * onu, Huon + b);
+            if (vn) __builtin_nontemporal_store((((hz[q] + hs[q]) * T(0.5)) * vv[q]) * omv, Hvom + b);
+        }
     }
 }
 
@@ -572,43 +606,66 @@ __global__ __launch_bounds__(256) void k_omega(G3 g, double *W, A Hu, A Hv, cons
     W[N * S2 + f] = 0.0;
 }
 
-// omega with the column's partial sums kept in registers (N <= NMAX): W is written once
-// per level instead of written, read back and rewritten.  The values are those of
-// k_omega: the same partial sums, then W = w - (Ws * (z_w - zb)) / h.  The sums and the
-// correction are FP64 for either value type T of the fields.  (1024 x 512 x 32:
-// 138 us against 149 us for k_omega; recomputing the partial sums in a second pass
-// instead of holding them took 195 us.)
-template <int NMAX, class T>
-__global__ __launch_bounds__(256) void k_omega_reg(G3 g, T *W, AG<T> Hu, AG<T> Hv, const T *z_w,
-                                                   const int32_t *BC)
+// omega of up to 64 levels (32 KB of LDS): W is written once per level instead of written, read
+// back and rewritten.  Each wave forms the divergences of its own levels into LDS; then
+// every wave runs the column's sum over all of them, so the partial sums and W = w -
+// (Ws * (z_w - zb)) / h are those of k_omega.  FP64 sums and correction for either type T.
+// Bound by HBM once enough loads are in flight: with a thread per column and the sums in
+// registers, each level's loads waited for the level before.  FP64 1024 x 512 x 32 (four
+// fields, 537 MB) 146 -> 117 us, 386 x 258 x 40 52 -> 24; FP32 100 -> 55, 49 -> 19.
+template <class T>
+__global__ __launch_bounds__(kColumns * kLevelWaves) void k_omega_split(G3 g, T *W, const T *Hu, const T *Hv,
+                                                                        const T *z_w, const int32_t *BC)
 {
-    COLUMN_INDEX
-    if (BC[f] >= 0) return;
+    extern __shared__ double div[];   // levels 1 .. N-1 of the block's columns
+    LEVEL_WAVE_INDEX(1, g.N)
+    const bool on = f < g.S2 && BC[f] < 0;
     const long long S2 = g.S2;
-    const int N = g.N;
-    double wk[NMAX];
+    const int N = g.N, lane = threadIdx.x % kColumns;
+    auto d = [&](int K) -> double & { return div[(K - 1) * kColumns + lane]; };
+    if (on)
+        for (int K = lo; K < hi; K += kBatch) {
+            // levels up to N-1 of arrays of N+1 levels: b + szI exists
+            T u0[kBatch], u1[kBatch], v0[kBatch], v1[kBatch];
+#pragma unroll
+            for (int q = 0; q < kBatch; q++) {
+                const long long b = BATCH_LEVEL(q) * S2 + f;
+                u0[q] = Hu[b];
+                u1[q] = Hu[b + 1];
+                v0[q] = Hv[b];
+                v1[q] = Hv[b + g.szI];
+            }
+#pragma unroll
+            for (int q = 0; q < kBatch; q++)
+                if (K + q < hi)
+                    d(K + q) = ((double)u1[q] - (double)u0[q]) + ((double)v1[q] - (double)v0[q]);
+        }
+    double zb = 0.0, h = 0.0;
+    if (on) {
+        zb = (double)z_w[f];
+        h = (double)z_w[(long long)(N - 1) * S2 + f] - zb;
+    }
+    __syncthreads();
+    if (!on) return;
     double w = 0.0;
-    W[f] = T(0);
+    for (int K = 1; K < lo; K++) w = w - d(K);
+    double Ws = w;
+    for (int K = lo; K < N; K++) Ws = Ws - d(K);
+    for (int K = lo; K < hi; K += kBatch) {
+        T z[kBatch];
 #pragma unroll
-    for (int K = 1; K < NMAX; K++) {
-        wk[K] = 0.0;
-        if (K < N) {
-            const long long b = K * S2 + f;
-            w = w - (((double)r3(Hu, b + 1) - (double)r3(Hu, b)) + ((double)r3(Hv, b + g.szI) - (double)r3(Hv, b)));
-            wk[K] = w;
+        for (int q = 0; q < kBatch; q++) z[q] = z_w[BATCH_LEVEL(q) * S2 + f];
+#pragma unroll
+        for (int q = 0; q < kBatch; q++) {
+            if (K + q >= hi) break;
+            w = w - d(K + q);
+            W[(K + q) * S2 + f] = T(w - (Ws * ((double)z[q] - zb)) / h);
         }
     }
-    const double zb = (double)z_w[f];
-    const double h = (double)z_w[(long long)(N - 1) * S2 + f] - zb;
-    const double Ws = w;   // N > 1
-#pragma unroll
-    for (int K = 1; K < NMAX; K++) {
-        if (K < N) {
-            const long long b = K * S2 + f;
-            W[b] = T(wk[K] - (Ws * ((double)z_w[b] - zb)) / h);
-        }
+    if (threadIdx.x < kColumns) {
+        W[f] = T(0);
+        W[(long long)N * S2 + f] = T(0);
     }
-    W[(long long)N * S2 + f] = T(0);
 }
 
 // ---- set_depth / set_zeta (step3D_uv.kernels.cpp:225-310) -------------------------
@@ -1429,7 +1486,7 @@ extern "C" int sf_set_maxflux(sf_ctx *c, const double *u, const double *v, doubl
 {
     CTX3(c);
     SF_REQUIRE(u && v && Huon && Hvom && Hz, "sf_set_maxflux: null field");
-    LAUNCH_COLUMNS(k_set_maxflux<double>, c, stream, grid3(c, sizeof(double)), u, v, Huon, Hvom, Hz);
+    LAUNCH_LEVEL_WAVES(k_set_maxflux<double>, 0, c, stream, grid3(c, sizeof(double)), u, v, Huon, Hvom, Hz);
 }
 
 extern "C" int sf_set_maxflux_f32(sf_ctx *c, const float *u, const float *v, float *Huon, float *Hvom,
@@ -1437,22 +1494,15 @@ extern "C" int sf_set_maxflux_f32(sf_ctx *c, const float *u, const float *v, flo
 {
     CTX3(c);
     SF_REQUIRE(u && v && Huon && Hvom && Hz, "sf_set_maxflux_f32: null field");
-    LAUNCH_COLUMNS(k_set_maxflux<float>, c, stream, grid3(c, sizeof(float)), u, v, Huon, Hvom, Hz);
+    LAUNCH_LEVEL_WAVES(k_set_maxflux<float>, 0, c, stream, grid3(c, sizeof(float)), u, v, Huon, Hvom, Hz);
 }
 
 template <class T>
 static int omega_launch(sf_ctx *c, T *W, const T *Huon, const T *Hvom, const T *z_w, const int32_t *BC,
                         void *stream)
 {
-    const long long n3 = (c->szK + 1LL) * c->S2;
-    const AG<T> hu{Huon, n3}, hv{Hvom, n3};
-    if (c->szK <= 16) {
-        LAUNCH_COLUMNS((k_omega_reg<16, T>), c, stream, grid3(c, sizeof(T)), W, hu, hv, z_w, BC);
-    }
-    if (c->szK <= 32) {
-        LAUNCH_COLUMNS((k_omega_reg<32, T>), c, stream, grid3(c, sizeof(T)), W, hu, hv, z_w, BC);
-    }
-    LAUNCH_COLUMNS((k_omega_reg<64, T>), c, stream, grid3(c, sizeof(T)), W, hu, hv, z_w, BC);
+    const size_t lds = sizeof(double) * kColumns * (size_t)(c->szK - 1);
+    LAUNCH_LEVEL_WAVES(k_omega_split<T>, lds, c, stream, grid3(c, sizeof(T)), W, Huon, Hvom, z_w, BC);
 }
 
 extern "C" int sf_omega(sf_ctx *c, double *W, const double *Huon, const double *Hvom, const double *z_w,
