@@ -339,6 +339,10 @@ int sf_prsgrd(sf_ctx *ctx, int32_t precision, const void *rho, const void *z_r, 
  * have szK levels and must not alias. */
 int sf_step3d_t(sf_ctx *ctx, int32_t precision, const void *t, void *tn, const void *Huon, const void *Hvom,
                 const void *Hz_old, const void *Hz_new, double dt, void *stream);
+/* The same step of two tracers in one pass over the fluxes and thicknesses; no new array
+ * may alias another array of the call. */
+int sf_step3d_ts(sf_ctx *ctx, int32_t precision, const void *t, void *tn, const void *s, void *sn, const void *Huon,
+                 const void *Hvom, const void *Hz_old, const void *Hz_new, double dt, void *stream);
 
 /* ---------------- coupled split-explicit step (ROMS 2D/3D coupling) ---------------- */
 

@@ -35,6 +35,8 @@ def _bind():
         lib.sf_prsgrd.restype = C.c_int32
         lib.sf_step3d_t.argtypes = [P, C.c_int32, P, P, P, P, P, P, C.c_double, P]
         lib.sf_step3d_t.restype = C.c_int32
+        lib.sf_step3d_ts.argtypes = [P, C.c_int32] + [P] * 8 + [C.c_double, P]
+        lib.sf_step3d_ts.restype = C.c_int32
         lib._sf_baroclinic_bound = True
     return lib
 
@@ -87,9 +89,9 @@ class Tracers:
     def step(self, GRID, OCEAN, dt: float, stream=None):
         """Advect T and S by the step's mass fluxes from Hz_old to the current Hz."""
         c = ops.ctx_of(GRID)
-        s = _lib.stream_handle(stream)
-        for old, new in ((self.T, self.T_new), (self.S, self.S_new)):
-            _lib.check(self.lib.sf_step3d_t(c.handle, self.precision, old.data_ptr(), new.data_ptr(),
-                                            OCEAN.Huon.data_ptr(), OCEAN.Hvom.data_ptr(), self.Hz_old.data_ptr(),
-                                            GRID.Hz.data_ptr(), float(dt), s), "sf_step3d_t")
-            old.copy_(new)
+        _lib.check(self.lib.sf_step3d_ts(c.handle, self.precision, self.T.data_ptr(), self.T_new.data_ptr(),
+                                         self.S.data_ptr(), self.S_new.data_ptr(), OCEAN.Huon.data_ptr(),
+                                         OCEAN.Hvom.data_ptr(), self.Hz_old.data_ptr(), GRID.Hz.data_ptr(),
+                                         float(dt), _lib.stream_handle(stream)), "sf_step3d_ts")
+        self.T.copy_(self.T_new)
+        self.S.copy_(self.S_new)
