@@ -1,6 +1,6 @@
-"""The tracer step at the edges of its rounds of eight levels, its blocks of 64 columns and
-its ghost writes (grids with a single interior row or column): FP64, bit for bit against the
-oracle, one tracer at a time and both in one pass."""
+"""The tracer step and the pressure gradient at the edges of their rounds of eight levels, their
+blocks of 64 columns and the tracers' ghost writes (grids with a single interior row or
+column): FP64, bit for bit against the oracle, one tracer at a time and both in one pass."""
 from __future__ import annotations
 
 import sys
@@ -66,3 +66,26 @@ def test_tracer_step_levels(szI, szJ, N):
                              O.ptr(Hz_new), 60.0)
     get = lambda t: t.detach().cpu().numpy().ravel()
     assert bitwise_equal(get(tr.T), Tn) and bitwise_equal(get(tr.S), Sn) and bitwise_equal(get(one), Tn)
+
+
+@pytest.mark.parametrize("szI,szJ,N", SIZES)
+def test_pressure_gradient_levels(szI, szJ, N):
+    import torch
+    from oracle import oracle as O
+
+    print(f"[case] pressure gradient levels {szI}x{szJ}x{N}", file=sys.stderr, flush=True)
+    GRID, OCEAN, tr, m, a, rng = _state(szI, szJ, N)
+    S2 = szI * szJ
+    get = lambda t: t.detach().cpu().numpy().ravel()
+    Hz = get(GRID.Hz)
+    m.z_r[:] = get(GRID.z_r)
+    m.z_w[:N * S2 + S2] = get(GRID.z_w)
+    ru, rv = rng.standard_normal((N + 1) * S2), rng.standard_normal((N + 1) * S2)
+    OCEAN.ru_t2.copy_(torch.from_numpy(ru))
+    OCEAN.rv_t2.copy_(torch.from_numpy(rv))
+    tr.pressure_gradient(GRID, OCEAN)
+    torch.cuda.synchronize()
+    rho = np.zeros(N * S2)
+    O.lib().sfo_rho_eos(m.cp, O.ptr(a["T"]), O.ptr(a["S"]), *tr.eos, O.ptr(rho))
+    O.lib().sfo_prsgrd(m.cp, O.ptr(rho), O.ptr(m.z_r), O.ptr(m.z_w), O.ptr(Hz), tr.g, tr.rho0, O.ptr(ru), O.ptr(rv))
+    assert bitwise_equal(get(OCEAN.ru_t2), ru) and bitwise_equal(get(OCEAN.rv_t2), rv)
