@@ -179,12 +179,14 @@ __device__ __forceinline__ V h_HvR(const HH &h, long long base, long long o) { r
 template <bool CHK, class HH, class V = typename HH::value_type>
 __device__ __forceinline__ V h_uxxR(const HH &h, long long base, long long o)
 {
-    return (h_uR<CHK>(h, base, o) + h_uR<CHK>(h, base, o + 1) >= 0) ? dxx<CHK>(h.u, base, o) : dxx<CHK>(h.u, base, o + 1);
+    const V here = dxx<CHK>(h.u, base, o), next = dxx<CHK>(h.u, base, o + 1);   // both: no branch around loads
+    return (h_uR<CHK>(h, base, o) + h_uR<CHK>(h, base, o + 1) >= 0) ? here : next;
 }
 template <bool CHK, class HH, class V = typename HH::value_type>
 __device__ __forceinline__ V h_ueeP(const HH &h, long long base, long long o)
 {
-    return (h_HvP<CHK>(h, base, o) + h_HvP<CHK>(h, base, o - h.W) >= 0) ? dee<CHK>(h.u, base, o, h.W) : dee<CHK>(h.u, base, o - h.W, h.W);
+    const V here = dee<CHK>(h.u, base, o, h.W), below = dee<CHK>(h.u, base, o - h.W, h.W);
+    return (h_HvP<CHK>(h, base, o) + h_HvP<CHK>(h, base, o - h.W) >= 0) ? here : below;
 }
 template <bool CHK, class HH, class V = typename HH::value_type>
 __device__ __forceinline__ V h_HuxxR(const HH &h, long long base, long long o)
@@ -380,11 +382,13 @@ void k_rhs3d_fused(G3 g, HG<T> h, A fomn, AG<T> Hz, AG<T> Wa, const int32_t *BC,
     // The face fluxes of the level are each evaluated once, into LDS -- x-faces
     // c' = -1 .. HTI-1 of every row (UFxR, VFxP; column c'+1) and e-faces of rows
     // r' = -1 .. TJ-1 (UFeP, VFeR; row r'+1) -- instead of once by each cell beside the
-    // face.  FP32 (50 VGPRs instead of 64-69): 1024 x 512 x 32 222 us against 273 us.
-    // FP64 also forms the Coriolis terms before the second barrier, so no cell reads the
-    // tile after it and one tile buffer suffices: 46 KB LDS and 80 VGPRs, three
-    // workgroups per CU instead of two (1024 x 512 x 32: 436 us against 443 us per cell
-    // with two buffers; 512 x 256 x 32: 96 us against 104 us).
+    // face.  FP64 also forms the Coriolis terms before the second barrier, so no cell reads
+    // the tile after it and one tile buffer suffices: 46 KB LDS and 80 VGPRs, three
+    // workgroups per CU instead of two.  A thread's x-face at its own column, not the one
+    // before, lets its four fluxes share the curvature terms (27 LDS reads for 47): FP32
+    // 1024 x 512 x 32 242 us -> 229, 386 x 258 x 40 72 -> 68; FP64 435 -> 430, 107 -> 103.
+    // What is left is traffic (1.5 times the fields, from the halos) beside 280 FP64
+    // instructions a level and wave.
     constexpr bool SB = sizeof(T) == 8;   // single tile buffer
     __shared__ T sl[SB ? 1 : 2][4][LN];
     __shared__ T fxu[TJ][HTI + 1], fxv[TJ][HTI + 1], feu[TJ + 1][HTI], fev[TJ + 1][HTI];
@@ -442,6 +446,27 @@ void k_rhs3d_fused(G3 g, HG<T> h, A fomn, AG<T> Hz, AG<T> Wa, const int32_t *BC,
             sb[3][e] = ok ? a3 : T(0);
         }
         __syncthreads();
+        // wave r = tile row r, lane c = column c: the point's x-face c' = c and e-face r' = r
+        // (one point for all four fluxes: they share the curvature terms, in pairs that the
+        // fences keep within FP64's 80 VGPRs), then the e-faces
+        // of row -1 (wave 0) and the x-faces of column -1 (wave 1).  Each is the expression
+        // the cells on either side of the face evaluate (UFxR(0) of the cell on its left is
+        // UFxR(-1) of the cell on its right), at a tile position they read.
+        fxu[r][c + 1] = UFxR<false>(hl, lb, 0);
+        fev[r + 1][c] = VFeR<false>(hl, lb, 0);
+        if constexpr (SB) __builtin_amdgcn_sched_barrier(0);
+        fxv[r][c + 1] = VFxP<false>(hl, lb, 0);
+        feu[r + 1][c] = UFeP<false>(hl, lb, 0);
+        if constexpr (SB) __builtin_amdgcn_sched_barrier(0);
+        if (r == 0) {
+            const long long p = 2LL * HLW + (c + 2);
+            feu[0][c] = UFeP<false>(hl, p, 0);
+            fev[0][c] = VFeR<false>(hl, p, 0);
+        } else if (r == 1 && c < TJ) {
+            const long long p = (long long)(c + 3) * HLW + 1;
+            fxu[c][0] = UFxR<false>(hl, p, 0);
+            fxv[c][0] = VFxP<false>(hl, p, 0);
+        }
         T cu = T(0), cv = T(0);   // SB: the cell's Coriolis terms, formed before the tile is reused
         if constexpr (SB) {
             if (act && rnode) {
@@ -454,27 +479,6 @@ void k_rhs3d_fused(G3 g, HG<T> h, A fomn, AG<T> Hz, AG<T> Wa, const int32_t *BC,
                 cu = (UF0 + UF1) * T(0.5);
                 cv = (VF0 + VF1) * T(0.5);
             }
-        }
-        // wave r = tile row r, lane c = column c.  Pass 1: x-face c' = c-1 of row r;
-        // pass 2: e-face of row r; pass 3: the e-faces of row -1 (wave 0) and the
-        // last x-face c' = HTI-1 of every row (wave 1).  Each is the expression the
-        // cells on either side of the face evaluate (UFxR(0) of the cell on its left
-        // is UFxR(-1) of the cell on its right), at a tile position they read.
-        {
-            const long long p = (long long)(r + 3) * HLW + (c + 1);
-            fxu[r][c] = UFxR<false>(hl, p, 0);
-            fxv[r][c] = VFxP<false>(hl, p, 0);
-        }
-        feu[r + 1][c] = UFeP<false>(hl, lb, 0);
-        fev[r + 1][c] = VFeR<false>(hl, lb, 0);
-        if (r == 0) {
-            const long long p = 2LL * HLW + (c + 2);
-            feu[0][c] = UFeP<false>(hl, p, 0);
-            fev[0][c] = VFeR<false>(hl, p, 0);
-        } else if (r == 1 && c < TJ) {
-            const long long p = (long long)(c + 3) * HLW + (HTI + 1);
-            fxu[c][HTI] = UFxR<false>(hl, p, 0);
-            fxv[c][HTI] = VFxP<false>(hl, p, 0);
         }
         __syncthreads();
         if (act) {
