@@ -11,11 +11,20 @@
 //
 // Four launches per substep, one thread per point: zeta predictor, momentum
 // predictor, zeta corrector (+ time averages), momentum corrector.  Boundary points
-// are written by the same launch (a ghost recomputes its interior source).
+// are written by the same launch (a ghost recomputes its interior source), those of open
+// edges too: a ghost's Chapman value needs only its own source, and one workgroup of a
+// velocity launch takes the edge faces and the volume constraint.  Bound by the latency of
+// the launches on small grids, by loads from L2 on large ones; blocks of points go to the
+// XCDs in bands.  All edges open with the volume constraint, per substep, against ten more
+// launches and no bands: FP64 512 x 256 60 -> 39 us, 1300 x 770 230 -> 130, 2048 x 1024
+// 355 -> 306; FP32 51 -> 31, 135 -> 90, 182 -> 144.
 // Neighbour reads go through L1/L2; each field is read from HBM about once per
 // launch.  The FP64 instance equals the oracle (oracle/sf_oracle_phys.c) bit for
 // bit; FP32 keeps the averages in FP64.
 #include "sf_internal.h"
+#include "volcons.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -136,6 +145,7 @@ struct Sub {
     T dt;
     int first;
     double w1;
+    bool band;                     // points in XCD bands
     Cpl c;
 };
 
@@ -153,13 +163,183 @@ __device__ __forceinline__ T pred_forcing(const Sub<T> &a, bool vdir, long long 
     return r + T(sf::ab_extrapolate(a.c.ab, F, F1[f], F2[f]));
 }
 
-// ---- P1: predicted zeta (+ predictor RHS), and the pressure surface gz ---------------
+// ---- open edges (sf_phys_substep_open) ----------------------------------------------
+// Chapman free surface on the ghost rho points and Flather normal velocity on the edge
+// faces of the open edges (flags: SF_OBC_WEST/EAST/SOUTH/NORTH), in place of the closed
+// walls' values (nonlinear/zetabc.py, the Chapman sketch, and
+// nonlinear/barotropicVelocityBC.py:66-98, Flather; ROMS zetabc/u2dbc/v2dbc):
+//   ghost  zn(g) = (zb(g) + Ce zn(i)) / (1 + Ce),  Ce = dt_s 0.5 (m(g)+m(i)) sqrt(g (h(g)+zb(g)))
+//   face   u = ext_u -/+ sqrt(g/D) (0.5 (zn(g)+zn(i)) - ext_z)   (- west/south, + east/north)
+// zb: the level the stage starts from, dt_s its time span, zn the stage's new surface.
+// Edge points b = 1 .. n (n = szJ-2 for west/east, szI-2 for south/north); b = 1 and b = n
+// also give the face value of the two ghost rows (zero gradient).
+struct Open {
+    int flags;
+    const double *ez[4], *eu[4];
+    int volcons;              // obc_volcons + conserve_mass after each velocity stage
+    double *vc_out;
+};
+
+// the open edge whose ghost rho point (i, j) is, or -1 (corners belong to none)
+__device__ __forceinline__ int ghost_edge(int flags, int i, int j, int L, int M)
+{
+    const bool rows = j >= 1 && j <= M - 1, cols = i >= 1 && i <= L - 1;
+    const int e = rows && i == 0 ? 0 : (rows && i == L ? 1 : (cols && j == 0 ? 2 : (cols && j == M ? 3 : -1)));
+    return e >= 0 && (flags & (1 << e)) ? e : -1;
+}
+
+// Chapman value of the ghost point fg; zi: the stage's new surface at its interior neighbour fi
 template <typename T>
-__global__ __launch_bounds__(256) void k_phys_pred_zeta(Sub<T> a)
+__device__ __forceinline__ T chapman(const PF<T> &p, int e, long long fg, long long fi, T zb, T zi, T dts)
+{
+    const T m = e < 2 ? T(0.5) * (p.pm[fg] + p.pm[fi]) : T(0.5) * (p.pn[fg] + p.pn[fi]);
+    const T Ce = (dts * m) * sqrt(p.g * (p.h[fg] + zb));
+    return (zb + Ce * zi) / (T(1) + Ce);
+}
+
+__device__ const double ob_zero = 0.0;   // read where an edge has no outer values
+
+__device__ __forceinline__ const double *of_edge(const double *const x[4], int e)
+{
+    return e == 0 ? x[0] : (e == 1 ? x[1] : (e == 2 ? x[2] : x[3]));
+}
+
+// Every edge face of the stage whose surface is zn, by the 256 threads of one workgroup:
+// the Flather values and, with volcons, the constraint that the corrector's free surface
+// then sees no net flow through the open edges.  The faces depend on zn alone, so this runs
+// beside the workgroups of the interior velocities.  Same sums as sf_obc_volcons: blocks of
+// 256 points by halving, then the blocks in order.
+// A serial chain that the interior's workgroups hide: the loads of B points a thread go out
+// together (one at a time, 2048 x 1024 took 220 us a substep for 178), B small enough that
+// the edges do not set the kernel's registers.
+template <typename T>
+__device__ void open_faces(const PF<T> &p, const Open &ob, const T *zn, T *x_u, T *x_v)
+{
+    constexpr int VB = 256, CH = 4, B = sizeof(T) == 8 ? 2 : 4;
+    __shared__ double sa[CH][VB], sf_[CH][VB], part[CH][2], total[3];
+    const int W = p.szI, L = p.szI - 1, M = p.szJ - 1, tid = threadIdx.x;
+    const sf::VolArgs<T> va = sf::vol_args(zn, p.h, p.pm, p.pn, x_u, x_v, p.szI, p.szJ, ob.flags);
+    const int n = va.nw + va.ne + va.ns + va.nn;
+    // point b of the edges: its edge e, its place k = 1 .. along it and its face, which lies
+    // between the rho points face - step and face; points past the last are the last again
+    auto point = [&](int b, int &e, int &k) {
+        k = b < n ? b : n - 1;
+        e = sf::vol_segment(va, k);
+        const int f = (int)sf::vol_face(va, e, k);
+        k = k + 1;
+        return f;
+    };
+    double area = 0.0, flux = 0.0;
+    for (int base = 0; base < n; base += VB * CH) {
+#pragma unroll 1
+        for (int q0 = 0; q0 < CH; q0 += B) {
+            T zl[B], zh[B], hl[B], hh[B], ml[B], mh[B];
+            double ez[B], eu[B];
+#pragma unroll
+            for (int q = 0; q < B; q++) {
+                int e, k;
+                const int f = point(base + (q0 + q) * VB + tid, e, k), lo = f - (e < 2 ? 1 : W);
+                const T *m = e < 2 ? p.pn : p.pm;
+                zl[q] = zn[lo];
+                zh[q] = zn[f];
+                hl[q] = p.h[lo];
+                hh[q] = p.h[f];
+                ml[q] = m[lo];
+                mh[q] = m[f];
+                const double *pz = of_edge(ob.ez, e), *pu = of_edge(ob.eu, e);
+                ez[q] = *(pz ? pz + k : &ob_zero);
+                eu[q] = *(pu ? pu + k : &ob_zero);
+            }
+#pragma unroll
+            for (int q = 0; q < B; q++) {
+                int e, k;
+                const int b = base + (q0 + q) * VB + tid, f = point(b, e, k);
+                double cff = 0.0, fl = 0.0;
+                if (b < n) {
+                    const bool inward = e == 0 || e == 2;
+                    const T D = T(0.5) * ((hl[q] + zl[q]) + (hh[q] + zh[q]));
+                    const T c = sqrt(p.g / D);
+                    const T dz = T(0.5) * (zl[q] + zh[q]) - T(ez[q]);
+                    const T val = inward ? T(eu[q]) - c * dz : T(eu[q]) + c * dz;
+                    T *x = (e < 2 ? x_u : x_v) + f;
+                    *x = val;
+                    // ghost rows (west/east) or columns (south/north) of the face
+                    const long long step = e < 2 ? W : 1;
+                    if (k == 1) x[-step] = val;
+                    if (k == (e < 2 ? M - 1 : L - 1)) x[step] = val;
+                    sf::vol_terms(zl[q], hl[q], zh[q], hh[q], ml[q], mh[q], val, inward, cff, fl);
+                }
+                sa[q0 + q][tid] = cff;
+                sf_[q0 + q][tid] = fl;
+            }
+        }
+        if (!ob.volcons) continue;
+        __syncthreads();
+        const int w = tid >> 6, t = tid & 63;   // wave w: block w of the round
+        double s0 = (sa[w][t] + sa[w][t + 128]) + (sa[w][t + 64] + sa[w][t + 192]);
+        double s1 = (sf_[w][t] + sf_[w][t + 128]) + (sf_[w][t + 64] + sf_[w][t + 192]);
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            s0 += __shfl_down(s0, d);
+            s1 += __shfl_down(s1, d);
+        }
+        if (t == 0) {
+            part[w][0] = s0;
+            part[w][1] = s1;
+        }
+        __syncthreads();
+        if (tid == 0)
+            for (int q = 0; q < CH && base + q * VB < n; q++) {
+                area += part[q][0];
+                flux += part[q][1];
+            }
+    }
+    if (!ob.volcons) return;
+    if (tid == 0) {
+        total[0] = area;
+        total[1] = flux;
+        total[2] = area > 0.0 ? flux / area : 0.0;
+        for (int q = 0; q < 3; q++) ob.vc_out[q] = total[q];
+    }
+    __syncthreads();
+    const double xs = total[2];
+    for (int base = tid; base < n; base += VB * CH) {   // each face by the thread that wrote it above
+        T v[CH];
+        int e, k;
+#pragma unroll
+        for (int q = 0; q < CH; q++) {
+            const int f = point(base + q * VB, e, k);
+            v[q] = (e < 2 ? x_u : x_v)[f];
+        }
+#pragma unroll
+        for (int q = 0; q < CH; q++) {
+            const int f = point(base + q * VB, e, k);
+            if (base + q * VB < n)
+                (e < 2 ? x_u : x_v)[f] = (e == 0 || e == 2) ? (T)((double)v[q] - xs) : (T)((double)v[q] + xs);
+        }
+    }
+}
+
+// Block of points of a velocity stage.  OPEN: the first eight blocks are the edges' -- one
+// works -- and the others leave the open edges' faces alone.
+template <bool OPEN>
+__device__ __forceinline__ long long uv_point(bool band)
+{
+    unsigned b = blockIdx.x, nb = gridDim.x;
+    if constexpr (OPEN) {
+        b -= 8;
+        nb -= 8;
+    }
+    return (long long)(band ? (b & 7) * (nb >> 3) + (b >> 3) : b) * blockDim.x + threadIdx.x;
+}
+
+// ---- P1: predicted zeta (+ predictor RHS), and the pressure surface gz ---------------
+template <typename T, bool OPEN>
+__global__ __launch_bounds__(256) void k_phys_pred_zeta(Sub<T> a, Open ob)
 {
     const int szI = a.p.szI, szJ = a.p.szJ;
     const long long S2 = (long long)szI * szJ;
-    const long long f = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long f = (long long)sf::column_block(a.band) * blockDim.x + threadIdx.x;
     if (f >= S2) return;
     int i = (int)(f % szI), j = (int)(f / szI);
     const bool ghost = i < 1 || i > szI - 2 || j < 1 || j > szJ - 2;
@@ -178,6 +358,10 @@ __global__ __launch_bounds__(256) void k_phys_pred_zeta(Sub<T> a)
             a.c.DU2[f] = du + a.c.w2p * (double)DUon(a.p, a.z1, a.u1, f);
             a.c.DV2[f] = dv + a.c.w2p * (double)DVom(a.p, a.z1, a.v1, f);
         }
+    }
+    if constexpr (OPEN) {   // fs is the ghost's interior neighbour
+        const int e = ghost ? ghost_edge(ob.flags, i, j, szI - 1, szJ - 1) : -1;
+        if (e >= 0) zs = chapman(a.p, e, f, fs, a.first ? a.z1[f] : a.z0[f], zs, a.first ? a.dt : T(2) * a.dt);
     }
     a.zs[f] = zs;
     const T cff4 = T(4.0 / 25.0), cff5 = T(1) - T(2) * cff4;
@@ -218,25 +402,32 @@ __device__ T pred_v(const Sub<T> &a, long long f, bool store_rhs)
     return (vb[f] * (Dat(a.p, zb, f) + Dat(a.p, zb, f - W)) + (cff * c1) * r) * fac;
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void k_phys_pred_uv(Sub<T> a)
+template <typename T, bool OPEN>
+__global__ __launch_bounds__(256) void k_phys_pred_uv(Sub<T> a, Open ob)
 {
+    if constexpr (OPEN) {
+        if (blockIdx.x == 0) open_faces(a.p, ob, (const T *)a.zs, a.us, a.vs);
+        if (blockIdx.x < 8) return;
+    }
     const int szI = a.p.szI, szJ = a.p.szJ, L = szI - 1, M = szJ - 1;
-    const long long S2 = (long long)szI * szJ, W = szI;
-    const long long f = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long S2 = (long long)szI * szJ, W = szI, f = uv_point<OPEN>(a.band);
     if (f >= S2) return;
     const int i = (int)(f % szI), j = (int)(f / szI);
-    // ubar: interior i in [2, L-1], j in [1, M-1]; walls/column 0 zero; ghost rows copy
-    T u;
-    if (i <= 1 || i >= L) u = T(0);
-    else if (j >= 1 && j <= M - 1) u = pred_u(a, f, true);
-    else u = pred_u(a, j == 0 ? f + W : f - W, false);
-    a.us[f] = u;
-    T v;
-    if (j <= 1 || j >= M) v = T(0);
-    else if (i >= 1 && i <= L - 1) v = pred_v(a, f, true);
-    else v = pred_v(a, i == 0 ? f + 1 : f - 1, false);
-    a.vs[f] = v;
+    if (!(OPEN && ((i == 1 && (ob.flags & SF_OBC_WEST)) || (i == L && (ob.flags & SF_OBC_EAST))))) {
+        // ubar: interior i in [2, L-1], j in [1, M-1]; walls/column 0 zero; ghost rows copy
+        T u;
+        if (i <= 1 || i >= L) u = T(0);
+        else if (j >= 1 && j <= M - 1) u = pred_u(a, f, true);
+        else u = pred_u(a, j == 0 ? f + W : f - W, false);
+        a.us[f] = u;
+    }
+    if (!(OPEN && ((j == 1 && (ob.flags & SF_OBC_SOUTH)) || (j == M && (ob.flags & SF_OBC_NORTH))))) {
+        T v;
+        if (j <= 1 || j >= M) v = T(0);
+        else if (i >= 1 && i <= L - 1) v = pred_v(a, f, true);
+        else v = pred_v(a, i == 0 ? f + 1 : f - 1, false);
+        a.vs[f] = v;
+    }
 }
 
 // ---- C1: corrected zeta, time averages, and the corrector pressure surface ----------
@@ -252,12 +443,12 @@ __device__ T corr_zeta(const Sub<T> &a, long long f, T *rstar)
     return a.z1[f] + pmn * ((a1 * r + a2 * a.rz1[f]) - a3 * a.rz0[f]);
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void k_phys_corr_zeta(Sub<T> a)
+template <typename T, bool OPEN>
+__global__ __launch_bounds__(256) void k_phys_corr_zeta(Sub<T> a, Open ob)
 {
     const int szI = a.p.szI, szJ = a.p.szJ;
     const long long S2 = (long long)szI * szJ;
-    const long long f = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long f = (long long)sf::column_block(a.band) * blockDim.x + threadIdx.x;
     if (f >= S2) return;
     int i = (int)(f % szI), j = (int)(f / szI);
     const bool ghost = i < 1 || i > szI - 2 || j < 1 || j > szJ - 2;
@@ -265,7 +456,11 @@ __global__ __launch_bounds__(256) void k_phys_corr_zeta(Sub<T> a)
     zeta_src(szI, szJ, si, sj);
     const long long fs = (long long)sj * szI + si;
     T rstar;
-    const T z2 = corr_zeta(a, fs, &rstar);
+    T z2 = corr_zeta(a, fs, &rstar);
+    if constexpr (OPEN) {
+        const int e = ghost ? ghost_edge(ob.flags, i, j, szI - 1, szJ - 1) : -1;
+        if (e >= 0) z2 = chapman(a.p, e, f, fs, a.z1[f], z2, a.dt);
+    }
     a.z2[f] = z2;
     const T cf4 = T(2.0 / 5.0), cf5 = T(1) - cf4;
     a.gz[f] = cf5 * z2 + cf4 * a.zs[f];
@@ -311,102 +506,31 @@ __device__ T corr_v(const Sub<T> &a, long long f)
     return (a.v1[f] * (Dat(a.p, a.z1, f) + Dat(a.p, a.z1, f - W)) + cff * tend) * fac;
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void k_phys_corr_uv(Sub<T> a)
+template <typename T, bool OPEN>
+__global__ __launch_bounds__(256) void k_phys_corr_uv(Sub<T> a, Open ob)
 {
+    if constexpr (OPEN) {
+        if (blockIdx.x == 0) open_faces(a.p, ob, (const T *)a.z2, a.u2, a.v2);
+        if (blockIdx.x < 8) return;
+    }
     const int szI = a.p.szI, szJ = a.p.szJ, L = szI - 1, M = szJ - 1;
-    const long long S2 = (long long)szI * szJ, W = szI;
-    const long long f = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long S2 = (long long)szI * szJ, W = szI, f = uv_point<OPEN>(a.band);
     if (f >= S2) return;
     const int i = (int)(f % szI), j = (int)(f / szI);
-    T u;
-    if (i <= 1 || i >= L) u = T(0);
-    else if (j >= 1 && j <= M - 1) u = corr_u(a, f);
-    else u = corr_u(a, j == 0 ? f + W : f - W);
-    a.u2[f] = u;
-    T v;
-    if (j <= 1 || j >= M) v = T(0);
-    else if (i >= 1 && i <= L - 1) v = corr_v(a, f);
-    else v = corr_v(a, i == 0 ? f + 1 : f - 1);
-    a.v2[f] = v;
-}
-
-// ---- open edges (sf_phys_substep_open) ----------------------------------------------
-// Chapman free surface on the ghost rho points and Flather normal velocity on the edge
-// faces of the open edges (flags: SF_OBC_WEST/EAST/SOUTH/NORTH), applied after the stage
-// kernels have written closed-wall values (nonlinear/zetabc.py, the Chapman sketch, and
-// nonlinear/barotropicVelocityBC.py:66-98, Flather; ROMS zetabc/u2dbc/v2dbc):
-//   ghost  zn(g) = (zb(g) + Ce zn(i)) / (1 + Ce),  Ce = dt_s 0.5 (m(g)+m(i)) sqrt(g (h(g)+zb(g)))
-//   face   u = ext_u -/+ sqrt(g/D) (0.5 (zn(g)+zn(i)) - ext_z)   (- west/south, + east/north)
-// zb: the level the stage starts from, dt_s its time span, zn the stage's new surface.
-// Edge points b = 1 .. n (n = szJ-2 for west/east, szI-2 for south/north); the threads of
-// b = 1 and b = n also write the face value into the two ghost rows (zero gradient).
-struct Open {
-    int flags;
-    const double *ez[4], *eu[4];
-    int volcons;              // obc_volcons + conserve_mass after each velocity stage
-    double *vc_work, *vc_out;
-};
-
-__device__ __forceinline__ void edge_points(int e, int b, int W, int L, int M, long long &fg, long long &fi,
-                                            long long &fu)
-{
-    if (e == 0) { fg = (long long)b * W; fi = fg + 1; fu = fi; }
-    else if (e == 1) { fg = (long long)b * W + L; fi = fg - 1; fu = fg; }
-    else if (e == 2) { fg = b; fi = (long long)W + b; fu = fi; }
-    else { fg = (long long)M * W + b; fi = fg - W; fu = fg; }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_open_zeta(Sub<T> a, Open ob, int corrector)
-{
-    const int e = blockIdx.y;
-    if (!(ob.flags & (1 << e))) return;
-    const int W = a.p.szI, L = a.p.szI - 1, M = a.p.szJ - 1;
-    const int n = e < 2 ? M - 1 : L - 1;
-    const int b = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (b > n) return;
-    long long fg, fi, fu;
-    edge_points(e, b, W, L, M, fg, fi, fu);
-    T *zn = corrector ? a.z2 : a.zs;
-    const T *zb = corrector ? a.z1 : (a.first ? a.z1 : a.z0);
-    const T dts = corrector ? a.dt : (a.first ? a.dt : T(2) * a.dt);
-    const T m = e < 2 ? T(0.5) * (a.p.pm[fg] + a.p.pm[fi]) : T(0.5) * (a.p.pn[fg] + a.p.pn[fi]);
-    const T Ce = (dts * m) * sqrt(a.p.g * (a.p.h[fg] + zb[fg]));
-    const T z = (zb[fg] + Ce * zn[fi]) / (T(1) + Ce);
-    zn[fg] = z;
-    if (corrector) {
-        const T cf4 = T(2.0 / 5.0), cf5 = T(1) - cf4;
-        a.gz[fg] = cf5 * z + cf4 * a.zs[fg];
-    } else {
-        const T cff4 = T(4.0 / 25.0), cff5 = T(1) - T(2) * cff4;
-        a.gz[fg] = a.first ? T(0.5) * (a.z1[fg] + z) : cff5 * a.z1[fg] + cff4 * (a.z0[fg] + z);
+    if (!(OPEN && ((i == 1 && (ob.flags & SF_OBC_WEST)) || (i == L && (ob.flags & SF_OBC_EAST))))) {
+        T u;
+        if (i <= 1 || i >= L) u = T(0);
+        else if (j >= 1 && j <= M - 1) u = corr_u(a, f);
+        else u = corr_u(a, j == 0 ? f + W : f - W);
+        a.u2[f] = u;
     }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_open_vel(Sub<T> a, Open ob, int corrector)
-{
-    const int e = blockIdx.y;
-    if (!(ob.flags & (1 << e))) return;
-    const int W = a.p.szI, L = a.p.szI - 1, M = a.p.szJ - 1;
-    const int n = e < 2 ? M - 1 : L - 1;
-    const int b = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (b > n) return;
-    long long fg, fi, fu;
-    edge_points(e, b, W, L, M, fg, fi, fu);
-    const T *zn = corrector ? a.z2 : a.zs;
-    T *x = e < 2 ? (corrector ? a.u2 : a.us) : (corrector ? a.v2 : a.vs);
-    const T D = T(0.5) * ((a.p.h[fg] + zn[fg]) + (a.p.h[fi] + zn[fi]));
-    const T c = sqrt(a.p.g / D);
-    const T ez = ob.ez[e] ? T(ob.ez[e][b]) : T(0), eu = ob.eu[e] ? T(ob.eu[e][b]) : T(0);
-    const T dz = T(0.5) * (zn[fg] + zn[fi]) - ez;
-    const T val = (e == 0 || e == 2) ? eu - c * dz : eu + c * dz;
-    x[fu] = val;
-    // ghost rows (west/east) or columns (south/north) of the face
-    const long long step = e < 2 ? W : 1;
-    if (b == 1) x[fu - step] = val;
-    if (b == n) x[fu + step] = val;
+    if (!(OPEN && ((j == 1 && (ob.flags & SF_OBC_SOUTH)) || (j == M && (ob.flags & SF_OBC_NORTH))))) {
+        T v;
+        if (j <= 1 || j >= M) v = T(0);
+        else if (i >= 1 && i <= L - 1) v = corr_v(a, f);
+        else v = corr_v(a, i == 0 ? f + 1 : f - 1);
+        a.v2[f] = v;
+    }
 }
 
 template <typename T>
@@ -447,32 +571,19 @@ int launch_phys(const sf_phys_fields *x, double dt, int first, double w1, void *
     a.first = first;
     a.w1 = w1;
     const long long S2 = (long long)x->szI * x->szJ;
-    const dim3 grid(sf::grid1d(S2)), block(256);
+    a.band = (double)S2 * sizeof(T) <= sf::kBandBytes;
+    const unsigned nb = sf::column_grid(S2);
     hipStream_t s = sf::as_stream(stream);
-    const int nedge = (x->szI > x->szJ ? x->szI : x->szJ);
-    const dim3 egrid(sf::grid1d(nedge), 4);
-    hipLaunchKernelGGL(k_phys_pred_zeta<T>, grid, block, 0, s, a);
-    if (ob) hipLaunchKernelGGL(k_open_zeta<T>, egrid, block, 0, s, a, *ob, 0);
-    const int prec = sizeof(T) == 8 ? SF_FP64 : SF_FP32;
-    const bool vc = ob && ob->volcons && ob->flags;
-    hipLaunchKernelGGL(k_phys_pred_uv<T>, grid, block, 0, s, a);
-    if (ob) hipLaunchKernelGGL(k_open_vel<T>, egrid, block, 0, s, a, *ob, 0);
-    // the volume constraint on the predicted velocities: the corrector's free surface
-    // then sees no net flow through the open edges
-    if (vc) {
-        const int rc = sf_obc_volcons(a.zs, x->h, x->pm, x->pn, a.us, a.vs, x->szI, x->szJ, prec, ob->flags, 1,
-                                      ob->vc_work, ob->vc_out, stream);
-        if (rc != SF_OK) return rc;
-    }
-    hipLaunchKernelGGL(k_phys_corr_zeta<T>, grid, block, 0, s, a);
-    if (ob) hipLaunchKernelGGL(k_open_zeta<T>, egrid, block, 0, s, a, *ob, 1);
-    hipLaunchKernelGGL(k_phys_corr_uv<T>, grid, block, 0, s, a);
-    if (ob) hipLaunchKernelGGL(k_open_vel<T>, egrid, block, 0, s, a, *ob, 1);
-    if (vc) {
-        const int rc = sf_obc_volcons(x->zeta[2], x->h, x->pm, x->pn, x->ubar[2], x->vbar[2], x->szI, x->szJ, prec,
-                                      ob->flags, 1, ob->vc_work, ob->vc_out, stream);
-        if (rc != SF_OK) return rc;
-    }
+    auto stages = [&](auto open, const Open &o) {
+        constexpr bool OPEN = decltype(open)::value;
+        const dim3 grid(nb), uv(nb + (OPEN ? 8 : 0)), block(256);
+        hipLaunchKernelGGL((k_phys_pred_zeta<T, OPEN>), grid, block, 0, s, a, o);
+        hipLaunchKernelGGL((k_phys_pred_uv<T, OPEN>), uv, block, 0, s, a, o);
+        hipLaunchKernelGGL((k_phys_corr_zeta<T, OPEN>), grid, block, 0, s, a, o);
+        hipLaunchKernelGGL((k_phys_corr_uv<T, OPEN>), uv, block, 0, s, a, o);
+    };
+    if (ob && ob->flags) stages(std::true_type{}, *ob);
+    else stages(std::false_type{}, Open{});
     return sf::check_launch("sf_phys_substep");
 }
 
@@ -541,7 +652,6 @@ extern "C" int sf_phys_substep_open(const sf_phys_fields *x, const sf_open_bc *o
         ob.eu[e] = obc->vel_ext[e];
     }
     ob.volcons = obc->volcons;
-    ob.vc_work = volcons_work;
     ob.vc_out = volcons_out;
     if (precision == SF_FP64) return launch_phys<double>(x, dt, first, cff1, stream, nullptr, &ob);
     if (precision == SF_FP32) return launch_phys<float>(x, dt, first, cff1, stream, nullptr, &ob);

@@ -12,6 +12,7 @@
 // fixed-shape block tree followed by an ordered sum of the block partials, so the
 // result is reproducible run to run.
 #include "sf_internal.h"
+#include "volcons.h"
 
 #include <mutex>
 
@@ -25,46 +26,7 @@ namespace {
 
 constexpr int VB = 256;
 
-template <typename T>
-struct VolArgs {
-    const T *z, *h, *pm, *pn;
-    T *u, *v;
-    int szI, szJ, flags;
-    int nw, ne, ns, nn;   // points per segment (0 when closed)
-};
-
-// boundary point b -> (flat index of the velocity point, area term, signed velocity)
-template <typename T>
-__device__ __forceinline__ void vol_point(const VolArgs<T> &a, int b, double &cff, double &fl)
-{
-    const int W = a.szI, L = a.szI - 1, M = a.szJ - 1;
-    int seg = 0;
-    if (b >= a.nw) {
-        b -= a.nw;
-        seg = 1;
-        if (b >= a.ne) {
-            b -= a.ne;
-            seg = 2;
-            if (b >= a.ns) {
-                b -= a.ns;
-                seg = 3;
-            }
-        }
-    }
-    if (seg <= 1) {   // west / east u points, rows j = 1 .. M-1
-        const int j = 1 + b, i = seg == 0 ? 1 : L;
-        const long long f = (long long)j * W + i;
-        const double onu = 2.0 / ((double)a.pn[f - 1] + (double)a.pn[f]);
-        cff = (0.5 * (((double)a.z[f - 1] + (double)a.h[f - 1]) + ((double)a.z[f] + (double)a.h[f]))) * onu;
-        fl = seg == 0 ? cff * (double)a.u[f] : -(cff * (double)a.u[f]);
-    } else {          // south / north v points, columns i = 1 .. L-1
-        const int i = 1 + b, j = seg == 2 ? 1 : M;
-        const long long f = (long long)j * W + i;
-        const double omv = 2.0 / ((double)a.pm[f - W] + (double)a.pm[f]);
-        cff = (0.5 * (((double)a.z[f - W] + (double)a.h[f - W]) + ((double)a.z[f] + (double)a.h[f]))) * omv;
-        fl = seg == 2 ? cff * (double)a.v[f] : -(cff * (double)a.v[f]);
-    }
-}
+using sf::VolArgs;
 
 template <typename T>
 __global__ __launch_bounds__(VB) void k_volcons_partial(VolArgs<T> a, int n, double *__restrict__ part)
@@ -72,7 +34,14 @@ __global__ __launch_bounds__(VB) void k_volcons_partial(VolArgs<T> a, int n, dou
     __shared__ double sa[VB], sf[VB];
     const int b = blockIdx.x * VB + threadIdx.x;
     double cff = 0.0, fl = 0.0;
-    if (b < n) vol_point(a, b, cff, fl);
+    if (b < n) {
+        int k = b;
+        const int e = sf::vol_segment(a, k);
+        const long long f = sf::vol_face(a, e, k);
+        const long long p = e < 2 ? f - 1 : f - a.szI;
+        const T *m = e < 2 ? a.pn : a.pm;
+        sf::vol_terms(a.z[p], a.h[p], a.z[f], a.h[f], m[p], m[f], e < 2 ? a.u[f] : a.v[f], e == 0 || e == 2, cff, fl);
+    }
     sa[threadIdx.x] = cff;
     sf[threadIdx.x] = fl;
     __syncthreads();
@@ -110,48 +79,19 @@ __global__ __launch_bounds__(VB) void k_volcons_apply(VolArgs<T> a, int n, const
     const int b = blockIdx.x * VB + threadIdx.x;
     if (b >= n) return;
     const double xs = out[2];
-    const int W = a.szI, L = a.szI - 1, M = a.szJ - 1;
-    int r = b;
-    if (r < a.nw) {
-        const long long f = (long long)(1 + r) * W + 1;
-        a.u[f] = (T)((double)a.u[f] - xs);
-        return;
-    }
-    r -= a.nw;
-    if (r < a.ne) {
-        const long long f = (long long)(1 + r) * W + L;
-        a.u[f] = (T)((double)a.u[f] + xs);
-        return;
-    }
-    r -= a.ne;
-    if (r < a.ns) {
-        const long long f = (long long)W + 1 + r;
-        a.v[f] = (T)((double)a.v[f] - xs);
-        return;
-    }
-    r -= a.ns;
-    const long long f = (long long)M * W + 1 + r;
-    a.v[f] = (T)((double)a.v[f] + xs);
+    int k = b;
+    const int e = sf::vol_segment(a, k);
+    T *x = e < 2 ? a.u : a.v;
+    const long long f = sf::vol_face(a, e, k);
+    x[f] = (e == 0 || e == 2) ? (T)((double)x[f] - xs) : (T)((double)x[f] + xs);
 }
 
 template <typename T>
 int run_volcons(const void *zeta, const void *h, const void *pm, const void *pn, void *ubar, void *vbar, int szI,
                 int szJ, int flags, int apply, double *work, double *out, void *stream)
 {
-    VolArgs<T> a;
-    a.z = (const T *)zeta;
-    a.h = (const T *)h;
-    a.pm = (const T *)pm;
-    a.pn = (const T *)pn;
-    a.u = (T *)ubar;
-    a.v = (T *)vbar;
-    a.szI = szI;
-    a.szJ = szJ;
-    a.flags = flags;
-    a.nw = (flags & SF_OBC_WEST) ? szJ - 2 : 0;
-    a.ne = (flags & SF_OBC_EAST) ? szJ - 2 : 0;
-    a.ns = (flags & SF_OBC_SOUTH) ? szI - 2 : 0;
-    a.nn = (flags & SF_OBC_NORTH) ? szI - 2 : 0;
+    const VolArgs<T> a = sf::vol_args((const T *)zeta, (const T *)h, (const T *)pm, (const T *)pn, (T *)ubar,
+                                      (T *)vbar, szI, szJ, flags);
     const int n = a.nw + a.ne + a.ns + a.nn;
     const int nblk = n > 0 ? (n + VB - 1) / VB : 1;
     hipStream_t s = sf::as_stream(stream);
