@@ -203,7 +203,10 @@ __global__ __launch_bounds__(NT) void k_mlp_fwd_bwd(const uint16_t *__restrict__
 // and the 16 sums are added in wave order: a fixed order for any grid, so the result is
 // deterministic.  Reads are coalesced (64 consecutive parameters of one block per wave
 // instruction).
+// One more workgroup sums the loss; a single thread beside the parameters, with 16 loads in
+// flight, took longer than all of them: 256 blocks' partials 8.0 us -> 4.4.
 constexpr int RP = 64, RS = 16;   // parameters and block slices per reduce workgroup
+constexpr int NPARAM_GROUPS = (NPARAM + RP - 1) / RP;
 
 // src[b * stride] summed over b = b0, b0 + db, ... < nb in that order, 16 loads in flight
 __device__ __forceinline__ float sum_strided(const float *__restrict__ src, long long stride, int b0, int db, int nb)
@@ -221,6 +224,21 @@ __device__ __forceinline__ float sum_strided(const float *__restrict__ src, long
     return acc;
 }
 
+// acc + x[0] + x[1] + ... in that order, 16 reads in flight
+__device__ __forceinline__ float sum_lds(const float *x, int n, float acc)
+{
+    int k = 0;
+    for (; k + 16 <= n; k += 16) {
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) v[u] = x[k + u];
+#pragma unroll
+        for (int u = 0; u < 16; u++) acc += v[u];
+    }
+    for (; k < n; k++) acc += x[k];
+    return acc;
+}
+
 __global__ __launch_bounds__(RP * RS) void k_mlp_reduce_adam(const float *__restrict__ partial,
                                                             const float *__restrict__ partial_loss, int nblk,
                                                             float *__restrict__ grad, float *__restrict__ w,
@@ -233,7 +251,19 @@ __global__ __launch_bounds__(RP * RS) void k_mlp_reduce_adam(const float *__rest
     __shared__ float red[RS][RP];
     const int lane = threadIdx.x & 63, slice = threadIdx.x >> 6;
     const int p = blockIdx.x * RP + lane;
-    if (blockIdx.x == 0 && threadIdx.x == 0 && loss_out) loss_out[0] = sum_strided(partial_loss, 1, 0, 1, nblk) * inv_count;
+    if (blockIdx.x == NPARAM_GROUPS) {   // the loss: block sums in increasing order
+        float *const all = red[0];
+        float acc = 0.0f;
+        for (int b0 = 0; b0 < nblk; b0 += RP * RS) {
+            const int b = b0 + threadIdx.x, nb = nblk - b0 < RP * RS ? nblk - b0 : RP * RS;
+            if (b < nblk) all[threadIdx.x] = partial_loss[b];
+            __syncthreads();
+            if (threadIdx.x == 0) acc = sum_lds(all, nb, acc);
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) loss_out[0] = acc * inv_count;
+        return;
+    }
     red[slice][lane] = p < NPARAM ? sum_strided(partial + p, NPARAM, slice, RS, nblk) : 0.0f;
     __syncthreads();
     if (slice != 0 || p >= NPARAM) return;
@@ -391,7 +421,7 @@ extern "C" int sf_mlp_train_step(sf_mlp *p, const uint16_t *X, const float *Y, c
                        p->partial, p->ploss);
     const float bc1 = adam ? 1.0f - powf(beta1, (float)step) : 1.0f;
     const float bc2 = adam ? 1.0f - powf(beta2, (float)step) : 1.0f;
-    hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((NPARAM + RP - 1) / RP), dim3(RP * RS), 0, s, p->partial, p->ploss,
+    hipLaunchKernelGGL(k_mlp_reduce_adam, dim3(NPARAM_GROUPS + 1), dim3(RP * RS), 0, s, p->partial, p->ploss,
                        nblocks, p->grad, p->w, p->m, p->v, p->wb, p->wpk, adam, lr, beta1, beta2, eps, bc1, bc2,
                        1.0f / (float)(batch * NOUT), p->loss);
     return sf::check_launch("sf_mlp_train_step");
