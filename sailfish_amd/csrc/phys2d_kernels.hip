@@ -225,7 +225,7 @@ __device__ void open_faces(const PF<T> &p, const Open &ob, const T *zn, T *x_u, 
     auto point = [&](int b, int &e, int &k) {
         k = b < n ? b : n - 1;
         e = sf::vol_segment(va, k);
-        const int f = (int)sf::vol_face(va, e, k);
+        const long long f = sf::vol_face(va, e, k);
         k = k + 1;
         return f;
     };
@@ -238,7 +238,7 @@ __device__ void open_faces(const PF<T> &p, const Open &ob, const T *zn, T *x_u, 
 #pragma unroll
             for (int q = 0; q < B; q++) {
                 int e, k;
-                const int f = point(base + (q0 + q) * VB + tid, e, k), lo = f - (e < 2 ? 1 : W);
+                const long long f = point(base + (q0 + q) * VB + tid, e, k), lo = f - (e < 2 ? 1 : W);
                 const T *m = e < 2 ? p.pn : p.pm;
                 zl[q] = zn[lo];
                 zh[q] = zn[f];
@@ -253,7 +253,8 @@ __device__ void open_faces(const PF<T> &p, const Open &ob, const T *zn, T *x_u, 
 #pragma unroll
             for (int q = 0; q < B; q++) {
                 int e, k;
-                const int b = base + (q0 + q) * VB + tid, f = point(b, e, k);
+                const int b = base + (q0 + q) * VB + tid;
+                const long long f = point(b, e, k);
                 double cff = 0.0, fl = 0.0;
                 if (b < n) {
                     const bool inward = e == 0 || e == 2;
@@ -308,12 +309,12 @@ __device__ void open_faces(const PF<T> &p, const Open &ob, const T *zn, T *x_u, 
         int e, k;
 #pragma unroll
         for (int q = 0; q < CH; q++) {
-            const int f = point(base + q * VB, e, k);
+            const long long f = point(base + q * VB, e, k);
             v[q] = (e < 2 ? x_u : x_v)[f];
         }
 #pragma unroll
         for (int q = 0; q < CH; q++) {
-            const int f = point(base + q * VB, e, k);
+            const long long f = point(base + q * VB, e, k);
             if (base + q * VB < n)
                 (e < 2 ? x_u : x_v)[f] = (e == 0 || e == 2) ? (T)((double)v[q] - xs) : (T)((double)v[q] + xs);
         }
