@@ -439,8 +439,9 @@ typedef struct sf_open_bc {
  * velocity stages (predicted and new state) the volume constraint
  * (nonlinear/obc_volcons.py:1-72, sf_obc_volcons) removes the net flow through the open
  * edges, so the free-surface updates conserve the volume (volcons_work:
- * sf_obc_volcons_work_size doubles, required with volcons and left unwritten: the sums stay
- * on chip; volcons_out: area, flux, ubar_xs of the last). */
+ * sf_obc_volcons_work_size doubles, required with volcons; written only where the edges are
+ * long for the grid, else the sums stay on chip; volcons_out: area, flux, ubar_xs of the
+ * last). */
 int sf_phys_substep_open(const sf_phys_fields *fields, const sf_open_bc *obc, int32_t precision, double dt,
                          int32_t first, double cff1, double *volcons_work, double *volcons_out, void *stream);
 

@@ -12,8 +12,9 @@
 // Four launches per substep, one thread per point: zeta predictor, momentum
 // predictor, zeta corrector (+ time averages), momentum corrector.  Boundary points
 // are written by the same launch (a ghost recomputes its interior source), those of open
-// edges too: a ghost's Chapman value needs only its own source, and one workgroup of a
-// velocity launch takes the edge faces and the volume constraint.  Bound by the latency of
+// edges too: a ghost's Chapman value needs only its own source, and the first workgroups of
+// a velocity launch take the edge faces, one of them the volume constraint too unless the
+// edges are long for the grid (launch_phys).  Bound by the latency of
 // the launches on small grids, by loads from L2 on large ones; blocks of points go to the
 // XCDs in bands.  All edges open with the volume constraint, per substep, against ten more
 // launches and no bands: FP64 512 x 256 60 -> 39 us, 1300 x 770 230 -> 130, 2048 x 1024
@@ -177,8 +178,10 @@ struct Open {
     int flags;
     const double *ez[4], *eu[4];
     int volcons;              // obc_volcons + conserve_mass after each velocity stage
-    double *vc_out;
+    double *vc_work, *vc_out;
+    int groups, blocks;       // workgroups on the edges, first blocks of a velocity launch kept for them
 };
+constexpr int kEdgeRound = 1024;   // edge points a workgroup takes at a time
 
 // the open edge whose ghost rho point (i, j) is, or -1 (corners belong to none)
 __device__ __forceinline__ int ghost_edge(int flags, int i, int j, int L, int M)
@@ -204,11 +207,11 @@ __device__ __forceinline__ const double *of_edge(const double *const x[4], int e
     return e == 0 ? x[0] : (e == 1 ? x[1] : (e == 2 ? x[2] : x[3]));
 }
 
-// Every edge face of the stage whose surface is zn, by the 256 threads of one workgroup:
-// the Flather values and, with volcons, the constraint that the corrector's free surface
-// then sees no net flow through the open edges.  The faces depend on zn alone, so this runs
-// beside the workgroups of the interior velocities.  Same sums as sf_obc_volcons: blocks of
-// 256 points by halving, then the blocks in order.
+// The edge faces of the stage whose surface is zn, by ob.groups workgroups of 256 threads:
+// the Flather values and, with volcons (one workgroup), the constraint that the corrector's
+// free surface then sees no net flow through the open edges.  The faces depend on zn alone,
+// so this runs beside the workgroups of the interior velocities.  Same sums as
+// sf_obc_volcons: blocks of 256 points by halving, then the blocks in order.
 // A serial chain that the interior's workgroups hide: the loads of B points a thread go out
 // together (one at a time, 2048 x 1024 took 220 us a substep for 178), B small enough that
 // the edges do not set the kernel's registers.
@@ -229,8 +232,9 @@ __device__ void open_faces(const PF<T> &p, const Open &ob, const T *zn, T *x_u, 
         k = k + 1;
         return f;
     };
+    static_assert(VB * CH == kEdgeRound, "a round of the edges");
     double area = 0.0, flux = 0.0;
-    for (int base = 0; base < n; base += VB * CH) {
+    for (int base = (int)blockIdx.x * kEdgeRound; base < n; base += ob.groups * kEdgeRound) {
 #pragma unroll 1
         for (int q0 = 0; q0 < CH; q0 += B) {
             T zl[B], zh[B], hl[B], hh[B], ml[B], mh[B];
@@ -321,15 +325,16 @@ __device__ void open_faces(const PF<T> &p, const Open &ob, const T *zn, T *x_u, 
     }
 }
 
-// Block of points of a velocity stage.  OPEN: the first eight blocks are the edges' -- one
-// works -- and the others leave the open edges' faces alone.
+// Block of points of a velocity stage.  OPEN: the first ob.blocks blocks (a multiple of
+// eight) are the edges' -- ob.groups of them work -- and the others leave the open edges'
+// faces alone.
 template <bool OPEN>
-__device__ __forceinline__ long long uv_point(bool band)
+__device__ __forceinline__ long long uv_point(bool band, const Open &ob)
 {
     unsigned b = blockIdx.x, nb = gridDim.x;
     if constexpr (OPEN) {
-        b -= 8;
-        nb -= 8;
+        b -= ob.blocks;
+        nb -= ob.blocks;
     }
     return (long long)(band ? (b & 7) * (nb >> 3) + (b >> 3) : b) * blockDim.x + threadIdx.x;
 }
@@ -407,11 +412,11 @@ template <typename T, bool OPEN>
 __global__ __launch_bounds__(256) void k_phys_pred_uv(Sub<T> a, Open ob)
 {
     if constexpr (OPEN) {
-        if (blockIdx.x == 0) open_faces(a.p, ob, (const T *)a.zs, a.us, a.vs);
-        if (blockIdx.x < 8) return;
+        if (blockIdx.x < (unsigned)ob.groups) open_faces(a.p, ob, (const T *)a.zs, a.us, a.vs);
+        if (blockIdx.x < (unsigned)ob.blocks) return;
     }
     const int szI = a.p.szI, szJ = a.p.szJ, L = szI - 1, M = szJ - 1;
-    const long long S2 = (long long)szI * szJ, W = szI, f = uv_point<OPEN>(a.band);
+    const long long S2 = (long long)szI * szJ, W = szI, f = uv_point<OPEN>(a.band, ob);
     if (f >= S2) return;
     const int i = (int)(f % szI), j = (int)(f / szI);
     if (!(OPEN && ((i == 1 && (ob.flags & SF_OBC_WEST)) || (i == L && (ob.flags & SF_OBC_EAST))))) {
@@ -511,11 +516,11 @@ template <typename T, bool OPEN>
 __global__ __launch_bounds__(256) void k_phys_corr_uv(Sub<T> a, Open ob)
 {
     if constexpr (OPEN) {
-        if (blockIdx.x == 0) open_faces(a.p, ob, (const T *)a.z2, a.u2, a.v2);
-        if (blockIdx.x < 8) return;
+        if (blockIdx.x < (unsigned)ob.groups) open_faces(a.p, ob, (const T *)a.z2, a.u2, a.v2);
+        if (blockIdx.x < (unsigned)ob.blocks) return;
     }
     const int szI = a.p.szI, szJ = a.p.szJ, L = szI - 1, M = szJ - 1;
-    const long long S2 = (long long)szI * szJ, W = szI, f = uv_point<OPEN>(a.band);
+    const long long S2 = (long long)szI * szJ, W = szI, f = uv_point<OPEN>(a.band, ob);
     if (f >= S2) return;
     const int i = (int)(f % szI), j = (int)(f / szI);
     if (!(OPEN && ((i == 1 && (ob.flags & SF_OBC_WEST)) || (i == L && (ob.flags & SF_OBC_EAST))))) {
@@ -577,15 +582,44 @@ int launch_phys(const sf_phys_fields *x, double dt, int first, double w1, void *
     hipStream_t s = sf::as_stream(stream);
     auto stages = [&](auto open, const Open &o) {
         constexpr bool OPEN = decltype(open)::value;
-        const dim3 grid(nb), uv(nb + (OPEN ? 8 : 0)), block(256);
+        const dim3 grid(nb), uv(nb + (OPEN ? o.blocks : 0)), block(256);
+        // the volume constraint in launches of its own, where the edges are shared out
+        auto volcons = [&](T *z, T *u, T *v) {
+            if (!OPEN || !ob->volcons || o.volcons) return (int)SF_OK;
+            return sf_obc_volcons(z, x->h, x->pm, x->pn, u, v, x->szI, x->szJ, sizeof(T) == 8 ? SF_FP64 : SF_FP32,
+                                  o.flags, 1, o.vc_work, o.vc_out, stream);
+        };
         hipLaunchKernelGGL((k_phys_pred_zeta<T, OPEN>), grid, block, 0, s, a, o);
         hipLaunchKernelGGL((k_phys_pred_uv<T, OPEN>), uv, block, 0, s, a, o);
+        int rc = volcons(a.zs, a.us, a.vs);
+        if (rc != SF_OK) return rc;
         hipLaunchKernelGGL((k_phys_corr_zeta<T, OPEN>), grid, block, 0, s, a, o);
         hipLaunchKernelGGL((k_phys_corr_uv<T, OPEN>), uv, block, 0, s, a, o);
+        rc = volcons(a.z2, a.u2, a.v2);
+        return rc != SF_OK ? rc : sf::check_launch("sf_phys_substep");
     };
-    if (ob && ob->flags) stages(std::true_type{}, *ob);
-    else stages(std::false_type{}, Open{});
-    return sf::check_launch("sf_phys_substep");
+    if (!ob || !ob->flags) return stages(std::false_type{}, Open{});
+    Open o = *ob;
+    // Without the volume constraint the edges are shared out, a round a workgroup.  With it,
+    // one workgroup sums and corrects them inside the launch as long as the interior's
+    // workgroups hide it, else the edges are shared out too and the constraint takes three
+    // launches of its own (about 8 us a stage).  One workgroup takes 5.6 ns a south or north
+    // face and 11.8 a west or east one (FP32 4.6 / 7.9: the loads of a column touch a line
+    // each), the interior 0.052 ns a point (FP32 0.024).  Per substep, one / shared out:
+    // FP64 2048 x 1024 308 / 326 us, 1000 x 600 93 / 101, 3000 x 200 114 / 99, 512 x 4096
+    // 367 / 340, 4096 x 64 108 / 62, 64 x 4096 194 / 85; FP32 149 / 158, 70 / 70, 90 / 70,
+    // 208 / 163, 94 / 45, 153 / 62.  The constraint in one workgroup on every grid took
+    // 4785 us at 262144 x 16 FP32.
+    constexpr bool F64 = sizeof(T) == 8;
+    const double we = ((o.flags & SF_OBC_WEST ? 1 : 0) + (o.flags & SF_OBC_EAST ? 1 : 0)) * (x->szJ - 2.0);
+    const double sn = ((o.flags & SF_OBC_SOUTH ? 1 : 0) + (o.flags & SF_OBC_NORTH ? 1 : 0)) * (x->szI - 2.0);
+    const double edges_ns = F64 ? 5.6 * sn + 11.8 * we : 4.6 * sn + 7.9 * we;
+    const bool one = edges_ns <= 0.75 * (F64 ? 0.052 : 0.024) * (double)S2 + 8000.0;
+    const int rounds = (int)((sn + we + (kEdgeRound - 1)) / kEdgeRound);
+    o.groups = o.volcons && one ? 1 : rounds;
+    o.blocks = (o.groups + 7) / 8 * 8;
+    o.volcons = o.volcons && one;
+    return stages(std::true_type{}, o);
 }
 
 }  // namespace
@@ -653,6 +687,7 @@ extern "C" int sf_phys_substep_open(const sf_phys_fields *x, const sf_open_bc *o
         ob.eu[e] = obc->vel_ext[e];
     }
     ob.volcons = obc->volcons;
+    ob.vc_work = volcons_work;
     ob.vc_out = volcons_out;
     if (precision == SF_FP64) return launch_phys<double>(x, dt, first, cff1, stream, nullptr, &ob);
     if (precision == SF_FP32) return launch_phys<float>(x, dt, first, cff1, stream, nullptr, &ob);
