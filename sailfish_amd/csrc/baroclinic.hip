@@ -55,21 +55,22 @@ __device__ __forceinline__ double pgf_diff(double r0f, double r1f, double r0p, d
     return fac3 * (C1 * C3 - C2 * C4);
 }
 
-// A block is 64 columns by four waves.  Per round, from the top, each wave takes LB levels
-// of both directions: their loads go out together, the differences of phi meet in LDS, and
-// every wave runs the columns' sums over the round.  Against a thread that walked its column
-// twice, once per direction: FP32 1024 x 512 x 32 161 -> 145 us (seven fields, 470 MB; the
-// FP64 differences take about 60 us of that), 386 x 258 x 40 45 -> 33, 90 x 60 x 20 19 -> 8;
-// FP64 1024 x 512 x 32 290 -> 243.
-template <class T, int LB>
+// A block is 256 / NW columns by NW level waves (NW by sf::level_waves).  Per round, from the
+// top, each wave takes LB levels of both directions: their loads go out together, the
+// differences of phi meet in LDS, and every wave runs the columns' sums over the round (one
+// level wave: from its registers).  Against a thread that walked its column twice, once per
+// direction: FP32 1024 x 512 x 32 (seven fields, 470 MB, without the density's 23 us) 167 ->
+// 148 us (the FP64 differences take about 60 us of that), 386 x 258 x 40 48 -> 36, 90 x 60 x 20
+// 19 -> 8, 3000 x 1500 x 4 (one level wave) 180 -> 165; FP64 1024 x 512 x 32 310 -> 250.
+template <class T, int LB, int NW>
 __global__ __launch_bounds__(256) void k_prsgrd(Col g, const T *rho, const T *z_r, const T *z_w, const T *Hz,
                                                 double grav, double rho0, T *ru, T *rv)
 {
-    constexpr int NW = 4, ROUND = NW * LB;
-    __shared__ double sP[2][2][ROUND][64];   // by buffer, direction, level of the round, column
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const long long f = (long long)sf::column_block(g.band) * 64 + lane;
+    constexpr int ROUND = NW * LB, COLS = 256 / NW;
+    __shared__ double sP[2][2][ROUND][NW > 1 ? COLS : 1];   // by buffer, direction, level of the round, column
+    const int col = threadIdx.x % COLS;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / COLS);
+    const long long f = (long long)sf::column_block(g.band) * COLS + col;
     const long long S2 = g.S2, W = g.szI;
     const int N = g.N, i = (int)(f % W), j = (int)(f / W), L = g.szI - 1, M = g.szJ - 1;
     const bool un = f < S2 && i >= 2 && i <= L - 1 && j >= 1 && j <= M - 1;
@@ -96,9 +97,11 @@ __global__ __launch_bounds__(256) void k_prsgrd(Col g, const T *rho, const T *z_
     // a round: levels top, top - 1, ...; the wave's are hi, hi - 1, ... (LB of them)
     for (int top = N - 2, buf = 0; top >= 0; top -= ROUND, buf ^= 1) {
         const int hi = top - wave * LB;
+        const bool mine = on && hi >= 0;   // the last round may end above the wave
         auto level = [&](int k) { return (long long)(k < 0 ? 0 : k) * S2 + f; };
         T hz[LB], hu[LB], hv[LB], xu[LB], xv[LB];
-        if (on) {
+        double pu[LB], pv[LB];
+        if (mine) {
             T r[LB + 1], rw[LB + 1], rs[LB + 1], z[LB + 1], zw[LB + 1], zs[LB + 1];
 #pragma unroll
             for (int q = 0; q <= LB; q++) {
@@ -121,23 +124,36 @@ __global__ __launch_bounds__(256) void k_prsgrd(Col g, const T *rho, const T *z_
             }
 #pragma unroll
             for (int q = 0; q < LB; q++) {
-                sP[buf][0][wave * LB + q][lane] = pgf_diff(r[q + 1], r[q], rw[q + 1], rw[q], z[q + 1], z[q], zw[q + 1], zw[q], fac3);
-                sP[buf][1][wave * LB + q][lane] = pgf_diff(r[q + 1], r[q], rs[q + 1], rs[q], z[q + 1], z[q], zs[q + 1], zs[q], fac3);
+                pu[q] = pgf_diff(r[q + 1], r[q], rw[q + 1], rw[q], z[q + 1], z[q], zw[q + 1], zw[q], fac3);
+                pv[q] = pgf_diff(r[q + 1], r[q], rs[q + 1], rs[q], z[q + 1], z[q], zs[q + 1], zs[q], fac3);
+                if constexpr (NW > 1) {
+                    sP[buf][0][wave * LB + q][col] = pu[q];
+                    sP[buf][1][wave * LB + q][col] = pv[q];
+                }
             }
         }
-        __syncthreads();   // the next round fills the other buffer
-        if (!on) continue;
-        double pu[LB], pv[LB];
+        if constexpr (NW > 1) __syncthreads();   // the next round fills the other buffer
+        if (!mine) continue;
+        if constexpr (NW > 1) {
 #pragma unroll
-        for (int m = 0; m < ROUND; m++) {
-            phiu = phiu + sP[buf][0][m][lane];
-            phiv = phiv + sP[buf][1][m][lane];
+            for (int m = 0; m < ROUND; m++) {
+                phiu = phiu + sP[buf][0][m][col];
+                phiv = phiv + sP[buf][1][m][col];
 #pragma unroll
-            for (int q = 0; q < LB; q++)
-                if (m == wave * LB + q) {
-                    pu[q] = phiu;
-                    pv[q] = phiv;
-                }
+                for (int q = 0; q < LB; q++)
+                    if (m == wave * LB + q) {
+                        pu[q] = phiu;
+                        pv[q] = phiv;
+                    }
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < LB; q++) {
+                phiu = phiu + pu[q];
+                phiv = phiv + pv[q];
+                pu[q] = phiu;
+                pv[q] = phiv;
+            }
         }
 #pragma unroll
         for (int q = 0; q < LB; q++) {
@@ -186,7 +202,8 @@ __global__ __launch_bounds__(256) void k_step3d_t(Col g, Tracers2<T> x, const T 
         auto level = [&](int k) { return (long long)(k < 0 ? 0 : (k < N ? k : N - 1)) * S2 + f; };
         T hu0[LB], hu1[LB], hv0[LB], hv1[LB], hzo[LB], hzn[LB];
         T c[NTR][LB + 2], e[NTR][LB], w[NTR][LB], n[NTR][LB], s[NTR][LB];
-        if (on) {
+        const bool mine = on && lo < N;   // the last round may end below the wave
+        if (mine) {
 #pragma unroll
             for (int q = 0; q < LB; q++) {
                 const long long b = level(lo + q);
@@ -218,7 +235,7 @@ __global__ __launch_bounds__(256) void k_step3d_t(Col g, Tracers2<T> x, const T 
             }
         }
         __syncthreads();   // the next round fills the other buffer
-        if (!on) continue;
+        if (!mine) continue;
         double Wk[LB + 1], Wr = Wlow;   // W at the tops of levels lo-1 .. lo+LB-1
         Wk[0] = Wlow;
 #pragma unroll
@@ -285,8 +302,13 @@ template <class T>
 int prsgrd_launch(sf_ctx *c, const void *rho, const void *z_r, const void *z_w, const void *Hz, double g,
                   double rho0, void *ru, void *rv, void *stream)
 {
-    hipLaunchKernelGGL((k_prsgrd<T, 2>), dim3(sf::column_grid(c->S2, 64)), dim3(256), 0, sf::as_stream(stream),
-                       col_of(c, sizeof(T)), (const T *)rho, (const T *)z_r, (const T *)z_w, (const T *)Hz, g, rho0, (T *)ru, (T *)rv);
+    auto go = [&](auto kernel, int cols) {
+        hipLaunchKernelGGL(kernel, dim3(sf::column_grid(c->S2, cols)), dim3(256), 0, sf::as_stream(stream),
+                           col_of(c, sizeof(T)), (const T *)rho, (const T *)z_r, (const T *)z_w, (const T *)Hz, g, rho0,
+                           (T *)ru, (T *)rv);
+    };
+    if (sf::level_waves(c, 16) == 4) go(k_prsgrd<T, 2, 4>, 64);
+    else go(k_prsgrd<T, 2, 1>, 256);
     return sf::check_launch("sf_prsgrd");
 }
 

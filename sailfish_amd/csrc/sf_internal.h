@@ -103,6 +103,19 @@ __device__ __forceinline__ unsigned column_pair_block(bool band)
     return band ? x * (gridDim.x >> 4) + k : k * 8 + x;
 }
 
+// Level waves of a kernel that can split a column's levels: four, unless the columns alone
+// give every SIMD (256 CUs of four) four waves and the column is short (at most `few` levels).
+// A split column repeats what belongs to the column (index division, metrics, the sums below
+// a wave's levels), which a few levels do not pay for: one / four waves at 4 levels, FP64
+// 3000 x 1500 set_maxflux 142 / 148 us, omega 104 / 139, pressure gradient 337 / 467, FP32
+// 68 / 117, 50 / 111, 189 / 287.  Where the lines lie, FP64 1024 x 512: set_maxflux 8 levels
+// 23.9 / 24.2, 16 levels 44.9 / 45.3 (700 x 400: 26.2 / 25.0); FP32 16 levels 24.4 / 24.5;
+// pressure gradient 16 levels 149 / 160 (FP32 72 / 79), 24 levels 232 / 231.
+inline int level_waves(const sf_ctx *c, size_t few)
+{
+    return c->S2 >= 4LL * 1024 * 64 && (size_t)c->szK <= few ? 1 : 4;
+}
+
 }  // namespace sf
 
 #define SF_REQUIRE(cond, ...)                 \

@@ -67,22 +67,29 @@ __device__ __forceinline__ bool isInnerCell(const G3 &g, long long f)
     const long long f = (long long)sf::column_block(g.band) * blockDim.x + threadIdx.x; \
     if (f >= g.S2) return;
 
-// Kernels whose levels are independent, or meet only in a sum: a block is kColumns columns
-// by kLevelWaves waves, a wave one run of levels lo .. hi-1 out of FIRST .. LAST-1.
-// BATCH_LEVEL: level K + q of a batch, the last one again past the run's end, so that a
-// batch's loads have no branch between them and are all in flight together.
-constexpr int kColumns = 64, kLevelWaves = 4, kBatch = 4;
+// Kernels whose levels are independent, or meet only in a sum: a block of 256 threads is
+// kThreads / LW columns by LW level waves (one wave's columns each); level wave w takes the
+// w-th run of levels lo .. hi-1 out of FIRST .. LAST-1.
+constexpr int kThreads = 256;
 #define LEVEL_WAVE_INDEX(FIRST, LAST)                                                               \
-    const long long f = (long long)sf::column_block(g.band) * kColumns + threadIdx.x % kColumns;     \
-    const int wave_ = __builtin_amdgcn_readfirstlane(threadIdx.x / kColumns);                        \
-    const int run_ = ((LAST) - (FIRST) + kLevelWaves - 1) / kLevelWaves;                             \
+    constexpr int COLS = kThreads / LW;                                                              \
+    const long long f = (long long)sf::column_block(g.band) * COLS + threadIdx.x % COLS;             \
+    const int wave_ = __builtin_amdgcn_readfirstlane(threadIdx.x / COLS);                            \
+    const int run_ = ((LAST) - (FIRST) + LW - 1) / LW;                                               \
     const int lo = (FIRST) + wave_ * run_ < (LAST) ? (FIRST) + wave_ * run_ : (LAST);                \
     const int hi = lo + run_ < (LAST) ? lo + run_ : (LAST);
-#define BATCH_LEVEL(q) (long long)(K + (q) < hi ? K + (q) : hi - 1)
-#define LAUNCH_LEVEL_WAVES(kern, lds, c, stream, ...)                                               \
-    hipLaunchKernelGGL(kern, dim3(sf::column_grid((c)->S2, kColumns)), dim3(kColumns * kLevelWaves), \
-                       lds, sf::as_stream(stream), __VA_ARGS__);                                     \
-    return sf::check_launch(__func__)
+
+// fn(K, n) for runs of n (a compile-time count) levels from K: four at a time, then the rest.
+// No branch stands between the loads of a run, so they are all in flight together.
+template <class F>
+__device__ __forceinline__ void level_batches(int lo, int hi, F &&fn)
+{
+    int K = lo;
+    for (; K + 4 <= hi; K += 4) fn(K, std::integral_constant<int, 4>{});
+    if (hi - K == 3) fn(K, std::integral_constant<int, 3>{});
+    else if (hi - K == 2) fn(K, std::integral_constant<int, 2>{});
+    else if (hi - K == 1) fn(K, std::integral_constant<int, 1>{});
+}
 
 // ---- addCoriolis (rhs_kernels.cpp:6-35) -------------------------------------------
 template <bool CHK>
@@ -554,22 +561,23 @@ void k_rhs3d_fused(G3 g, HG<T> h, A fomn, AG<T> Hz, AG<T> Wa, const int32_t *BC,
 // ---- set_maxflux (step3D_uv.kernels.cpp:372-405) ----------------------------------
 // the fluxes are stored with streaming (non-temporal) stores: no thread of the launch
 // reads them back.  Both fluxes of a level are formed together, so Hz is read once.
-// HBM-bound; against a thread per column: FP64 700 x 400 x 32 67 -> 56 us, 386 x 258 x 40
-// 37 -> 30, 1024 x 512 x 32 (five fields, 671 MB) 135 -> 140; FP32 63 -> 54 there.
-template <class T>
-__global__ __launch_bounds__(kColumns * kLevelWaves) void k_set_maxflux(G3 g, const T *u, const T *v, T *Huon,
-                                                                        T *Hvom, const T *Hz)
+// HBM-bound.  Against a thread that took its column's levels one by one: FP64 700 x 400 x 32
+// 59 -> 47 us, 386 x 258 x 40 34 -> 24, 1024 x 512 x 32 (five fields, 671 MB) 136 -> 134; FP32
+// 53 -> 44 there; few levels on a large grid (one level wave) FP64 1500 x 800 x 5 41 -> 34.
+template <class T, int LW>
+__global__ __launch_bounds__(kThreads) void k_set_maxflux(G3 g, const T *u, const T *v, T *Huon, T *Hvom, const T *Hz)
 {
     LEVEL_WAVE_INDEX(0, g.N)
     if (f >= g.S2) return;
     const bool un = isUNode(g, f), vn = isVNode(g, f);
     if (!un && !vn) return;   // the others have i, j >= 1: b - 1 and b - szI exist
     const T onu = un ? T(g.on_u[f]) : T(0), omv = vn ? T(g.om_v[f]) : T(0);
-    for (int K = lo; K < hi; K += kBatch) {
-        T hz[kBatch], hw[kBatch], hs[kBatch], uu[kBatch], vv[kBatch];
+    level_batches(lo, hi, [&](int K, auto n) {
+        constexpr int NB = decltype(n)::value;
+        T hz[NB], hw[NB], hs[NB], uu[NB], vv[NB];
 #pragma unroll
-        for (int q = 0; q < kBatch; q++) {
-            const long long b = BATCH_LEVEL(q) * g.S2 + f;
+        for (int q = 0; q < NB; q++) {
+            const long long b = (K + q) * g.S2 + f;
             hz[q] = Hz[b];
             hw[q] = Hz[b - 1];
             hs[q] = Hz[b - g.szI];
@@ -577,13 +585,12 @@ __global__ __launch_bounds__(kColumns * kLevelWaves) void k_set_maxflux(G3 g, co
             vv[q] = v[b];
         }
 #pragma unroll
-        for (int q = 0; q < kBatch; q++) {
-            if (K + q >= hi) break;
+        for (int q = 0; q < NB; q++) {
             const long long b = (K + q) * g.S2 + f;
             if (un) __builtin_nontemporal_store((((hz[q] + hw[q]) * T(0.5)) * uu[q]) * onu, Huon + b);
             if (vn) __builtin_nontemporal_store((((hz[q] + hs[q]) * T(0.5)) * vv[q]) * omv, Hvom + b);
         }
-    }
+    });
 }
 
 // ---- omega (step3D_uv.kernels.cpp:62-165) -----------------------------------------
@@ -610,63 +617,63 @@ __global__ __launch_bounds__(256) void k_omega(G3 g, double *W, A Hu, A Hv, cons
     W[N * S2 + f] = 0.0;
 }
 
-// omega of up to 64 levels (32 KB of LDS): W is written once per level instead of written, read
+// omega of up to 64 levels (at most 32 KB of LDS): W is written once per level instead of written, read
 // back and rewritten.  Each wave forms the divergences of its own levels into LDS; then
 // every wave runs the column's sum over all of them, so the partial sums and W = w -
 // (Ws * (z_w - zb)) / h are those of k_omega.  FP64 sums and correction for either type T.
 // Bound by HBM once enough loads are in flight: with a thread per column and the sums in
 // registers, each level's loads waited for the level before.  FP64 1024 x 512 x 32 (four
-// fields, 537 MB) 146 -> 117 us, 386 x 258 x 40 52 -> 24; FP32 100 -> 55, 49 -> 19.
-template <class T>
-__global__ __launch_bounds__(kColumns * kLevelWaves) void k_omega_split(G3 g, T *W, const T *Hu, const T *Hv,
-                                                                        const T *z_w, const int32_t *BC)
+// fields, 537 MB) 142 -> 113 us, 386 x 258 x 40 50 -> 21; FP32 91 -> 49, 47 -> 15; 1500 x 800 x 5
+// (one level wave) FP64 33 -> 26, FP32 22 -> 16.
+template <class T, int LW>
+__global__ __launch_bounds__(kThreads) void k_omega_split(G3 g, T *W, const T *Hu, const T *Hv, const T *z_w,
+                                                          const int32_t *BC)
 {
     extern __shared__ double div[];   // levels 1 .. N-1 of the block's columns
     LEVEL_WAVE_INDEX(1, g.N)
     const bool on = f < g.S2 && BC[f] < 0;
     const long long S2 = g.S2;
-    const int N = g.N, lane = threadIdx.x % kColumns;
-    auto d = [&](int K) -> double & { return div[(K - 1) * kColumns + lane]; };
+    const int N = g.N, col = threadIdx.x % COLS;
+    auto d = [&](int K) -> double & { return div[(K - 1) * COLS + col]; };
     if (on)
-        for (int K = lo; K < hi; K += kBatch) {
+        level_batches(lo, hi, [&](int K, auto n) {
             // levels up to N-1 of arrays of N+1 levels: b + szI exists
-            T u0[kBatch], u1[kBatch], v0[kBatch], v1[kBatch];
+            constexpr int NB = decltype(n)::value;
+            T u0[NB], u1[NB], v0[NB], v1[NB];
 #pragma unroll
-            for (int q = 0; q < kBatch; q++) {
-                const long long b = BATCH_LEVEL(q) * S2 + f;
+            for (int q = 0; q < NB; q++) {
+                const long long b = (K + q) * S2 + f;
                 u0[q] = Hu[b];
                 u1[q] = Hu[b + 1];
                 v0[q] = Hv[b];
                 v1[q] = Hv[b + g.szI];
             }
 #pragma unroll
-            for (int q = 0; q < kBatch; q++)
-                if (K + q < hi)
-                    d(K + q) = ((double)u1[q] - (double)u0[q]) + ((double)v1[q] - (double)v0[q]);
-        }
+            for (int q = 0; q < NB; q++) d(K + q) = ((double)u1[q] - (double)u0[q]) + ((double)v1[q] - (double)v0[q]);
+        });
     double zb = 0.0, h = 0.0;
     if (on) {
         zb = (double)z_w[f];
         h = (double)z_w[(long long)(N - 1) * S2 + f] - zb;
     }
-    __syncthreads();
+    if constexpr (LW > 1) __syncthreads();
     if (!on) return;
     double w = 0.0;
     for (int K = 1; K < lo; K++) w = w - d(K);
     double Ws = w;
     for (int K = lo; K < N; K++) Ws = Ws - d(K);
-    for (int K = lo; K < hi; K += kBatch) {
-        T z[kBatch];
+    level_batches(lo, hi, [&](int K, auto n) {
+        constexpr int NB = decltype(n)::value;
+        T z[NB];
 #pragma unroll
-        for (int q = 0; q < kBatch; q++) z[q] = z_w[BATCH_LEVEL(q) * S2 + f];
+        for (int q = 0; q < NB; q++) z[q] = z_w[(K + q) * S2 + f];
 #pragma unroll
-        for (int q = 0; q < kBatch; q++) {
-            if (K + q >= hi) break;
+        for (int q = 0; q < NB; q++) {
             w = w - d(K + q);
             W[(K + q) * S2 + f] = T(w - (Ws * ((double)z[q] - zb)) / h);
         }
-    }
-    if (threadIdx.x < kColumns) {
+    });
+    if (wave_ == 0) {
         W[f] = T(0);
         W[(long long)N * S2 + f] = T(0);
     }
@@ -1549,12 +1556,29 @@ extern "C" int sf_rhs3d_f32(sf_ctx *c, const double *fomn, const float *u, const
     return rhs3d_launch<float>(c, fomn, u, v, Huon, Hvom, W, Hz, BC, ru, rv, launch_threads, cor, adv, stream);
 }
 
+// launch of a kernel of kThreads / LW columns a block
+template <class K, class... Args>
+static void launch_level_waves(K kernel, int LW, size_t lds, sf_ctx *c, void *stream, Args... args)
+{
+    hipLaunchKernelGGL(kernel, dim3(sf::column_grid(c->S2, kThreads / LW)), dim3(kThreads), lds, sf::as_stream(stream),
+                       args...);
+}
+
+template <class T>
+static int set_maxflux_launch(sf_ctx *c, const T *u, const T *v, T *Huon, T *Hvom, const T *Hz, void *stream)
+{
+    const G3 g = grid3(c, sizeof(T));
+    if (sf::level_waves(c, 64 / sizeof(T)) == 4) launch_level_waves(k_set_maxflux<T, 4>, 4, 0, c, stream, g, u, v, Huon, Hvom, Hz);
+    else launch_level_waves(k_set_maxflux<T, 1>, 1, 0, c, stream, g, u, v, Huon, Hvom, Hz);
+    return sf::check_launch("sf_set_maxflux");
+}
+
 extern "C" int sf_set_maxflux(sf_ctx *c, const double *u, const double *v, double *Huon, double *Hvom,
                               const double *Hz, void *stream)
 {
     CTX3(c);
     SF_REQUIRE(u && v && Huon && Hvom && Hz, "sf_set_maxflux: null field");
-    LAUNCH_LEVEL_WAVES(k_set_maxflux<double>, 0, c, stream, grid3(c, sizeof(double)), u, v, Huon, Hvom, Hz);
+    return set_maxflux_launch(c, u, v, Huon, Hvom, Hz, stream);
 }
 
 extern "C" int sf_set_maxflux_f32(sf_ctx *c, const float *u, const float *v, float *Huon, float *Hvom,
@@ -1562,15 +1586,19 @@ extern "C" int sf_set_maxflux_f32(sf_ctx *c, const float *u, const float *v, flo
 {
     CTX3(c);
     SF_REQUIRE(u && v && Huon && Hvom && Hz, "sf_set_maxflux_f32: null field");
-    LAUNCH_LEVEL_WAVES(k_set_maxflux<float>, 0, c, stream, grid3(c, sizeof(float)), u, v, Huon, Hvom, Hz);
+    return set_maxflux_launch(c, u, v, Huon, Hvom, Hz, stream);
 }
 
 template <class T>
 static int omega_launch(sf_ctx *c, T *W, const T *Huon, const T *Hvom, const T *z_w, const int32_t *BC,
                         void *stream)
 {
-    const size_t lds = sizeof(double) * kColumns * (size_t)(c->szK - 1);
-    LAUNCH_LEVEL_WAVES(k_omega_split<T>, lds, c, stream, grid3(c, sizeof(T)), W, Huon, Hvom, z_w, BC);
+    const G3 g = grid3(c, sizeof(T));
+    const int lw = sf::level_waves(c, 64 / sizeof(T));
+    const size_t lds = sizeof(double) * (kThreads / lw) * (size_t)(g.N - 1);
+    if (lw == 4) launch_level_waves(k_omega_split<T, 4>, 4, lds, c, stream, g, W, Huon, Hvom, z_w, BC);
+    else launch_level_waves(k_omega_split<T, 1>, 1, lds, c, stream, g, W, Huon, Hvom, z_w, BC);
+    return sf::check_launch("sf_omega");
 }
 
 extern "C" int sf_omega(sf_ctx *c, double *W, const double *Huon, const double *Hvom, const double *z_w,
