@@ -594,6 +594,9 @@ __global__ __launch_bounds__(kThreads) void k_set_maxflux(G3 g, const T *u, cons
 }
 
 // ---- omega (step3D_uv.kernels.cpp:62-165) -----------------------------------------
+// Deep columns, a thread each: a chain of dependent levels.  Launched in blocks of 64 columns,
+// as set_maxflux's split columns, so that a column runs on the XCD whose L2 holds its fluxes
+// (24 x 18 x 100 after set_maxflux 150 -> 97 us against blocks of 256).
 __global__ __launch_bounds__(256) void k_omega(G3 g, double *W, A Hu, A Hv, const double *z_w,
                                                const int32_t *BC)
 {
@@ -1608,7 +1611,9 @@ extern "C" int sf_omega(sf_ctx *c, double *W, const double *Huon, const double *
     SF_REQUIRE(W && Huon && Hvom && z_w && BC, "sf_omega: null field");
     if (c->szK <= 64) return omega_launch<double>(c, W, Huon, Hvom, z_w, BC, stream);
     const long long n3 = (c->szK + 1LL) * c->S2;
-    LAUNCH_COLUMNS(k_omega, c, stream, grid3(c, sizeof(double)), W, A{Huon, n3}, A{Hvom, n3}, z_w, BC);
+    hipLaunchKernelGGL(k_omega, dim3(sf::column_grid(c->S2, 64)), dim3(64), 0, sf::as_stream(stream),
+                       grid3(c, sizeof(double)), W, A{Huon, n3}, A{Hvom, n3}, z_w, BC);
+    return sf::check_launch("sf_omega");
 }
 
 extern "C" int sf_omega_f32(sf_ctx *c, float *W, const float *Huon, const float *Hvom, const float *z_w,

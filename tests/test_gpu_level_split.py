@@ -158,3 +158,42 @@ def test_few_levels_on_a_large_grid(dt):
     ratio = [a / b for a, b in zip(level[4], level[12])]
     print(f"[few levels] {dt} set_maxflux, omega, prsgrd: {ratio}", file=sys.stderr, flush=True)
     assert max(ratio) < 1.25, ratio
+
+
+def test_deep_omega_reads_its_own_chiplets_fluxes():
+    """24 x 18 x 100, deeper than the split form of omega takes: set_maxflux and omega after each
+    other against each alone, repeated.  Columns on the same XCD in both read the fluxes from
+    that XCD's L2: 1.3 times; on different ones it took 1.9."""
+    import torch
+    from sailfish_amd import mod_operators as ops
+    print("[case] deep omega after set_maxflux", file=sys.stderr, flush=True)
+    _c, GRID, OCEAN, BOUNDARY = _fields(24, 18, 100, "f64")
+    c, BC = ops.ctx_of(GRID), BOUNDARY.device_maps()["bcIdxFieldIdx2"]
+    Hu, Hv, W = OCEAN.Huon.reshape(-1), OCEAN.Hvom.reshape(-1), OCEAN.W.reshape(-1)
+    Hz, z_w = GRID.Hz.reshape(-1), GRID.z_w.reshape(-1)
+    maxflux = lambda: ops.set_maxflux(None, None, (OCEAN.u_t2, OCEAN.v_t2, Hu, Hv, Hz), ctx=c)
+    omega = lambda: ops.omega(None, None, (W, OCEAN.u_t2, OCEAN.v_t2, Hu, Hv, z_w, BC), ctx=c)
+
+    def us(*fns):
+        g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            for fn in fns:
+                fn()
+            with torch.cuda.graph(g, stream=s):
+                for _ in range(20):
+                    for fn in fns:
+                        fn()
+        t = []
+        for _ in range(7):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            g.replay()
+            b.record()
+            torch.cuda.synchronize()
+            t.append(a.elapsed_time(b) * 50.0)
+        return sorted(t)[3]
+
+    ratio = us(maxflux, omega) / (us(maxflux) + us(omega))
+    print(f"[deep omega] {ratio}", file=sys.stderr, flush=True)
+    assert ratio < 1.6, ratio
