@@ -1693,17 +1693,21 @@ void ens_launch_tj(sf_ens *e, int first, double w1, int rot, hipStream_t s)
                                e->list, e->order, rot, w1);
         return;
     }
+    // The tile loop's own registers take FP64's one-point-a-thread form (512 threads) past 128:
+    // one workgroup a CU where two of 256 threads fit.  21 basins of 256 x 128 to 1024 x 512, a
+    // grid of 512: 5.76 ms for twelve substeps with 512 threads, 4.51 with 256.
+    constexpr int NP = sizeof(T) == 8 && TJ == 8 ? 256 : NT;
     if (first && e->nts)
-        hipLaunchKernelGGL((k_phys_ensemble<T, TI, TJ, NT, true, true>), dim3(G), dim3(NT), 0, s, m, e->list,
+        hipLaunchKernelGGL((k_phys_ensemble<T, TI, TJ, NP, true, true>), dim3(G), dim3(NP), 0, s, m, e->list,
                            e->ntiles, e->order, rot, w1);
     else if (first)
-        hipLaunchKernelGGL((k_phys_ensemble<T, TI, TJ, NT, true, false>), dim3(G), dim3(NT), 0, s, m, e->list,
+        hipLaunchKernelGGL((k_phys_ensemble<T, TI, TJ, NP, true, false>), dim3(G), dim3(NP), 0, s, m, e->list,
                            e->ntiles, e->order, rot, w1);
     else if (e->nts)
-        hipLaunchKernelGGL((k_phys_ensemble<T, TI, TJ, NT, false, true>), dim3(G), dim3(NT), 0, s, m, e->list,
+        hipLaunchKernelGGL((k_phys_ensemble<T, TI, TJ, NP, false, true>), dim3(G), dim3(NP), 0, s, m, e->list,
                            e->ntiles, e->order, rot, w1);
     else
-        hipLaunchKernelGGL((k_phys_ensemble<T, TI, TJ, NT, false, false>), dim3(G), dim3(NT), 0, s, m, e->list,
+        hipLaunchKernelGGL((k_phys_ensemble<T, TI, TJ, NP, false, false>), dim3(G), dim3(NP), 0, s, m, e->list,
                            e->ntiles, e->order, rot, w1);
 }
 
