@@ -33,7 +33,7 @@ import torch
 from . import _lib
 from . import mod_operators as ops
 from .main3d import initial_depths
-from .phys2d import PhysStepper, issue_substeps, sf_phys_fields
+from .phys2d import COUNTER, STATE, STEPPER, PhysStepper, issue_substeps, methods, own, sf_phys_fields
 from .rhs import rhs3d
 
 P = C.c_void_p
@@ -144,6 +144,43 @@ class CoupledState:
                                 w2p, w2c, ab)
 
 
+COUPLING = methods(CoupledState, "couple_fields")
+
+
+def _coupled_substeps(compTimes, OCEAN, st: CoupledState, lib, stream):
+    """The nfast + 1 coupled barotropic substeps of a baroclinic step."""
+    compTimes.first2DTimeStep()
+    nsub = compTimes.nfast + 1
+    if nsub > 0 and own(compTimes, COUNTER) and own(OCEAN, STATE) and own(st, COUPLING) and own(st.stepper, STEPPER):
+        OCEAN.Zt_avg1.zero_()
+        OCEAN.DU_avg1.zero_()
+        OCEAN.DV_avg1.zero_()
+        a = st.stepper.fields(OCEAN)
+        cp = st.couple_fields(compTimes.iic - compTimes.ntfirst, 1, compTimes.weight2)
+        w2 = [filtered_transport_weights(compTimes.weight2, iif) for iif in range(1, nsub + 1)]
+        w2p, w2c = ((C.c_double * nsub)(*w) for w in zip(*w2))
+        issue_substeps(compTimes, OCEAN, nsub, "sf_phys_run", lambda n, w1, _clamp, done: lib.sf_phys_run(
+            C.byref(a), C.addressof(cp), w2p, w2c, None, None, None, st.stepper.precision, float(compTimes.dtfast), 1,
+            w1, n, int(st.fused), st.tile_j, stream, C.byref(done)))
+        return
+    for _ in range(nsub):     # a caller's own counter, state or step
+        if compTimes.isFirst2DStep():
+            OCEAN.Zt_avg1.zero_()
+            OCEAN.DU_avg1.zero_()
+            OCEAN.DV_avg1.zero_()
+        compTimes.next2DTimeStep()
+        OCEAN.cycleTimes2D()
+        a = st.stepper.fields(OCEAN)
+        cp = st.couple_fields(compTimes.iic - compTimes.ntfirst, compTimes.iif, compTimes.weight2)
+        common = (st.stepper.precision, float(compTimes.dtfast), int(compTimes.iif == 1), compTimes.cff1())
+        if st.fused:
+            _lib.check(lib.sf_phys_substep_coupled_fused(C.byref(a), C.byref(cp), *common, st.tile_j, stream),
+                       "sf_phys_substep_coupled_fused")
+        else:
+            _lib.check(lib.sf_phys_substep_coupled(C.byref(a), C.byref(cp), *common, stream),
+                       "sf_phys_substep_coupled")
+
+
 def coupled_step(compTimes, GRID, OCEAN, BOUNDARY, st: CoupledState, history=None):
     """One baroclinic step of the coupled form."""
     c = ops.ctx_of(GRID)
@@ -164,18 +201,7 @@ def coupled_step(compTimes, GRID, OCEAN, BOUNDARY, st: CoupledState, history=Non
                                    OCEAN.u_t2.data_ptr(), OCEAN.v_t2.data_ptr(), st.sustr.data_ptr(),
                                    st.svstr.data_ptr(), st.rdrg, st.rufrc.data_ptr(), st.rvfrc.data_ptr(), stream),
                "sf_couple_rufrc")
-    compTimes.first2DTimeStep()
-    OCEAN.Zt_avg1.zero_()
-    OCEAN.DU_avg1.zero_()
-    OCEAN.DV_avg1.zero_()
-    nsub = compTimes.nfast + 1
-    a = st.stepper.fields(OCEAN)
-    cp = st.couple_fields(compTimes.iic - compTimes.ntfirst, 1, compTimes.weight2)
-    w2 = [filtered_transport_weights(compTimes.weight2, iif) for iif in range(1, nsub + 1)]
-    w2p, w2c = ((C.c_double * nsub)(*w) for w in zip(*w2))
-    issue_substeps(compTimes, OCEAN, nsub, "sf_phys_run", lambda n, w1, _clamp, done: lib.sf_phys_run(
-        C.byref(a), C.addressof(cp), w2p, w2c, None, None, None, st.stepper.precision, float(compTimes.dtfast), 1, w1,
-        n, int(st.fused), st.tile_j, stream, C.byref(done)))
+    _coupled_substeps(compTimes, OCEAN, st, lib, stream)
     if history is not None:
         history.maybe_write(compTimes, OCEAN)
     st.Hz_old.copy_(GRID.Hz)

@@ -66,6 +66,10 @@ class T_OCEAN:
 
     def cycleTimes2D(self):
         """mod_ocean.py:120-155"""
+        if type(self) is not T_OCEAN:     # a subclass may keep its views elsewhere
+            for name in _ROT2D:
+                self._rotate(self, name)
+            return
         d = self.__dict__
         for t0, t1, t2 in _VIEWS2D:
             d[t0], d[t1], d[t2] = d[t1], d[t2], d[t0]

@@ -11,6 +11,7 @@ import numpy as np
 import torch
 
 from . import _lib
+from .mod_comptimes import CompTimes
 from .mod_constants import g as G_CONST
 from .mod_ocean import T_OCEAN, _VIEWS2D
 
@@ -137,11 +138,29 @@ class PhysStepper:
         _lib.check(rc, "sf_phys_substep")
 
 
+def methods(cls, *names):
+    """``cls`` and the functions it has under ``names`` now (see ``own``)."""
+    return cls, {n: vars(cls)[n] for n in names}
+
+
+def own(obj, cls_methods) -> bool:
+    """``obj`` is of that very class and none of the methods was replaced, on it or on the
+    class: calling them, once or not at all, is known to do nothing else."""
+    cls, fns = cls_methods
+    return type(obj) is cls and vars(obj).keys().isdisjoint(fns) and all(vars(cls)[n] is f for n, f in fns.items())
+
+
+COUNTER = methods(CompTimes, "first2DTimeStep", "isFirst2DStep", "next2DTimeStep", "cff1")
+STATE = methods(T_OCEAN, "cycleTimes2D")
+STEPPER = methods(PhysStepper, "fields", "step")
+
+
 def issue_substeps(compTimes, OCEAN, nsub: int, what: str, issue, clamp=None):
     """``nsub`` substeps through one native call: advances the 2D time counter, collects
     each substep's averaging weight (and ``clamp(time2D)``), calls
     ``issue(nsub, weights, clamps, done)`` and rotates the host's views as the substeps did.
-    If a substep fails, counter and views stop there, as a loop of single substeps would."""
+    If a substep fails, counter and views stop there, as a loop of single substeps would.
+    For a counter and a state that are ``own``: theirs is the only work between substeps."""
     w = (C.c_double * max(nsub, 1))()
     cl = (C.c_double * max(nsub, 1))() if clamp is not None else None
     times = []
@@ -166,14 +185,14 @@ def run_phys(compTimes, GRID, OCEAN, nsteps: int, stepper: PhysStepper | None = 
     """``nsteps`` physics substeps (next2DTimeStep, cycleTimes2D, substep); the
     first substep of the run is forward/backward Euler."""
     st = stepper or PhysStepper(GRID, OCEAN)
-    if type(st).step is PhysStepper.step and type(OCEAN).cycleTimes2D is T_OCEAN.cycleTimes2D:
+    if own(st, STEPPER) and own(OCEAN, STATE) and own(compTimes, COUNTER):
         a = st.fields(OCEAN)
         ob = (C.addressof(st.open_bc), st.vc_work.data_ptr(), st.vc_out.data_ptr()) if st.open_edges else (None,) * 3
         issue_substeps(compTimes, OCEAN, int(nsteps), "sf_phys_run", lambda n, w1, _clamp, done: st.lib.sf_phys_run(
             C.byref(a), None, None, None, *ob, st.precision, float(compTimes.dtfast), int(bool(start_first)), w1, n,
             int(st.fused), st.tile_j, _lib.stream_handle(), C.byref(done)))
         return st
-    for n in range(int(nsteps)):     # a caller's own step or state class
+    for n in range(int(nsteps)):     # a caller's own step, state or counter
         compTimes.next2DTimeStep()
         OCEAN.cycleTimes2D()
         st.step(compTimes, OCEAN, first=(start_first and n == 0))

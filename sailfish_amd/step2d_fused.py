@@ -19,6 +19,7 @@ import torch
 from . import _lib
 from . import mod_operators as ops
 from .mod_boundary import clamped_value
+from .phys2d import COUNTER, STATE, issue_substeps, methods, own
 
 _I32P = C.POINTER(C.c_int32)
 SF_SUBSTEP_ZERO_VBAR = 1
@@ -123,8 +124,8 @@ class FusedStepper:
         _lib.check(rc, "sf_step2d_substep")
 
     def run(self, compTimes, OCEAN, nsub: int, zero_vbar: bool = False):
-        """``nsub`` substeps (next2DTimeStep, cycleTimes2D, step) through one native call."""
-        from .phys2d import issue_substeps
+        """``nsub`` substeps (next2DTimeStep, cycleTimes2D, step) through one native call
+        (see ``issue_substeps``)."""
         a = self.fields(OCEAN)
         flags = SF_SUBSTEP_ZERO_VBAR if zero_vbar else 0
         issue_substeps(compTimes, OCEAN, nsub, "sf_step2d_run", lambda n, w1, cl, done: self.lib.sf_step2d_run(
@@ -155,6 +156,17 @@ def step2d_substep(compTimes, GRID, OCEAN, BOUNDARY, zero_vbar: bool = False):
     _stepper(GRID, OCEAN, BOUNDARY).step(compTimes, OCEAN, zero_vbar=zero_vbar)
 
 
+STEPPER = methods(FusedStepper, "fields", "step", "run")
+
+
 def step2d_run(compTimes, GRID, OCEAN, BOUNDARY, nsub: int, zero_vbar: bool = False):
     """``nsub`` fused substeps, each after next2DTimeStep and cycleTimes2D."""
-    _stepper(GRID, OCEAN, BOUNDARY).run(compTimes, OCEAN, int(nsub), zero_vbar=zero_vbar)
+    if own(compTimes, COUNTER) and own(OCEAN, STATE):
+        st = _stepper(GRID, OCEAN, BOUNDARY)
+        if own(st, STEPPER):
+            st.run(compTimes, OCEAN, int(nsub), zero_vbar=zero_vbar)
+            return
+    for _ in range(int(nsub)):     # a caller's own step, state or counter
+        compTimes.next2DTimeStep()
+        OCEAN.cycleTimes2D()
+        step2d_substep(compTimes, GRID, OCEAN, BOUNDARY, zero_vbar=zero_vbar)
