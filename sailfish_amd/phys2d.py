@@ -161,6 +161,8 @@ def issue_substeps(compTimes, OCEAN, nsub: int, what: str, issue, clamp=None):
     ``issue(nsub, weights, clamps, done)`` and rotates the host's views as the substeps did.
     If a substep fails, counter and views stop there, as a loop of single substeps would.
     For a counter and a state that are ``own``: theirs is the only work between substeps."""
+    if nsub < 0:
+        return
     w = (C.c_double * max(nsub, 1))()
     cl = (C.c_double * max(nsub, 1))() if clamp is not None else None
     times = []

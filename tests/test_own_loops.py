@@ -203,3 +203,17 @@ def test_method_replaced_on_the_class(log, monkeypatch):
     ct, oc, st = _counter(log), _state(log), _stepper(log)
     run_phys(ct, GRID, oc, 3, st)
     assert log == ["next", "substep"] * 3
+
+
+@pytest.mark.parametrize("nsub", [-1, -2, -5])
+def test_negative_counts_do_nothing(log, nsub):
+    ct, oc = _counter(log), _state(log)
+    grid = types.SimpleNamespace(**vars(GRID), _sf_fused=_fused(log))
+    slots = [oc.slot_of("zeta", f"t{k}") for k in range(3)]
+    run_phys(ct, GRID, oc, nsub, _stepper(log))
+    main2d(ct, grid, oc, None, nsub, fused=True)
+    step2d_fused.step2d_run(ct, grid, oc, None, nsub)
+    grid._sf_fused.run(ct, oc, nsub)
+    phys2d.issue_substeps(ct, oc, nsub, "x", lambda *a: _lib.SF_ERR_ARG)
+    assert (ct.iif, ct.time2D) == (0, 0.0) and not log
+    assert [oc.slot_of("zeta", f"t{k}") for k in range(3)] == slots
