@@ -865,15 +865,15 @@ __global__ __launch_bounds__(256) void k_step3d_uv(G3 g, UVArgs<T> a, double cff
 // FP32 202 -> 181.
 //
 // Addressing: an array's scalar base, advanced per level and passed through an empty asm
-// statement so that the unrolled levels keep no bases of their own, plus the column's 32-bit
-// byte offset.
-template <class T>
-__device__ __forceinline__ T ldc(const T *p, uint32_t o)
+// statement so that the unrolled levels keep no bases of their own, plus the column's byte
+// offset O: 32 bits, or 64 where a level passes 4 GiB.
+template <class T, class O>
+__device__ __forceinline__ T ldc(const T *p, O o)
 {
     return *(const __attribute__((address_space(1))) T *)((const __attribute__((address_space(1))) char *)p + o);
 }
-template <class T>
-__device__ __forceinline__ void stc(T *p, uint32_t o, T v)
+template <class T, class O>
+__device__ __forceinline__ void stc(T *p, O o, T v)
 {
     *(__attribute__((address_space(1))) T *)((__attribute__((address_space(1))) char *)p + o) = v;
 }
@@ -899,7 +899,7 @@ __device__ __forceinline__ long long level_start(int K, int N, long long S2)
     return (K < N ? K : N - 1) * S2;
 }
 
-template <class T, int NMAX>
+template <class T, int NMAX, class O>
 __global__ __launch_bounds__(64) void k_step3d_uv_col(G3 g, UVArgs<T> a, double cff, double lambda, double Dt)
 {
     const bool vdir = sf::column_pair_second();
@@ -911,8 +911,8 @@ __global__ __launch_bounds__(64) void k_step3d_uv_col(G3 g, UVArgs<T> a, double 
     if (!(vdir ? vn : un)) return;
     __shared__ T sds[NMAX][64];
     T D[NMAX], R[NMAX];
-    const uint32_t d = (uint32_t)((vdir ? g.szI : 1) * (long long)sizeof(T));
-    const uint32_t fo = (uint32_t)(f * (long long)sizeof(T)), fd = fo - d;
+    const O d = (O)((vdir ? g.szI : 1) * (long long)sizeof(T));
+    const O fo = (O)(f * (long long)sizeof(T)), fd = fo - d;
     const T mldt = T((-lambda) * Dt);
     const T *xold = vdir ? a.tmpV : a.tmpU, *r = vdir ? a.rv : a.ru;
     T *x = vdir ? a.v : a.u;
@@ -1002,7 +1002,7 @@ __global__ __launch_bounds__(64) void k_step3d_uv_col(G3 g, UVArgs<T> a, double 
     };
     // adjustBarotropicVelocity of one direction: yk(K) the stored velocity, hd the byte
     // offset of the neighbour the thickness averages with
-    auto barotropic = [&](bool kept, const T *y, uint32_t hd, const double *Davg, const double *met, T *t1, T *t2) {
+    auto barotropic = [&](bool kept, const T *y, O hd, const double *Davg, const double *met, T *t1, T *t2) {
         double Hsum = 0.0, Hy = 0.0;
         // four levels' loads at a time, the last level again past the column's end
 #pragma unroll
@@ -1049,7 +1049,7 @@ __global__ __launch_bounds__(64) void k_step3d_uv_col(G3 g, UVArgs<T> a, double 
             }
         }
         back_store(a.v, 0.0, true);
-        barotropic(true, a.v, fo - (uint32_t)(g.szI * (long long)sizeof(T)), a.DV_avg1, g.om_v, a.vbar_t1, a.vbar_t2);
+        barotropic(true, a.v, fo - (O)(g.szI * (long long)sizeof(T)), a.DV_avg1, g.om_v, a.vbar_t1, a.vbar_t2);
     }
 }
 
@@ -1678,17 +1678,20 @@ extern "C" int sf_set_lateral_uv_bcs_f32(sf_ctx *c, double t, float *u, float *v
 template <class T>
 static int step3d_uv_launch(sf_ctx *c, const UVArgs<T> &a, double cff, double lambda, double Dt, void *stream)
 {
-    if (c->szK > SF_STEP3D_REG_LEVELS) {
-        LAUNCH_COLUMNS(k_step3d_uv<T>, c, stream, grid3(c, sizeof(T)), a, cff, lambda, Dt);
-    }
-    SF_REQUIRE(c->S2 * sizeof(T) < (1ull << 32), "sf_step3d_uv: a level of %lld points exceeds 4 GiB", c->S2);
-    // by_levels: the fewest levels an instance holds; registers and LDS of the unused ones
-    // would cost waves (FP64: 3 waves per SIMD up to 24 levels, 2 up to 48, 1 to 64)
-    return by_levels(c->szK, [&](auto nmax) {
-        hipLaunchKernelGGL((k_step3d_uv_col<T, decltype(nmax)::value>), dim3(2 * sf::column_grid(c->S2, 64)), dim3(64), 0,
-                           sf::as_stream(stream), grid3(c, sizeof(T)), a, cff, lambda, Dt);
+    auto columns = [&](auto nmax, auto off) {
+        hipLaunchKernelGGL((k_step3d_uv_col<T, decltype(nmax)::value, decltype(off)>),
+                           dim3(2 * sf::column_grid(c->S2, 64)), dim3(64), 0, sf::as_stream(stream),
+                           grid3(c, sizeof(T)), a, cff, lambda, Dt);
         return sf::check_launch("sf_step3d_uv");
-    });
+    };
+    // by_levels: the fewest levels an instance holds; registers and LDS of the unused ones
+    // would cost waves (FP64: 3 waves per SIMD up to 24 levels, 2 up to 48, 1 to 64).  Levels
+    // past 4 GiB have the 16-level instance alone: the fields of 17 such levels fit no card.
+    const bool wide = c->S2 * sizeof(T) >= (1ull << 32);
+    if (!wide && c->szK <= SF_STEP3D_REG_LEVELS)
+        return by_levels(c->szK, [&](auto nmax) { return columns(nmax, uint32_t{}); });
+    if (wide && c->szK <= 16) return columns(std::integral_constant<int, 16>{}, uint64_t{});
+    LAUNCH_COLUMNS(k_step3d_uv<T>, c, stream, grid3(c, sizeof(T)), a, cff, lambda, Dt);
 }
 
 extern "C" int sf_step3d_uv(sf_ctx *c, double *u, double *v, const double *ru, const double *rv, double *ubar_t1,
