@@ -303,7 +303,7 @@ int prsgrd_launch(sf_ctx *c, const void *rho, const void *z_r, const void *z_w, 
                   double rho0, void *ru, void *rv, void *stream)
 {
     auto go = [&](auto kernel, int cols) {
-        hipLaunchKernelGGL(kernel, dim3(sf::column_grid(c->S2, cols)), dim3(256), 0, sf::as_stream(stream),
+        hipLaunchKernelGGL(kernel, sf::wide_grid(sf::column_grid(c->S2, cols), 256), dim3(256), 0, sf::as_stream(stream),
                            col_of(c, sizeof(T)), (const T *)rho, (const T *)z_r, (const T *)z_w, (const T *)Hz, g, rho0,
                            (T *)ru, (T *)rv);
     };
@@ -323,7 +323,7 @@ int tracer_launch(sf_ctx *c, int ntr, const void *const *t, void *const *tn, con
         x.tn[m] = (T *)tn[m];
     }
     auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(sf::column_grid(c->S2, 64)), dim3(256), 0, sf::as_stream(stream),
+        hipLaunchKernelGGL(kernel, sf::wide_grid(sf::column_grid(c->S2, 64), 256), dim3(256), 0, sf::as_stream(stream),
                            col_of(c, sizeof(T)), x, (const T *)Huon, (const T *)Hvom, (const T *)Hz_old,
                            (const T *)Hz_new, dt);
     };

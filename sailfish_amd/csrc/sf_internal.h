@@ -90,17 +90,27 @@ inline unsigned grid1d(long long n, int block = kBlock1D)
 // tracer step 503 -> 520.  So bands up to 100 MB a field.
 constexpr double kBandBytes = 100e6;
 inline unsigned column_grid(long long n, int block = kBlock1D) { return (grid1d(n, block) + 7) / 8 * 8; }
+// The grid of `blocks` (a multiple of 16 or 8) blocks of `threads`: a launch takes fewer than
+// 2^32 threads along x, so more of them go to rows of blocks (no bands there: fields of that
+// size pass kBandBytes by far).
+inline dim3 wide_grid(unsigned blocks, unsigned threads)
+{
+    unsigned y = 1;
+    while ((unsigned long long)(blocks / y + 16) * threads >= (1ull << 32)) y *= 2;
+    return y == 1 ? dim3(blocks) : dim3((blocks / y + 16) / 16 * 16, y);
+}
 __device__ __forceinline__ unsigned column_block(bool band)
 {
-    return band ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+    return band ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.y * gridDim.x + blockIdx.x;
 }
-// the same with two blocks per block of columns (grid 2 * column_grid), one after the other
+// the same with two blocks per block of columns (grid of 2 * column_grid), one after the other
 // on the same XCD
-__device__ __forceinline__ bool column_pair_second() { return (blockIdx.x >> 3) & 1; }
+__device__ __forceinline__ unsigned column_pair_id() { return blockIdx.y * gridDim.x + blockIdx.x; }
+__device__ __forceinline__ bool column_pair_second() { return (column_pair_id() >> 3) & 1; }
 __device__ __forceinline__ unsigned column_pair_block(bool band)
 {
-    const unsigned x = blockIdx.x & 7, k = blockIdx.x >> 4;
-    return band ? x * (gridDim.x >> 4) + k : k * 8 + x;
+    const unsigned x = column_pair_id() & 7, k = column_pair_id() >> 4;
+    return band ? x * ((gridDim.x * gridDim.y) >> 4) + k : k * 8 + x;
 }
 
 // Level waves of a kernel that can split a column's levels: four, unless the columns alone

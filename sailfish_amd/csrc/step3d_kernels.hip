@@ -1563,8 +1563,8 @@ extern "C" int sf_rhs3d_f32(sf_ctx *c, const double *fomn, const float *u, const
 template <class K, class... Args>
 static void launch_level_waves(K kernel, int LW, size_t lds, sf_ctx *c, void *stream, Args... args)
 {
-    hipLaunchKernelGGL(kernel, dim3(sf::column_grid(c->S2, kThreads / LW)), dim3(kThreads), lds, sf::as_stream(stream),
-                       args...);
+    hipLaunchKernelGGL(kernel, sf::wide_grid(sf::column_grid(c->S2, kThreads / LW), kThreads), dim3(kThreads), lds,
+                       sf::as_stream(stream), args...);
 }
 
 template <class T>
@@ -1680,7 +1680,7 @@ static int step3d_uv_launch(sf_ctx *c, const UVArgs<T> &a, double cff, double la
 {
     auto columns = [&](auto nmax, auto off) {
         hipLaunchKernelGGL((k_step3d_uv_col<T, decltype(nmax)::value, decltype(off)>),
-                           dim3(2 * sf::column_grid(c->S2, 64)), dim3(64), 0, sf::as_stream(stream),
+                           sf::wide_grid(2 * sf::column_grid(c->S2, 64), 64), dim3(64), 0, sf::as_stream(stream),
                            grid3(c, sizeof(T)), a, cff, lambda, Dt);
         return sf::check_launch("sf_step3d_uv");
     };
@@ -1754,8 +1754,9 @@ int step3d_uv_coupled_launch(sf_ctx *c, const sf_uv_coupled *p, double lambda, d
     const bool fits = (unsigned long long)(c->szK + 1) * (unsigned long long)c->S2 * sizeof(T) < (1ull << 32);
     if (fits && c->szK <= SF_STEP3D_REG_LEVELS)
         return by_levels(c->szK, [&](auto nmax) {
-            hipLaunchKernelGGL((k_step3d_uv_coupled_col<T, decltype(nmax)::value>), dim3(2 * sf::column_grid(c->S2, 64)),
-                               dim3(64), 0, sf::as_stream(stream), grid3(c, sizeof(T)), a, lambda, Dt);
+            hipLaunchKernelGGL((k_step3d_uv_coupled_col<T, decltype(nmax)::value>),
+                               sf::wide_grid(2 * sf::column_grid(c->S2, 64), 64), dim3(64), 0, sf::as_stream(stream),
+                               grid3(c, sizeof(T)), a, lambda, Dt);
             return sf::check_launch("sf_step3d_uv_coupled");
         });
     LAUNCH_COLUMNS(k_step3d_uv_coupled<T>, c, stream, grid3(c, sizeof(T)), a, lambda, Dt);

@@ -77,3 +77,50 @@ def test_step3d_uv_levels_past_4_gib(dt, szJ):
     del u, v, ub, vb, out
     torch.cuda.empty_cache()
     assert not any(x for _n, x in bad), bad
+
+
+def test_split_columns_past_2_30_points():
+    """set_maxflux, omega, pressure gradient and tracer step of more than 2^30 columns (four
+    threads to a column pass what one launch takes along x), FP32."""
+    import torch
+    from sailfish_amd.baroclinic import _bind
+    szJ, N = 16400, 4
+    print(f"[case] split columns of {SZI} x {szJ}", file=sys.stderr, flush=True)
+    _need(torch, 150)
+    lib, s, out = _bind(), _lib.stream_handle(), []
+    for sz in (12, szJ):
+        r = lambda lo, hi, seed, n=N, t=torch.float32: _rows(torch, sz, n, lo, hi, seed, t)
+        A, Hz, B, Cc, W = r(-1, 1, 1), r(9, 11, 2), r(-1, 1, 3, N + 1), r(-1, 1, 4, N + 1), r(0, 1, 5, N + 1)
+        for k in range(N + 1):
+            W[k] += 10.0 * k          # z_w of the pressure gradient; omega writes it afterwards
+        metric = r(0.9, 1.1, 7, 1, torch.float64)
+        BC = torch.full((sz, SZI), -1, dtype=torch.int32, device="cuda")
+        ctx = _ctx(torch, sz, N, metric)
+        p = lambda *t: [x.data_ptr() for x in t]
+        _lib.check(lib.sf_prsgrd(ctx, _lib.SF_FP32, *p(A, W, W, Hz), 9.8, 1025.0, *p(B, Cc), s), "sf_prsgrd")
+        first = [_rows_of(x) for x in (B, Cc)]
+        _lib.call("sf_set_maxflux_f32", ctx, *p(A, A, B, Cc, Hz), s)
+        second = [_rows_of(x) for x in (B, Cc)]
+        _lib.call("sf_omega_f32", ctx, *p(W, B, Cc, Hz, BC), s)
+        third = [_rows_of(W)]
+        new = torch.zeros_like(A[:1])
+        one = _ctx(torch, sz, 1, metric)
+        _lib.check(lib.sf_step3d_t(one, _lib.SF_FP32, *p(A, new, B, Cc, Hz[:1], Hz[1:]), 60.0, s), "sf_step3d_t")
+        torch.cuda.synchronize()
+        for c in (ctx, one):
+            lib.sf_ctx_destroy(c)
+        out.append(first + second + third + [_rows_of(new)])
+        del A, Hz, B, Cc, W, metric, BC, new
+        torch.cuda.empty_cache()
+    names = ("prsgrd ru", "prsgrd rv", "Huon", "Hvom", "W", "tracer")
+    bad = [(n, k) for n, a, b in zip(names, *out) for k in range(3) if not torch.equal(a[k], b[k])]
+    assert not bad, bad
+    assert all(o[3] for o in out[1]), [n for n, o in zip(names, out[1]) if not o[3]]
+
+
+def _rows_of(t):
+    """(first six rows, row six, last six rows, every row between equals row six)."""
+    n, szJ = t.shape[0], t.shape[1]
+    alike = all(bool((t[k, r:min(r + 2048, szJ - 6)] == t[k, 5]).all())
+                for k in range(n) for r in range(6, szJ - 6, 2048))
+    return t[:, :6].cpu(), t[:, 5].cpu(), t[:, -6:].cpu(), alike
