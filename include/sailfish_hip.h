@@ -315,6 +315,13 @@ int sf_phys_substep_fused(const sf_phys_fields *fields, int32_t precision, doubl
  * would give fewer than 1024 workgroups); tile_j = 0 chooses among more shapes. */
 int sf_phys_fused_default_tile(int32_t precision, int32_t szI, int32_t szJ);
 
+/* Shape (xi, eta) of the tile that tile_j = 0 takes in sf_phys_substep_fused (SF_TILE_PLAIN),
+ * sf_phys_substep_coupled_fused and sf_phys_substep_closure_fused. */
+#define SF_TILE_PLAIN 0
+#define SF_TILE_COUPLED 1
+#define SF_TILE_CLOSURE 2
+int sf_phys_fused_tile(int32_t precision, int32_t form, int32_t szI, int32_t szJ, int32_t *ti, int32_t *tj);
+
 /* ---------------- baroclinic terms: state equation, pressure gradient, tracers ------- */
 
 /* Linear equation of state (utility/test.in:2130-2160) on the szK levels of T and S:

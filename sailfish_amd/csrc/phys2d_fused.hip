@@ -14,6 +14,17 @@ extern "C" int sf_phys_fused_default_tile(int32_t precision, int32_t szI, int32_
     return tiles8 < 1024 ? 4 : 8;
 }
 
+extern "C" int sf_phys_fused_tile(int32_t precision, int32_t form, int32_t szI, int32_t szJ, int32_t *ti, int32_t *tj)
+{
+    SF_REQUIRE(ti && tj && szI >= 4 && szJ >= 4, "sf_phys_fused_tile: bad arguments");
+    SF_REQUIRE(precision == SF_FP64 || precision == SF_FP32, "sf_phys_fused_tile: unknown precision %d", precision);
+    SF_REQUIRE(form >= SF_TILE_PLAIN && form <= SF_TILE_CLOSURE, "sf_phys_fused_tile: unknown form %d", form);
+    const PhysTile t = phys_tile_of(precision == SF_FP64, form == SF_TILE_COUPLED, form == SF_TILE_CLOSURE, szI, szJ);
+    *ti = t.ti;
+    *tj = t.tj;
+    return SF_OK;
+}
+
 extern "C" int sf_phys_substep_fused(const sf_phys_fields *x, int32_t precision, double dt, int32_t first,
                                      double cff1, int32_t tile_j, void *stream)
 {

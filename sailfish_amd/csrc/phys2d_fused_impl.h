@@ -59,6 +59,11 @@ struct ClosureIn {
     const void *f;
 };
 
+// shape (xi, eta) of a tile
+struct PhysTile {
+    int ti, tj;
+};
+
 namespace {
 
 template <typename T>
@@ -1442,37 +1447,62 @@ int launch_fused(const sf_phys_fields *x, double dt, int first, double w1, void 
     return SF_ERR_ARG;
 }
 
-// Tile height tj: 4, 8 or 16 (64-wide tiles), or 0 for the tile that measured fastest on the
-// grid's size (microseconds per substep, graph replays, at the sizes named):
+// The tile of a substep that names none (microseconds per substep, graph replays):
 //  - grids of at most one 16 x 8 tile per CU: core and ring on different waves, all loads at
 //    the start of the tile (128 x 64: FP64 6.4 against 9.1 with 64 x 4 tiles, FP32 5.6 / 7.7);
-//  - up to two 32 x 8 tiles per CU: the same form with 32 x 8 tiles (512 x 256: FP64 11.6
-//    against 12.5, FP32 8.1 / 9.1; 640 x 320 has 800 such tiles and loses, 18.9 / 16.8 and
-//    12.4 / 10.4).  Coupled FP64 instances gain up to 1024 64 x 8 tiles (768 x 384: 26.1
-//    against 28.1; 1024 x 512: 39.6 / 36.4).  The closure needs the registers of a whole CU:
-//    one tile per CU (343 x 129: 11.0 / 12.6; 512 x 256: 18.4 / 14.5);
-//  - FP64 grids whose 64 x 4 tiles all fit at once (three per CU; 513 x 255: 14.3 against 16.5);
-//  - else 64 x 8 tiles; coupled FP32 64 x 4 below four 64 x 8 tiles per CU (768 x 384: 15.5
-//    against 16.8), the closure 64 x 4 (its 64 x 8 instances exceed two waves per SIMD).
+//  - the same form with 32 x 8 tiles while all of them are resident (by their registers two a
+//    CU, FP32 without coupling three) and their number divides by eight, so that they go to
+//    the XCDs in bands (xcd_band): FP64 512 x 256 (512 tiles) 11.5 against 11.8 with 64 x 8,
+//    but 544 x 256 (544, a second round) 15.3 against 14.3 with 64 x 4; FP32 768 x 256 (768)
+//    9.7 against 10.4, 640 x 320 (800) 12.3 against 10.4; coupled FP32 512 x 256 8.9 against
+//    10.4 with 64 x 4, 544 x 256 12.5 against 11.1;
+//  - without bands they lose earlier: FP64 keeps them up to one a CU (352 x 184, 253 tiles,
+//    8.9 against 10.9; 480 x 168, 315, 11.2 against 10.7), FP32 up to two where the tiles they
+//    replace have no bands either (544 x 240, 510 tiles, 8.9 against 10.3 with 270 64 x 8;
+//    475 x 245, 465, 10.7 against 9.0 with 248; 672 x 248, 651, 12.2 against 11.4; coupled
+//    663 x 166, 441, 11.0 against 11.9 with 462 64 x 4; 475 x 245 11.2 against 10.5 with 496);
+//  - coupled FP64 gains from them up to 1024 64 x 8 tiles (768 x 384: 25.0 against 28.1), but
+//    without bands not past two a CU while 64 x 8 tiles are all resident, two a CU
+//    (640 x 184, 460 tiles, 15.1 either way; 640 x 296, 740, 20.9 against 19.2 with 370;
+//    832 x 344, 1118, 28.4 against 29.7 with 559).  The closure needs the registers of a whole
+//    CU: one tile per CU (343 x 129: 11.0 / 12.6; 512 x 256: 18.4 / 14.5);
+//  - else 64 x 8 tiles, or 64 x 4 where one of those a CU leaves none idle and one of these
+//    more than fills it: FP64 with more than one 64 x 8 tile per CU and at most three 64 x 4
+//    (513 x 255: 14.3 against 16.3; 640 x 272: 14.8 / 16.8; 480 x 248, one per CU: 12.6 / 11.3);
+//    coupled FP32 below four 64 x 8 tiles per CU (768 x 384: 15.5 against 16.8); the closure
+//    (its 64 x 8 instances exceed two waves per SIMD).
+inline PhysTile phys_tile_of(bool f64, bool coupled, bool closure, int szI, int szJ)
+{
+    constexpr long long CU = 256;
+    auto tiles = [&](int TI, int TJ) {
+        const int oi = szI % TI == 1 ? 1 : 0, oj = szJ % TJ == 1 ? 1 : 0;
+        return (long long)((szI + oi + TI - 1) / TI) * ((szJ + oj + TJ - 1) / TJ);
+    };
+    const bool few8 = tiles(64, 8) < 4 * CU;
+    const long long t32 = tiles(32, 8);
+    const bool banded = t32 % 8 == 0;
+    if (closure) return t32 <= CU ? PhysTile{32, 8} : PhysTile{64, 4};
+    if (tiles(16, 8) <= CU) return PhysTile{16, 8};
+    const long long alt = tiles(64, coupled ? 4 : 8);   // of FP32, where 32 x 8 are not taken
+    bool small;
+    if (coupled && f64) small = few8 && (banded || t32 <= 2 * CU || tiles(64, 8) > 2 * CU);
+    else if (banded) small = t32 <= (f64 || coupled ? 2 : 3) * CU;
+    else small = t32 <= CU || (!f64 && t32 <= 2 * CU && alt % 8 != 0);
+    if (small) return PhysTile{32, 8};
+    if (coupled) return PhysTile{64, !f64 && few8 ? 4 : 8};
+    return PhysTile{64, f64 && tiles(64, 8) > CU && tiles(64, 4) <= 3 * CU ? 4 : 8};
+}
+
+// Tile height tj: 4, 8 or 16 (64-wide tiles), or 0 for phys_tile_of's choice.
 template <typename T>
 int dispatch_tj(const sf_phys_fields *x, double dt, int first, double w1, int tj, void *stream,
                 const sf_couple_fields *cp = nullptr, const ClosureIn *cl = nullptr)
 {
-    constexpr long long CU = 256;
-    constexpr bool F64 = sizeof(T) == 8;
     if (tj == 0) {
-        auto tiles = [&](int TI, int TJ) {
-            const int oi = x->szI % TI == 1 ? 1 : 0, oj = x->szJ % TJ == 1 ? 1 : 0;
-            return (long long)((x->szI + oi + TI - 1) / TI) * ((x->szJ + oj + TJ - 1) / TJ);
-        };
-        const bool few8 = tiles(64, 8) < 4 * CU;
-        const long long t32 = tiles(32, 8);
-        if (!cl && tiles(16, 8) <= CU) return launch_fused<T, 16, 8, 128, 192>(x, dt, first, w1, stream, cp);
-        if (cl ? t32 <= CU : (cp && F64 ? few8 : t32 <= 2 * CU + 64))
-            return launch_fused<T, 32, 8, 256, 256>(x, dt, first, w1, stream, cp, cl);
-        if (cl) tj = 4;
-        else if (cp) tj = few8 ? 4 : 8;
-        else tj = F64 && tiles(64, 4) <= 3 * CU ? 4 : 8;
+        const PhysTile t = phys_tile_of(sizeof(T) == 8, cp, cl, x->szI, x->szJ);
+        if (t.ti == 16) return launch_fused<T, 16, 8, 128, 192>(x, dt, first, w1, stream, cp);
+        if (t.ti == 32) return launch_fused<T, 32, 8, 256, 256>(x, dt, first, w1, stream, cp, cl);
+        tj = t.tj;
     }
     switch (tj) {
     case 4: return launch_fused<T, 64, 4, 256>(x, dt, first, w1, stream, cp, cl);

@@ -56,6 +56,8 @@ def _bind():
     lib.sf_phys_run.restype = C.c_int32
     lib.sf_phys_fused_default_tile.argtypes = [C.c_int32, C.c_int32, C.c_int32]
     lib.sf_phys_fused_default_tile.restype = C.c_int32
+    lib.sf_phys_fused_tile.argtypes = [C.c_int32] * 4 + [C.POINTER(C.c_int32)] * 2
+    lib.sf_phys_fused_tile.restype = C.c_int32
     return lib
 
 
