@@ -89,47 +89,6 @@ struct PFA {
     float cl_ynorm[4];
 };
 
-// Visit the points of region [3-LO, 3+TI+HI) x [3-LO, 3+TJ+HI) of the frame: the
-// TI*TJ core points first (slot k >= 0, point tid + k*NT in row-major core order),
-// then the ring around the core (slot -1).
-template <int TI, int TJ, int NT, int LO, int HI, typename F>
-__device__ __forceinline__ void for_region(int tid, F &&fn)
-{
-    constexpr int CORE = TI * TJ;
-    static_assert(CORE % NT == 0, "core must be a multiple of the block");
-#pragma unroll
-    for (int k = 0; k < CORE / NT; k++) {
-        const int idx = tid + k * NT;
-        fn(k, 3 + idx % TI, 3 + idx / TI);
-    }
-    constexpr int W = TI + LO + HI, H = TJ + LO + HI;
-    constexpr int RING = W * H - CORE;
-    if constexpr (RING > 0) {
-        constexpr int NBOT = LO * W, WROW = LO + HI, NMID = TJ * WROW;
-#pragma unroll
-        for (int k = 0; k < (RING + NT - 1) / NT; k++) {
-            const int t = tid + k * NT;
-            if (t < RING) {
-                int a, b;
-                if (t < NBOT) {
-                    b = 3 - LO + t / W;
-                    a = 3 - LO + t % W;
-                } else if (t < NBOT + NMID) {
-                    const int s = t - NBOT;
-                    b = 3 + s / WROW;
-                    const int c = s % WROW;
-                    a = c < LO ? 3 - LO + c : 3 + TI + (c - LO);
-                } else {
-                    const int s = t - NBOT - NMID;
-                    b = 3 + TJ + s / W;
-                    a = 3 - LO + s % W;
-                }
-                fn(-1, a, b);
-            }
-        }
-    }
-}
-
 // FP64 closure instances of 64-wide tiles keep the network's feature tiles in frame planes
 // 1..5, written only from stage A on, and one more (a barrier ends the closure phase): 27 KB
 // less LDS, so two 64 x 4 workgroups fit a CU.  Smaller planes cannot hold the tiles; they
