@@ -104,6 +104,18 @@ def measured_traffic(dtype_name):
         return None
 
 
+def phys_tile(precision, szI, szJ, tile_j=0):
+    """[xi, eta] of the tile that sf_phys_substep_fused takes (tile_j = 0: its own choice)."""
+    import ctypes as C
+    from sailfish_amd import _lib
+    from sailfish_amd.phys2d import _bind
+    if tile_j:
+        return [64, tile_j]
+    a, b = C.c_int32(), C.c_int32()
+    _lib.check(_bind().sf_phys_fused_tile(precision, 0, szI, szJ, C.byref(a), C.byref(b)), "sf_phys_fused_tile")
+    return [a.value, b.value]
+
+
 def run_phys_gpu(args, dtype_name, steps, warmup):
     import torch
     from sailfish_amd import configs
@@ -114,7 +126,8 @@ def run_phys_gpu(args, dtype_name, steps, warmup):
     cfg = configs.basin2(args.szI, args.szJ, dx=args.dx)
     ct, GRID, OCEAN, _B = build_model(cfg, dtype=dtype, ndtfast=30)
     st = PhysStepper(GRID, OCEAN, rdrg=cfg["rdrg"], fused=True, tile_j=args.tile_j)
-    tile_j = args.tile_j or st.lib.sf_phys_fused_default_tile(st.precision, GRID.szI, GRID.szJ)
+    tile_j = args.tile_j
+    tile = phys_tile(st.precision, GRID.szI, GRID.szJ, tile_j)
     S2 = GRID.szI * GRID.szJ
     n = [0]
 
@@ -174,7 +187,7 @@ def run_phys_gpu(args, dtype_name, steps, warmup):
                     bpp_read=PHYS_BULK * bulk + PHYS_F64 * 8,
                     achieved=bpp * S2 / (kern_ms * 1e-3) / 1e9, finite=finite,
                     zmax=float(OCEAN.zeta_t2.abs().max()), nk=nk, kernel="k_phys_fused",
-                    entry="sf_phys_substep_fused", tile=[64, tile_j], substeps=n[0] + nk)
+                    entry="sf_phys_substep_fused", tile=tile, substeps=n[0] + nk)
 
     # the timed region: K substeps captured in HIP graphs, each node with its own
     # arguments (slot rotation and averaging weight of that substep).  Three graphs,
@@ -244,7 +257,7 @@ def run_phys_gpu(args, dtype_name, steps, warmup):
     return dict(cfg=cfg, S2=S2, ms_per_step=ms_per_step, ms_per_step_launched=ms_per_step_launched, wall=wall,
                 kern_ms=kern_ms, bpp=bpp_contract, bpp_read=bpp,
                 achieved=achieved, finite=finite, zmax=zmax, nk=nk, kernel="k_phys_fused",
-                entry="sf_phys_substep_fused", tile=[64, tile_j], substeps=n[0],
+                entry="sf_phys_substep_fused", tile=tile, substeps=n[0],
                 replays_ms=rep_ms, warm_replays=nwarm)
 
 
@@ -261,7 +274,6 @@ def run_large_grid_gpu(args):
     cfg = configs.basin2_analytic(n, n, dx=args.dx)
     ct, GRID, OCEAN, _B = build_model(cfg, dtype=torch.float32, ndtfast=30)
     st = PhysStepper(GRID, OCEAN, rdrg=cfg["rdrg"], fused=True)
-    tile_j = st.lib.sf_phys_fused_default_tile(st.precision, GRID.szI, GRID.szJ)
     for k in range(3):
         ct.next2DTimeStep()
         OCEAN.cycleTimes2D()
@@ -277,7 +289,7 @@ def run_large_grid_gpu(args):
     a.record()
     for k in range(nk):
         ct.next2DTimeStep()
-        rc |= fn(C.byref(blocks[k % 3]), st.precision, float(ct.dtfast), 0, ct.cff1(), tile_j, sh)
+        rc |= fn(C.byref(blocks[k % 3]), st.precision, float(ct.dtfast), 0, ct.cff1(), 0, sh)
     b.record()
     torch.cuda.synchronize()
     _lib.check(rc, "sf_phys_substep_fused")
