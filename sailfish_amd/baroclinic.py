@@ -89,6 +89,14 @@ class Tracers:
     def step(self, GRID, OCEAN, dt: float, stream=None):
         """Advect T and S by the step's mass fluxes from Hz_old to the current Hz."""
         c = ops.ctx_of(GRID)
+        if self.T_new.data_ptr() == self.S_new.data_ptr():     # one buffer for both new tracers
+            for old, new in ((self.T, self.T_new), (self.S, self.S_new)):
+                _lib.check(self.lib.sf_step3d_t(c.handle, self.precision, old.data_ptr(), new.data_ptr(),
+                                                OCEAN.Huon.data_ptr(), OCEAN.Hvom.data_ptr(), self.Hz_old.data_ptr(),
+                                                GRID.Hz.data_ptr(), float(dt), _lib.stream_handle(stream)),
+                           "sf_step3d_t")
+                old.copy_(new)
+            return
         _lib.check(self.lib.sf_step3d_ts(c.handle, self.precision, self.T.data_ptr(), self.T_new.data_ptr(),
                                          self.S.data_ptr(), self.S_new.data_ptr(), OCEAN.Huon.data_ptr(),
                                          OCEAN.Hvom.data_ptr(), self.Hz_old.data_ptr(), GRID.Hz.data_ptr(),
