@@ -306,8 +306,9 @@ int sf_phys_substep(const sf_phys_fields *fields, int32_t precision, double dt, 
  * on an LDS-staged tile of 64 x tile_j points (tile_j = 4, 8 or 16; 0 = the tile that
  * measured fastest on the grid's size, down to 16 x 8 on small grids)
  * with a 3/2-point halo, so no intermediate state goes to memory.  scratch[] is
- * not used.  Results equal sf_phys_substep bit for bit in both precisions.  Same
- * reference lineage as sf_phys_substep. */
+ * not used.  FP64 results equal sf_phys_substep bit for bit; FP32 agrees to rounding
+ * (contraction on) and is the same for every tile.  Same reference lineage as
+ * sf_phys_substep. */
 int sf_phys_substep_fused(const sf_phys_fields *fields, int32_t precision, double dt, int32_t first,
                           double cff1, int32_t tile_j, void *stream);
 

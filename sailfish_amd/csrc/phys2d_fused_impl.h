@@ -13,7 +13,7 @@
 //   stage  region (frame coords, core = [3, 3+T))   writes (LDS plane)
 //   L      [0, T+5)    z1                               Z1
 //   A      [1, T+5)    DU1 = D*u*on_u, DV1 = D*v*om_v   DU, DV
-//   P1     [1, T+4)    predicted zeta zs, its RHS rz    ZS, RZ
+//   P1     [1, T+4)    predicted zeta zs, its RHS rz    ZS
 //   P2     [2, T+4)    predicted ubar us, vbar vs       US, VS
 //   C0     [2, T+4)    DUs, DVs of the predicted state  DU, DV (reused)
 //   C1     [2, T+3)    corrected zeta z2 (+ averages)   Z1 (reused as Z2)
@@ -1432,7 +1432,7 @@ int launch_fused(const sf_phys_fields *x, double dt, int first, double w1, void 
 //    (its 64 x 8 instances exceed two waves per SIMD).
 inline PhysTile phys_tile_of(bool f64, bool coupled, bool closure, int szI, int szJ)
 {
-    constexpr long long CU = 256;
+    constexpr long long CU = sf::kCUs;
     auto tiles = [&](int TI, int TJ) {
         const int oi = szI % TI == 1 ? 1 : 0, oj = szJ % TJ == 1 ? 1 : 0;
         return (long long)((szI + oi + TI - 1) / TI) * ((szJ + oj + TJ - 1) / TJ);

@@ -62,14 +62,16 @@ constexpr int kBlock1D = 256;
 // (FP64 reference discretisation) and 432 MiB (FP64 physics).
 constexpr double kStreamingBytes = 320.0 * (1 << 20);
 
-// compute units of a device, queried once per device (256 on MI355X)
+// compute units of an MI355X, where a rule of sizes was measured on the whole card
+constexpr int kCUs = 256;
+// compute units of a device, queried once per device
 inline int cu_count(int device)
 {
     static int cache[64];
-    if (device < 0 || device >= 64) return 256;
+    if (device < 0 || device >= 64) return kCUs;
     if (cache[device] == 0) {
         int v = 0;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || v <= 0) v = 256;
+        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || v <= 0) v = kCUs;
         cache[device] = v;
     }
     return cache[device];
@@ -114,7 +116,7 @@ __device__ __forceinline__ unsigned column_pair_block(bool band)
 }
 
 // Level waves of a kernel that can split a column's levels: four, unless the columns alone
-// give every SIMD (256 CUs of four) four waves and the column is short (at most `few` levels).
+// give every SIMD (four a CU) four waves and the column is short (at most `few` levels).
 // A split column repeats what belongs to the column (index division, metrics, the sums below
 // a wave's levels), which a few levels do not pay for: one / four waves at 4 levels, FP64
 // 3000 x 1500 set_maxflux 142 / 148 us, omega 104 / 139, pressure gradient 337 / 467, FP32
@@ -123,7 +125,7 @@ __device__ __forceinline__ unsigned column_pair_block(bool band)
 // pressure gradient 16 levels 149 / 160 (FP32 72 / 79), 24 levels 232 / 231.
 inline int level_waves(const sf_ctx *c, size_t few)
 {
-    return c->S2 >= 4LL * 1024 * 64 && (size_t)c->szK <= few ? 1 : 4;
+    return c->S2 >= 4LL * 4 * kCUs * 64 && (size_t)c->szK <= few ? 1 : 4;
 }
 
 }  // namespace sf

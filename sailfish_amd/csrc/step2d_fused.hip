@@ -59,7 +59,6 @@ constexpr int W2 = TI + 4;           // R2 frame width
 constexpr int H2 = TJ + 4;
 constexpr int N2 = W2 * H2;
 constexpr int NCORE = TI * TJ;
-constexpr int kCUs = 256;
 
 // dense boundary-code values
 constexpr int kKeep = -1;
@@ -544,7 +543,7 @@ int launch(sf_ctx *c, const sf_step2d_fields *a, double dtfast, double cff1, dou
         // four (FP32) workgroups share a CU.  Per substep, 832 / 512 threads: FP64
         // 388 x 260 (231 tiles) 7.9 / 9.1 us, 513 x 255 (288) 11.9 / 10.6, 1023 x 511
         // (1024) 25.0 / 23.7; FP32 6.4 / 8.2, 9.3 / 8.4, 18.7 / 17.1
-        if (P.tiles_i * P.tiles_j <= kCUs) shape(std::integral_constant<int, 832>{});
+        if (P.tiles_i * P.tiles_j <= sf::kCUs) shape(std::integral_constant<int, 832>{});
         else shape(std::integral_constant<int, 512>{});
         int rc = sf::check_launch("sf_step2d_substep (tiles)");
         if (rc != SF_OK) return rc;

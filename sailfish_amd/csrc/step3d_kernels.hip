@@ -860,7 +860,11 @@ __global__ __launch_bounds__(256) void k_step3d_uv(G3 g, UVArgs<T> a, double cff
 // correct_mean's shift applied, and the depth sums run in the reference's level order.  At
 // u-but-not-v points the u wave solves its eliminated system a second time for v, as
 // solve_tri does on the shared scratch.  Each thread reads tmpU (tmpV) only before it writes
-// u (v), and no other thread's column of them, so they may alias u / v.  The depth sums
+// u (v), and no other thread's column of them, so they may alias u / v.  Bands of columns at
+// every size: a wave's level chain leaves HBM time to spare, so eight far-apart streams cost
+// nothing and the west and south neighbours' thickness and depth come from L2 (always / up to
+// kBandBytes: FP64 1024 x 512 x 32 344 / 406 us, 1500 x 800 x 32 751 / 751, 3000 x 1500 x 10
+// 861 / 887; FP32 456 / 520 there, 1500 x 800 x 32 390 / 401).  The depth sums
 // fetch four levels at a time: FP64 1024 x 512 x 32 397 -> 361 us, 386 x 258 x 40 92 -> 81;
 // FP32 202 -> 181.
 //
@@ -892,11 +896,13 @@ __device__ __forceinline__ bool has_level(int K, int N)
     return K < N;
 }
 
-// first element of level K, or of the last one past it, as a scalar of its own
-__device__ __forceinline__ long long level_start(int K, int N, long long S2)
+// start of level K, or of the last one past it, in steps of a level (elements or bytes), as a
+// scalar of its own
+template <class O>
+__device__ __forceinline__ O level_start(int K, int N, O step)
 {
     asm volatile("" : "+s"(N));
-    return (K < N ? K : N - 1) * S2;
+    return (O)(K < N ? K : N - 1) * step;
 }
 
 template <class T, int NMAX, class O>
@@ -1240,28 +1246,11 @@ __global__ __launch_bounds__(256) void k_step3d_uv_coupled(G3 g, UVC<T> a, doubl
 // so that the compiler does not fold the unrolled levels into per-level 64-bit scalar
 // bases (dozens of arrays x levels, which it spilled to VGPR lanes and restored at every
 // use).
-template <class T>
-__device__ __forceinline__ T ldb(const T *p, uint32_t o)
-{
-    return *(const __attribute__((address_space(1))) T *)((const __attribute__((address_space(1))) char *)p + o);
-}
-template <class T>
-__device__ __forceinline__ void stb(T *p, uint32_t o, T v)
-{
-    *(__attribute__((address_space(1))) T *)((__attribute__((address_space(1))) char *)p + o) = v;
-}
 __device__ __forceinline__ uint32_t next_level(uint32_t o, uint32_t stride)
 {
     o += stride;
     asm("" : "+v"(o));
     return o;
-}
-
-// byte offset of level K, or of the last one past it, as a scalar of its own
-__device__ __forceinline__ uint32_t level_offset(int K, int N, uint32_t stride)
-{
-    asm volatile("" : "+s"(N));
-    return (uint32_t)(K < N ? K : N - 1) * stride;
 }
 
 template <class T, int NMAX>
@@ -1294,24 +1283,24 @@ __global__ __launch_bounds__(64) void k_step3d_uv_coupled_col(G3 g, UVC<T> a, do
         // operands of the level at byte offset ob (z_r and Akv of the level above)
         auto load = [&](uint32_t ob, bool top) {
             Lv q{};
-            q.hn0 = ldb(a.Hz, ob);
-            q.hn1 = ldb(a.Hz, ob - dB);
-            q.ho0 = ldb(a.Hz_old, ob);
-            q.ho1 = ldb(a.Hz_old, ob - dB);
-            q.xo = ldb((const T *)x, ob);
-            q.rk = ldb(r, ob);
-            if (ab > 0) q.rk1 = ldb(r1, ob);
-            if (ab > 1) q.rk2 = ldb(r2, ob);
+            q.hn0 = ldc(a.Hz, ob);
+            q.hn1 = ldc(a.Hz, ob - dB);
+            q.ho0 = ldc(a.Hz_old, ob);
+            q.ho1 = ldc(a.Hz_old, ob - dB);
+            q.xo = ldc((const T *)x, ob);
+            q.rk = ldc(r, ob);
+            if (ab > 0) q.rk1 = ldc(r1, ob);
+            if (ab > 1) q.rk2 = ldc(r2, ob);
             if (!top) {
-                q.z0 = ldb(a.z_r, ob + SB);
-                q.z1 = ldb(a.z_r, ob + SB - dB);
-                q.k0 = ldb(a.Akv, ob + SB);
-                q.k1 = ldb(a.Akv, ob + SB - dB);
+                q.z0 = ldc(a.z_r, ob + SB);
+                q.z1 = ldc(a.z_r, ob + SB - dB);
+                q.k0 = ldc(a.Akv, ob + SB);
+                q.k1 = ldc(a.Akv, ob + SB - dB);
             }
             return q;
         };
-        T zf0 = ldb(a.z_r, o0), zd0 = ldb(a.z_r, o0 - dB);
-        const T xbot = ldb((const T *)x, o0);
+        T zf0 = ldc(a.z_r, o0), zd0 = ldc(a.z_r, o0 - dB);
+        const T xbot = ldc((const T *)x, o0);
         T sdp = T(0);   // sub-diagonal of the level below
         uint32_t ob = o0;
         Lv cur = load(ob, N - 1 == 0);
@@ -1333,7 +1322,7 @@ __global__ __launch_bounds__(64) void k_step3d_uv_coupled_col(G3 g, UVC<T> a, do
                 if (ab == 0) rab = cur.rk;
                 else if (ab == 1) rab = T(1.5) * cur.rk - T(0.5) * cur.rk1;
                 else rab = (T(23.0 / 12.0) * cur.rk - T(16.0 / 12.0) * cur.rk1) + T(5.0 / 12.0) * cur.rk2;
-                stb(keep, ob, cur.rk);
+                stc(keep, ob, cur.rk);
                 T rhs = ((cur.ho0 + cur.ho1) * T(0.5)) * cur.xo + cdt_mn * rab;
                 const T hn = (cur.hn0 + cur.hn1) * T(0.5);
                 if (K == 0) {
@@ -1368,9 +1357,9 @@ __global__ __launch_bounds__(64) void k_step3d_uv_coupled_col(G3 g, UVC<T> a, do
                 T h0[4], h1[4];
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
-                    const uint32_t o = o0 + level_offset(K + q, N, SB);
-                    h0[q] = ldb(a.Hz, o);
-                    h1[q] = ldb(a.Hz, o - dB);
+                    const uint32_t o = o0 + level_start(K + q, N, SB);
+                    h0[q] = ldc(a.Hz, o);
+                    h1[q] = ldc(a.Hz, o - dB);
                 }
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
@@ -1395,12 +1384,12 @@ __global__ __launch_bounds__(64) void k_step3d_uv_coupled_col(G3 g, UVC<T> a, do
             if (has_level(K, N)) {
                 T hf0[4];
 #pragma unroll
-                for (int q = 0; q < 4; q++) hf0[q] = ldb((const T *)Hf, o0 + level_offset(K + q, N, SB));
+                for (int q = 0; q < 4; q++) hf0[q] = ldc((const T *)Hf, o0 + level_start(K + q, N, SB));
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     if (!has_level(K + q, N)) continue;
                     const T xk = T((double)R[K + q] - CF);
-                    stb(x, o0 + level_offset(K + q, N, SB), xk);
+                    stc(x, o0 + level_start(K + q, N, SB), xk);
                     const T hf = T(0.5 * ((double)hf0[q] + (double)xk * (met * (double)D[K + q])));
                     R[K + q] = hf;
                     FC = FC + (double)hf;
@@ -1412,7 +1401,7 @@ __global__ __launch_bounds__(64) void k_step3d_uv_coupled_col(G3 g, UVC<T> a, do
 #pragma unroll
         for (int K = 0; K < NMAX; K++) {
             if (has_level(K, N)) {
-                stb(Hf, ob, T((double)R[K] - (met * (double)D[K]) * FC));
+                stc(Hf, ob, T((double)R[K] - (met * (double)D[K]) * FC));
                 ob = next_level(ob, SB);
             }
         }
