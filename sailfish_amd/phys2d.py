@@ -167,22 +167,33 @@ def issue_substeps(compTimes, OCEAN, nsub: int, what: str, issue, clamp=None):
         return
     w = (C.c_double * max(nsub, 1))()
     cl = (C.c_double * max(nsub, 1))() if clamp is not None else None
-    times = []
+    before = compTimes.iif, compTimes.time2D
     for n in range(nsub):
         compTimes.next2DTimeStep()
         w[n] = compTimes.cff1()
         if cl is not None:
             cl[n] = clamp(compTimes.time2D)
-        times.append({k: getattr(compTimes, k) for k in ("iif", "time2D") if hasattr(compTimes, k)})
     done = C.c_int32(0)
     rc = issue(nsub, w, cl, done)
     n = nsub if rc == _lib.SF_OK else min(done.value + 1, nsub)
-    if 0 < n < nsub:
-        for k, v in times[n - 1].items():
-            setattr(compTimes, k, v)
+    if n < nsub:
+        compTimes.iif, compTimes.time2D = before
+        for _ in range(n):
+            compTimes.next2DTimeStep()
     for _ in range(n % 3):
         OCEAN.cycleTimes2D()
     _lib.check(rc, what)
+
+
+# substeps of one native call of a run: it holds their weights and keeps signals waiting.  A
+# multiple of three, so that the slots are back where they were and the next call takes the
+# same fields
+RUN_CHUNK = 3 * 1024
+
+
+def chunks(nsub: int):
+    """(first substep, count) of the native calls of ``nsub`` substeps."""
+    return [(n, min(RUN_CHUNK, nsub - n)) for n in range(0, nsub, RUN_CHUNK)]
 
 
 def run_phys(compTimes, GRID, OCEAN, nsteps: int, stepper: PhysStepper | None = None, start_first: bool = True):
@@ -192,9 +203,11 @@ def run_phys(compTimes, GRID, OCEAN, nsteps: int, stepper: PhysStepper | None = 
     if own(st, STEPPER) and own(OCEAN, STATE) and own(compTimes, COUNTER):
         a = st.fields(OCEAN)
         ob = (C.addressof(st.open_bc), st.vc_work.data_ptr(), st.vc_out.data_ptr()) if st.open_edges else (None,) * 3
-        issue_substeps(compTimes, OCEAN, int(nsteps), "sf_phys_run", lambda n, w1, _clamp, done: st.lib.sf_phys_run(
-            C.byref(a), None, None, None, *ob, st.precision, float(compTimes.dtfast), int(bool(start_first)), w1, n,
-            int(st.fused), st.tile_j, _lib.stream_handle(), C.byref(done)))
+        for n0, count in chunks(int(nsteps)):
+            first = int(bool(start_first) and n0 == 0)
+            issue_substeps(compTimes, OCEAN, count, "sf_phys_run", lambda n, w1, _clamp, done: st.lib.sf_phys_run(
+                C.byref(a), None, None, None, *ob, st.precision, float(compTimes.dtfast), first, w1, n,
+                int(st.fused), st.tile_j, _lib.stream_handle(), C.byref(done)))
         return st
     for n in range(int(nsteps)):     # a caller's own step, state or counter
         compTimes.next2DTimeStep()

@@ -19,7 +19,7 @@ import torch
 from . import _lib
 from . import mod_operators as ops
 from .mod_boundary import clamped_value
-from .phys2d import COUNTER, STATE, issue_substeps, methods, own
+from .phys2d import COUNTER, STATE, chunks, issue_substeps, methods, own
 
 _I32P = C.POINTER(C.c_int32)
 SF_SUBSTEP_ZERO_VBAR = 1
@@ -124,13 +124,14 @@ class FusedStepper:
         _lib.check(rc, "sf_step2d_substep")
 
     def run(self, compTimes, OCEAN, nsub: int, zero_vbar: bool = False):
-        """``nsub`` substeps (next2DTimeStep, cycleTimes2D, step) through one native call
-        (see ``issue_substeps``)."""
+        """``nsub`` substeps (next2DTimeStep, cycleTimes2D, step) through native calls (see
+        ``issue_substeps``)."""
         a = self.fields(OCEAN)
         flags = SF_SUBSTEP_ZERO_VBAR if zero_vbar else 0
-        issue_substeps(compTimes, OCEAN, nsub, "sf_step2d_run", lambda n, w1, cl, done: self.lib.sf_step2d_run(
-            self.ctx.handle, C.byref(a), self.precision, float(compTimes.dtfast), w1, cl, flags, n,
-            _lib.stream_handle(), C.byref(done)), clamp=clamped_value)
+        for _n0, count in chunks(nsub):
+            issue_substeps(compTimes, OCEAN, count, "sf_step2d_run", lambda n, w1, cl, done: self.lib.sf_step2d_run(
+                self.ctx.handle, C.byref(a), self.precision, float(compTimes.dtfast), w1, cl, flags, n,
+                _lib.stream_handle(), C.byref(done)), clamp=clamped_value)
 
     def _cached_fields(self, OCEAN):
         key = (id(OCEAN), OCEAN.zeta_t0.data_ptr(), OCEAN.ubar_t0.data_ptr(), OCEAN.rubar_t0.data_ptr())

@@ -217,3 +217,44 @@ def test_negative_counts_do_nothing(log, nsub):
     phys2d.issue_substeps(ct, oc, nsub, "x", lambda *a: _lib.SF_ERR_ARG)
     assert (ct.iif, ct.time2D) == (0, 0.0) and not log
     assert [oc.slot_of("zeta", f"t{k}") for k in range(3)] == slots
+
+
+class RunLib(Lib):
+    """The native run: records (first, count) of each call."""
+
+    def __getattr__(self, name):
+        def call(*args):
+            if name == "sf_phys_run":
+                self.log.append((args[9], args[11]))
+                args[-1]._obj.value = args[11]
+            else:
+                self.log.append((None, args[7]))
+                args[-1]._obj.value = args[7]
+            return _lib.SF_OK
+        return call
+
+
+@pytest.mark.parametrize("nsub", [3071, 3072, 3073, 20000])
+def test_long_runs_go_in_bounded_calls(log, nsub):
+    """A native call keeps signals waiting and holds its weights: a long run takes several, and
+    its memory does not grow with it."""
+    import tracemalloc
+    for run in ("phys", "step2d"):
+        log.clear()
+        ct, oc = _counter(log), _state(log)
+        slot = oc.slot_of("zeta", "t2")
+        st, fs = _stepper(log), _fused(log)
+        st.lib, fs.lib = RunLib(log), RunLib(log)
+        grid = types.SimpleNamespace(**vars(GRID), _sf_fused=fs)
+        tracemalloc.start()
+        if run == "phys":
+            run_phys(ct, GRID, oc, nsub, st)
+        else:
+            main2d(ct, grid, oc, None, nsub, fused=True)
+        peak = tracemalloc.get_traced_memory()[1]
+        tracemalloc.stop()
+        counts = [c for _f, c in log]
+        assert sum(counts) == nsub and max(counts) <= 3072 and all(c % 3 == 0 for c in counts[:-1])
+        assert run == "step2d" or [f for f, _c in log] == [1] + [0] * (len(log) - 1)
+        assert ct.iif == nsub and oc.slot_of("zeta", "t2") == (slot + nsub) % 3
+        assert peak < 300_000, peak
