@@ -394,8 +394,9 @@ void k_rhs3d_fused(G3 g, HG<T> h, A fomn, AG<T> Hz, AG<T> Wa, const int32_t *BC,
     // workgroups per CU instead of two.  A thread's x-face at its own column, not the one
     // before, lets its four fluxes share the curvature terms (27 LDS reads for 47): FP32
     // 1024 x 512 x 32 242 us -> 229, 386 x 258 x 40 72 -> 68; FP64 435 -> 430, 107 -> 103.
-    // What is left is traffic (1.5 times the fields, from the halos) beside 280 FP64
-    // instructions a level and wave.
+    // What bounds it: FP64 moves 2.04 GB at 1024 x 512 x 32 (its fields are 1.07; other tiles'
+    // XCDs read the halos again) in 409 us, the copy's rate; FP32 0.81 GB (0.54) in 215-225 us,
+    // with 326 vector instructions a level and wave.
     constexpr bool SB = sizeof(T) == 8;   // single tile buffer
     __shared__ T sl[SB ? 1 : 2][4][LN];
     __shared__ T fxu[TJ][HTI + 1], fxv[TJ][HTI + 1], feu[TJ + 1][HTI], fev[TJ + 1][HTI];
@@ -561,9 +562,10 @@ void k_rhs3d_fused(G3 g, HG<T> h, A fomn, AG<T> Hz, AG<T> Wa, const int32_t *BC,
 // ---- set_maxflux (step3D_uv.kernels.cpp:372-405) ----------------------------------
 // the fluxes are stored with streaming (non-temporal) stores: no thread of the launch
 // reads them back.  Both fluxes of a level are formed together, so Hz is read once.
-// HBM-bound.  Against a thread that took its column's levels one by one: FP64 700 x 400 x 32
-// 59 -> 47 us, 386 x 258 x 40 34 -> 24, 1024 x 512 x 32 (five fields, 671 MB) 136 -> 134; FP32
-// 53 -> 44 there; few levels on a large grid (one level wave) FP64 1500 x 800 x 5 41 -> 34.
+// HBM-bound: FP64 1024 x 512 x 32 moves 0.71 GB (five fields, 0.67) in 149 us of a pass.  Launched
+// over and over, inputs partly in the last-level cache, against a thread that took its column's
+// levels one by one: 136 -> 134 us, FP32 53 -> 44; FP64 700 x 400 x 32 59 -> 47, 386 x 258 x 40
+// 34 -> 24; few levels on a large grid (one level wave) 1500 x 800 x 5 41 -> 34.
 template <class T, int LW>
 __global__ __launch_bounds__(kThreads) void k_set_maxflux(G3 g, const T *u, const T *v, T *Huon, T *Hvom, const T *Hz)
 {
